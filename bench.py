@@ -324,8 +324,8 @@ def bench_lines(args, ctx, lib, dv, dg, f, params):
     out["cells_4"], out["cells_5"] = int((r == 4).sum()), int((r == 5).sum())
     out["roofline"] = {"bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None,
                        "note": "latency-bound: streamlines of a few voxels each, in the saddles' order; "
-                               "the stage is speculation, in-order replays of interacting lines and host "
-                               "read-backs per window"}
+                               "the stage is the tracing of every line alone (the longest one's FP64 steps) "
+                               "and some eight rounds over the recorded tapes"}
     if not args.no_cpu:
         sys.path.insert(0, os.path.join(ROOT, "tests"))
         import oracle_lib  # noqa: E402  (checker / baseline only)

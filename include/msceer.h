@@ -91,14 +91,14 @@ typedef struct msceer_label_stats {
     float ms_pass3;             /* integration pass 3 */
     int64_t reintegrated_pass3;  /* pass-3 re-integrations (all of them, whatever their precision) */
     int64_t escalated_fp64;     /* with MSCEER_FP32_FIRST: of those, left in doubt by the FP32 trace and traced again in FP64 */
-    int64_t lines_asc;          /* msceer_ondemand, needASC1: streamlines traced from the 2-saddles (speculation included) */
+    int64_t lines_asc;          /* msceer_ondemand, needASC1: streamlines traced from the 2-saddles */
     int64_t lines_dsc;          /* needDSC1: streamlines traced from the 1-saddles */
-    int64_t lines_replayed;     /* of the 1-manifold streamlines, re-traced in order inside a component */
-    int32_t line_windows;       /* speculation windows of the 1-manifold stage */
-    int32_t line_cuts;          /* windows cut short by a replay that left its component */
+    int64_t lines_replayed;     /* of the 1-manifold streamlines, cut short by the labels of earlier ones */
+    int32_t line_windows;       /* windows of lines the 1-manifold stage traced at once */
+    int32_t line_cuts;          /* windows cut short at a line still changing after the last round */
     float ms_lines;             /* the 1-manifold stage */
     int32_t line_alone;         /* 1-manifold streamlines traced alone, in order */
-    int32_t line_overflows;     /* windows cut short where the footprint pool ran out */
+    int32_t line_overflows;     /* windows cut short where the tape pool ran out */
     int64_t maxima;             /* needDSC2: critical hexes of the steepest pairing */
     int64_t saddles2;           /* needDSC2: critical quads */
     int64_t regions_dsc;        /* needDSC2: descending certain regions after simplification */

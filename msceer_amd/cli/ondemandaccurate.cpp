@@ -90,7 +90,7 @@ int main(int argc, char** argv) {
             printf("built maxgraph: %lld maxima, %lld 2-saddles -> %lld descending regions\n", (long long)st.maxima,
                    (long long)st.saddles2, (long long)st.regions_dsc);
         if (a1 || d1)
-            printf("1-manifold streamlines: %lld from 2-saddles, %lld from 1-saddles (%lld re-traced in order)\n",
+            printf("1-manifold streamlines: %lld from 2-saddles, %lld from 1-saddles (%lld cut short by earlier ones)\n",
                    (long long)st.lines_asc, (long long)st.lines_dsc, (long long)st.lines_replayed);
         if (dbg && a2) {
             char lname[2048];

@@ -123,13 +123,12 @@ struct msceer_ctx {
     msceer::DevBuf ldir;  // ldir walk records and visited bitmaps
     // accurate labelling
     msceer::DevBuf gradf, gradd, scan, label, label2, dest, seedmask, redo, stamp, rep, rep2, restriction, host_io, mask;
-    // accurate 1-manifolds: per-cell line stamps (two words, kept cleared
-    // between calls) and the saddle / window scratch
+    // accurate 1-manifolds: per-cell line stamps (two words, older tags are
+    // ignored) with the next tag, and the saddle / window scratch
     msceer::DevBuf line_stamps, lines;
+    uint32_t line_tag = 0;
     // descending 3-manifolds: their labels and seed mask
     msceer::DevBuf label_dsc, seedmask2;
-    bool line_stamps_clear = false;
-    uint64_t line_stamps_cells = 0;
     msceer::HostBuf host_stage;  // pinned staging of host-side merges (cleanup)
     uint32_t* h_ctl = nullptr;  // pinned mirror of the control block
     // 8, 9: certain-round groups; 12-15: integration passes; 16, 17: the

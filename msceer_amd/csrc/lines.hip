@@ -21,26 +21,28 @@
 // the target.  One reference thread runs this in order, so later streamlines
 // stop on earlier ones: the result is defined by that order.
 //
-// On the GPU the order is kept exactly by speculation over windows of
-// streamlines ("lines"; the saddle's own label is a line without a trace):
-//  1. every line of the window is traced at once against the labels committed
-//     before the window plus its own, recording its footprint: the cells it
-//     tested for the target and the cells it labelled (a cell labelled by
-//     lines of the window belongs to the lowest of them, wstamp);
-//  2. lines are joined (union-find) when one labels a cell in another's
-//     footprint.  A line whose footprint no earlier line of the window
-//     labels saw exactly the labels it would see in order: its labels stand;
-//  3. each component is replayed by one lane, its lines in order: those
-//     depending on an earlier line are re-traced against the committed labels
-//     and the labels of their component's earlier lines.  A replayed line
-//     that tests a cell of another component's labels, or labels a cell its
-//     component did not label in speculation, went beyond what the
-//     speculation saw: the window is cut before it;
-//  4. the labels of the lines before the cut are committed; the next window
-//     starts at the cut.  The first line of a window depends on nothing, so
-//     every window commits at least one line.
-// A line whose footprint does not fit the pool ends its window; first in a
-// window, it is traced alone, in order.
+// On the GPU the order is kept exactly, over windows of streamlines ("lines";
+// the saddle's own label is a line without a trace):
+//  1. every line of the window is traced at once, one lane a line, and records
+//     a tape: what it would ask of the labels if only its own stopped it
+//     (lines_core.hpp).  Nothing is read from the labels but, in later
+//     windows, the committed ones;
+//  2. rounds: every line is evaluated along its tape, one wave a line, against
+//     the labels the lines gave in the round before (per cell the lowest line
+//     that gives it; an earlier line's label counts, a later one's does not).
+//     Line k of the window is exact once the lines before it are, so round k
+//     at the latest; in practice the rounds stop changing anything after five
+//     to ten, and then every line is exact;
+//  3. the labels are committed; the next window follows.
+// A line whose tape does not fit the pool ends its window; first in a window,
+// it is traced alone, in order.
+//
+// What bounds it: the tracing, the latency of the longest streamline's steps
+// (FP64 chains of a few hundred cycles and, at each voxel entered, a gather
+// of 8 corners): 2.7 ms a family on the 256^3 labelling volume.  A tape holds
+// 20 to 40 entries on average, so a round is a few dependent reads per line
+// (90 us).  Tracing interacting lines again in order, a lane per component,
+// took 77 ms there and reading labels at every step of the first trace 42 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -72,10 +74,26 @@ __device__ __forceinline__ uint32_t wave_append(bool want, uint32_t* counter) {
 
 // ---- the saddles and their seeds -------------------------------------------
 
-// Critical cells of dimension sdim, keyed (float key of the value of the
-// highest vertex -- negated for DSC -- << 32 | cell id): sorted descending,
-// this is the reference's processing order (pairs (value, id) sorted
-// ascending and taken from the end).
+// Key of saddle c: the float key of the value of its highest vertex (by value,
+// id) -- negated for DSC -- << 32 | cell id.
+__device__ __forceinline__ uint64_t saddle_key(const CellGeom& m, int X, int Y, const float* __restrict__ f, int asc,
+                                               uint32_t c) {
+    int64_t x, y, z;
+    m.xyz(c, x, y, z);
+    int64_t best = -1;
+    for (int k = 0; k < 8; k++) {
+        if (((k & 1) && !(x & 1)) || ((k & 2) && !(y & 1)) || ((k & 4) && !(z & 1))) continue;
+        const int64_t vx = (x >> 1) + (k & 1), vy = (y >> 1) + ((k >> 1) & 1), vz = (z >> 1) + (k >> 2);
+        const int64_t v = vx + (int64_t)X * (vy + (int64_t)Y * vz);
+        if (best < 0 || f[v] > f[best] || (!(f[best] > f[v]) && v > best)) best = v;
+    }
+    const float val = f[best];
+    return ((uint64_t)value_key(asc ? val : -1.0f * val) << 32) | (uint64_t)c;
+}
+
+// Keys of the critical cells of dimension sdim: sorted descending, this is the
+// reference's processing order (pairs (value, id) sorted ascending and taken
+// from the end).
 __global__ void __launch_bounds__(kThreads)
 line_saddles_kernel(const uint8_t* __restrict__ grad, CellGeom m, int X, int Y, const float* __restrict__ f,
                     int sdim, int asc, uint64_t* __restrict__ keys, uint32_t* count, uint32_t cap) {
@@ -84,26 +102,26 @@ line_saddles_kernel(const uint8_t* __restrict__ grad, CellGeom m, int X, int Y, 
     for (uint64_t base = (uint64_t)blockIdx.x * kThreads; base < C; base += stride) {
         const uint64_t c = base + threadIdx.x;
         bool want = false;
-        uint64_t key = 0;
         if (c < C && critical(grad, (uint32_t)c)) {
             int64_t x, y, z;
             m.xyz((uint32_t)c, x, y, z);
-            if ((int)((x & 1) + (y & 1) + (z & 1)) == sdim) {
-                // highest vertex by (value, id) among the cell's vertices
-                int64_t best = -1;
-                for (int k = 0; k < 8; k++) {
-                    if (((k & 1) && !(x & 1)) || ((k & 2) && !(y & 1)) || ((k & 4) && !(z & 1))) continue;
-                    const int64_t vx = (x >> 1) + (k & 1), vy = (y >> 1) + ((k >> 1) & 1), vz = (z >> 1) + (k >> 2);
-                    const int64_t v = vx + (int64_t)X * (vy + (int64_t)Y * vz);
-                    if (best < 0 || f[v] > f[best] || (!(f[best] > f[v]) && v > best)) best = v;
-                }
-                const float val = f[best];
-                key = ((uint64_t)value_key(asc ? val : -1.0f * val) << 32) | (uint64_t)(uint32_t)c;
-                want = true;
-            }
+            want = (int)((x & 1) + (y & 1) + (z & 1)) == sdim;
         }
         const uint32_t at = wave_append(want, count);
-        if (want && at < cap) keys[at] = key;
+        if (want && at < cap) keys[at] = saddle_key(m, X, Y, f, asc, (uint32_t)c);
+    }
+}
+
+// The same keys from the lower-star pass's list of the critical cells of that
+// dimension (in any order).
+__global__ void __launch_bounds__(kThreads)
+line_saddle_list_kernel(MList list, CellGeom m, int X, int Y, const float* __restrict__ f, int asc,
+                        uint64_t* __restrict__ keys, uint32_t n) {
+    __shared__ uint32_t prefix[kSubs + 2];
+    const uint32_t total = min(mlist_prefix(list, prefix), n);
+    for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < total; i += gridDim.x * kThreads) {
+        const uint32_t c = mlist_at(list, prefix, i);
+        keys[i] = saddle_key(m, X, Y, f, asc, c);
     }
 }
 
@@ -126,169 +144,240 @@ struct LineArgs {
     bool asc;
     double gthr, ethr;
     int max_iters;
-    uint32_t* wstamp;  // per cell, kNoLine outside a window
-    uint32_t* pstamp;  // per cell, kNoLine outside a window
-    uint32_t* lstamp;  // per cell, kNoLine outside a window
-    uint32_t* own;     // per cell, kNoLine outside a window
-    Pool pool;
-    uint32_t* fhead;   // first footprint chunk per line of the window (kNoLine: none)
-    uint32_t* whead;   // first chunk of the cells each line labelled
-    uint32_t* mhead;   // first chunk of the cells each line's stops could label
-    uint32_t* touched; // cells labelled speculatively in the window
+    TapePool pool;
+    uint64_t* wmask;   // per chunk: list entries whose cell carries the target after them
+    uint32_t* active;  // lines of the window with a tape
+    uint32_t* head;    // their first chunks
+    uint32_t* ended;   // where they ended: slots along the tape, 0 at its end
+    uint32_t* stamp[2];  // per cell: round tag << kLineBits | lowest line of the window giving it its label
     uint32_t* ctl;     // kLcWords words
 };
 
 enum LineCtl : int {
-    kLcOverflow = 0,  // lowest line whose footprint did not fit the pool
-    kLcFail = 1,      // lowest line whose replay left its component
-    kLcComps = 2,     // components of the window
-    kLcTraced = 3,    // streamlines traced (all phases)
-    kLcReplayed = 4,  // streamlines re-traced in replays
-    kLcVoxels = 5,    // voxel traversals (all phases)
-    kLcTouched = 6,   // cells labelled speculatively in the window
-    kLcPoolTop = 7,   // next free word of the footprint pool
-    kLcWhyTest = 8,   // replays stopped by a test of another component's cell
-    kLcWhyLabel = 9,  // replays stopped by a label the speculation did not give
+    kLcOverflow = 0,  // lowest line whose tape did not fit the pool
+    kLcActive = 1,    // lines of the window with a tape
+    kLcTraced = 2,    // streamlines traced
+    kLcVoxels = 3,    // voxel traversals
+    kLcTop = 4,       // next free chunk of the pool
+    kLcCut = 5,       // streamlines that ended before their tape
+    kLcChanged = 6,   // three words: lines a round changed (rotating)
+    kLcLowest = 9,    // three words: the lowest of them
     kLcWords = 12
 };
 
-// 1. Speculation over lines [w0, w1).
-__global__ void __launch_bounds__(kThreads) line_spec_kernel(LineArgs a, uint32_t w0, uint32_t w1) {
-    const uint32_t i = w0 + blockIdx.x * kThreads + threadIdx.x;
-    if (i >= w1) return;
-    SpecLabels lab{a.restr, a.target, a.wstamp, a.pstamp, a.own, i, a.pool, a.touched, &a.ctl[kLcTouched]};
-    const uint32_t c = a.slots[i];
+// Stamps: the tag falls from round to round, so that a round's stamps replace
+// older ones under atomicMin and nothing is cleared between rounds, windows or
+// calls; the arrays are refilled when the tags run out.
+constexpr int kLineBits = 20;
+constexpr uint32_t kLineMask = (1u << kLineBits) - 1u;
+constexpr uint32_t kTopTag = (1u << (32 - kLineBits)) - 2u;  // the first tag after a refill
+constexpr uint32_t kMaxRounds = 512;                         // of one window
+
+// 1. Tapes of lines [w0, w1): a lane per line, a wave per work-group, so that
+// the longest lines' waves share no work-group's registers and LDS.
+constexpr int kTapeThreads = 64;
+__global__ void __launch_bounds__(kTapeThreads) line_tape_kernel(LineArgs a, uint32_t w0, uint32_t w1) {
+    __shared__ uint32_t hist[kHistory * kTapeThreads];
+    const uint32_t i = w0 + blockIdx.x * kTapeThreads + threadIdx.x;
+    const uint32_t c = i < w1 && i % 7 != 6 ? a.slots[i] : kNoLine;
+    uint32_t first = kNoLine;
     if (c != kNoLine) {
-        if (i % 7 == 6) {
-            lab.write(c);  // the saddle's own label
-        } else {
-            uint32_t vox = 0;
-            trace_line(a.src, a.g, a.m, c, a.asc, a.gthr, a.ethr, a.max_iters, lab, &vox);
-            atomicAdd(&a.ctl[kLcTraced], 1u);
-            atomicAdd(&a.ctl[kLcVoxels], vox);
-        }
+        TapeLabels lab{a.restr, a.target, w0 > 0, a.pool, hist + threadIdx.x, (uint32_t)kTapeThreads};
+        uint32_t vox = 0;
+        trace_line(a.src, a.g, a.m, c, a.asc, a.gthr, a.ethr, a.max_iters, lab, &vox);
+        lab.finish();
+        if (lab.over) atomicMin(&a.ctl[kLcOverflow], i);
+        else first = lab.head;
+        atomicAdd(&a.ctl[kLcTraced], 1u);
+        atomicAdd(&a.ctl[kLcVoxels], vox);
     }
-    lab.finish();
-    a.fhead[i - w0] = lab.over ? kNoLine : lab.all.head;
-    a.whead[i - w0] = lab.over ? kNoLine : lab.wrote.head;
-    a.mhead[i - w0] = lab.over ? kNoLine : lab.maybe.head;
-    if (lab.over) atomicMin(&a.ctl[kLcOverflow], i);
+    const uint32_t at = wave_append(first != kNoLine, &a.ctl[kLcActive]);
+    if (first != kNoLine) {
+        a.active[at] = i;
+        a.head[at] = first;
+        a.ended[at] = 0;
+    }
 }
 
-// 2. Components: a line joins the lowest line of [w0, wc) that labels any
-// cell of its footprint (every line that labels a cell also has it in its
-// footprint, so all lines touching a labelled cell meet in one component).
-__global__ void __launch_bounds__(kThreads) line_init_parent_kernel(uint32_t* parent, uint32_t n) {
-    const uint32_t r = blockIdx.x * kThreads + threadIdx.x;
-    if (r < n) parent[r] = r;
-}
-// Also flags the lines that depend on an earlier line of the window (an
-// earlier line labels a cell of their footprint): only those are re-traced.
-__global__ void __launch_bounds__(kThreads)
-line_union_kernel(LineArgs a, uint32_t w0, uint32_t wc, uint32_t* parent, uint8_t* dep) {
-    const uint32_t i = w0 + blockIdx.x * kThreads + threadIdx.x;
-    if (i >= wc) return;
-    bool d = false;
-    for (uint32_t ch = a.fhead[i - w0]; ch != kNoLine; ch = a.pool.cells[ch]) {
-        for (uint32_t j = 1; j < kChunk; j++) {
-            const uint32_t c = a.pool.cells[ch + j];
-            if (c == kNoLine) break;
-            const uint32_t owners[2] = {a.wstamp[c], a.pstamp[c]};
-            for (uint32_t w : owners)
-                if (w != i && w >= w0 && w < wc) {
-                    lf_union(parent, i - w0, w - w0);
-                    d = d || w < i;
+// The lines of a window end before the first one whose tape did not fit.
+__device__ __forceinline__ uint32_t window_end(const LineArgs& a, uint32_t w1) { return min(a.ctl[kLcOverflow], w1); }
+
+// Links of a tape: for every entry the line's previous kList entry of the same
+// cell.  A wave per line; pairs of chunks whose cells' boxes do not meet are
+// skipped, so a long tape costs little more than its length.
+struct CellBox {
+    int lo[3], hi[3];
+};
+__global__ void __launch_bounds__(kTapeThreads) line_links_kernel(LineArgs a) {
+    __shared__ uint32_t s_chunk[kMaxTapeChunks];
+    __shared__ CellBox s_box[kMaxTapeChunks];
+    const uint32_t lane = threadIdx.x;
+    const uint32_t n_active = a.ctl[kLcActive];
+    for (uint32_t t = blockIdx.x; t < n_active; t += gridDim.x) {
+        uint32_t q = 0;
+        for (uint32_t ch = a.head[t]; ch != kNoLine; q++) {
+            uint64_t* const e = a.pool.slots + (uint64_t)ch * kTapeChunk;
+            const uint64_t mine = e[lane];
+            const uint32_t next = __builtin_amdgcn_readfirstlane((uint32_t)mine);
+            const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)(mine >> 32));
+            const bool valid = lane >= 1 && lane <= n;
+            const uint32_t c = (uint32_t)mine, hi = (uint32_t)(mine >> 32);
+            const bool list = valid && ((hi >> kKindShift) & 3u) == kList;
+            int64_t p[3] = {0, 0, 0};
+            if (valid) a.m.xyz(c, p[0], p[1], p[2]);
+            CellBox box;
+            for (int d = 0; d < 3; d++) {
+                int lo = valid ? (int)p[d] : 0x7fffffff, hi3 = valid ? (int)p[d] : -1;
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) {
+                    lo = min(lo, __shfl_xor(lo, o));
+                    hi3 = max(hi3, __shfl_xor(hi3, o));
                 }
-        }
-    }
-    dep[i - w0] = d ? 1 : 0;
-}
-__global__ void __launch_bounds__(kThreads) line_keys_kernel(uint32_t* parent, uint32_t n, uint64_t* keys) {
-    const uint32_t r = blockIdx.x * kThreads + threadIdx.x;
-    if (r < n) keys[r] = ((uint64_t)lf_find(parent, r) << 32) | r;
-}
-// First entry of every component in the sorted keys.
-__global__ void __launch_bounds__(kThreads)
-line_starts_kernel(const uint64_t* keys, uint32_t n, uint32_t* starts, uint32_t* count) {
-    const uint32_t stride = gridDim.x * kThreads;
-    for (uint32_t base = blockIdx.x * kThreads; base < n; base += stride) {
-        const uint32_t r = base + threadIdx.x;
-        const bool want = r < n && (r == 0 || (keys[r] >> 32) != (keys[r - 1] >> 32));
-        const uint32_t at = wave_append(want, count);
-        if (want) starts[at] = r;
-    }
-}
-
-// 3. Replay: one lane per component, its lines in order.  A line no earlier
-// line of the window depends on keeps its speculative labels (the cells of
-// its footprint it claimed in wstamp: no earlier line labels any cell it
-// reads, so it saw what it would see in order); the others are re-traced.
-__device__ void keep_speculation(const LineArgs& a, uint32_t w0, uint32_t i) {
-    for (uint32_t ch = a.fhead[i - w0]; ch != kNoLine; ch = a.pool.cells[ch])
-        for (uint32_t j = 1; j < kChunk; j++) {
-            const uint32_t c = a.pool.cells[ch + j];
-            if (c == kNoLine) break;
-            if (a.wstamp[c] == i) a.lstamp[c] = i;
-        }
-}
-
-__global__ void __launch_bounds__(kThreads)
-line_replay_kernel(LineArgs a, uint32_t w0, uint32_t wc, const uint64_t* keys, const uint32_t* starts,
-                   uint32_t* parent, const uint8_t* dep) {
-    const uint32_t k = blockIdx.x * kThreads + threadIdx.x;
-    if (k >= a.ctl[kLcComps]) return;
-    const uint32_t n = wc - w0;
-    const uint32_t s0 = starts[k];
-    const uint32_t root = (uint32_t)(keys[s0] >> 32);
-    uint32_t replayed = 0, vox = 0;
-    for (uint32_t q = s0; q < n && (uint32_t)(keys[q] >> 32) == root; q++) {
-        const uint32_t i = w0 + (uint32_t)keys[q];
-        if (!dep[i - w0]) {
-            keep_speculation(a, w0, i);
-            continue;
-        }
-        ReplayLabels lab{a.restr, a.target,      a.wstamp,       a.pstamp, a.lstamp, a.own,
-                         a.pool.cells, a.whead[i - w0], a.mhead[i - w0], parent, w0, wc, root, i,
-                         &a.ctl[kLcWhyTest], false};
-        const uint32_t c = a.slots[i];
-        if (c != kNoLine) {
-            if (i % 7 == 6) {
-                lab.write(c);
-            } else {
-                trace_line(a.src, a.g, a.m, c, a.asc, a.gthr, a.ethr, a.max_iters, lab, &vox);
-                replayed++;
+                box.lo[d] = lo;
+                box.hi[d] = hi3;
             }
+            uint32_t prev = kNoPrev;
+            for (uint32_t b = 0; b < q; b++) {
+                const CellBox& o = s_box[b];
+                bool meet = true;
+                for (int d = 0; d < 3; d++) meet = meet && o.lo[d] <= box.hi[d] && box.lo[d] <= o.hi[d];
+                if (!meet) continue;
+                const uint32_t och = s_chunk[b];
+                const uint64_t theirs = a.pool.slots[(uint64_t)och * kTapeChunk + lane];
+                const uint32_t on = kTapeChunk - 1;  // every chunk but the last is full
+                const uint32_t ohi = (uint32_t)(theirs >> 32);
+                const uint64_t olist = __ballot(lane >= 1 && lane <= on && ((ohi >> kKindShift) & 3u) == kList);
+                for (uint64_t rest = olist; rest; rest &= rest - 1) {
+                    const int j = __ffsll((unsigned long long)rest) - 1;
+                    if (__shfl((uint32_t)theirs, j) == c) prev = och * kTapeChunk + (uint32_t)j;
+                }
+            }
+            const uint64_t lists = __ballot(list);
+            for (uint64_t rest = lists; rest; rest &= rest - 1) {
+                const int j = __ffsll((unsigned long long)rest) - 1;
+                if (__shfl(c, j) == c && (uint32_t)j < lane) prev = ch * kTapeChunk + (uint32_t)j;
+            }
+            if (valid && prev != kNoPrev) e[lane] = (uint64_t)((hi & ~kNoPrev) | prev) << 32 | c;
+            if (lane == 0) {
+                s_chunk[q] = ch;
+                s_box[q] = box;
+            }
+            __syncthreads();
+            ch = next;
         }
-        if (lab.bad) {
-            atomicMin(&a.ctl[kLcFail], i);
-            break;
-        }
+        __syncthreads();
     }
-    atomicAdd(&a.ctl[kLcReplayed], replayed);
-    atomicAdd(&a.ctl[kLcVoxels], vox);
 }
 
-// 4. Commit the labels of the lines before `cut`, then clear the stamps of
-// every cell labelled speculatively in the window.
-__global__ void __launch_bounds__(kThreads) line_commit_kernel(LineArgs a, uint32_t cut) {
-    const uint32_t n = min(a.ctl[kLcTouched], a.pool.capacity);
-    for (uint32_t t = blockIdx.x * kThreads + threadIdx.x; t < n; t += gridDim.x * kThreads) {
-        const uint32_t c = a.touched[t];
-        if (a.lstamp[c] < cut) a.restr[c] = a.target;
-    }
+// The k-th slot of a saddle's own label from line w0 on.
+__device__ __forceinline__ uint64_t saddle_slot(uint32_t w0, uint32_t k) {
+    return (uint64_t)w0 + (6u - w0 % 7u) + 7ull * k;
 }
-__global__ void __launch_bounds__(kThreads) line_clear_kernel(LineArgs a) {
-    const uint32_t n = min(a.ctl[kLcTouched], a.pool.capacity);
-    for (uint32_t t = blockIdx.x * kThreads + threadIdx.x; t < n; t += gridDim.x * kThreads) {
-        const uint32_t c = a.touched[t];
-        a.wstamp[c] = kNoLine;
-        a.pstamp[c] = kNoLine;
-        a.lstamp[c] = kNoLine;
-        a.own[c] = kNoLine;
+
+// 2. One round: every line of [w0, wc) evaluated along its tape against the
+// stamps of the round before (tag + 1), its labels stamped with `tag`.  A
+// round after one that changed nothing has nothing to do.
+__global__ void __launch_bounds__(kThreads)
+line_round_kernel(LineArgs a, uint32_t w0, uint32_t w1, uint32_t round, uint32_t tag) {
+    const uint32_t wc = window_end(a, w1);
+    uint32_t* const changed = a.ctl + kLcChanged;
+    uint32_t* const lowest = a.ctl + kLcLowest;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        changed[(round + 1) % 3] = 0;
+        lowest[(round + 1) % 3] = kNoLine;
+    }
+    if (round > 0 && changed[(round + 2) % 3] == 0) return;
+    const uint32_t* const in = a.stamp[round & 1];
+    uint32_t* const out = a.stamp[(round & 1) ^ 1];
+    // the saddles' own labels
+    const uint64_t threads = (uint64_t)gridDim.x * kThreads;
+    for (uint64_t i = saddle_slot(w0, blockIdx.x * kThreads + threadIdx.x); i < wc; i += 7 * threads)
+        atomicMin(&out[a.slots[i]], tag << kLineBits | (uint32_t)(i - w0));
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t waves = gridDim.x * (kThreads / 64);
+    const uint32_t n_active = a.ctl[kLcActive];
+    uint32_t n_changed = 0, low = kNoLine;
+    for (uint32_t t = blockIdx.x * (kThreads / 64) + threadIdx.x / 64; t < n_active; t += waves) {
+        const uint32_t line = __builtin_amdgcn_readfirstlane(a.active[t]);
+        if (line >= wc) continue;
+        TapeState s;
+        uint32_t ended = 0, ord = 0;
+        bool diff = false;
+        for (uint32_t ch = a.head[t]; ch != kNoLine && !ended; ord++) {
+            const uint64_t e = a.pool.slots[(uint64_t)ch * kTapeChunk + lane];
+            const uint32_t next = __builtin_amdgcn_readfirstlane((uint32_t)e);
+            const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)(e >> 32));
+            const bool valid = lane >= 1 && lane <= n;
+            const uint32_t c = (uint32_t)e, hi = (uint32_t)(e >> 32), kind = (hi >> kKindShift) & 3u;
+            bool labelled = false;
+            if (valid) {
+                const uint32_t v = in[c];
+                labelled = round > 0 && (v >> kLineBits) == tag + 1 && (v & kLineMask) < line - w0;
+                if (w0 > 0) labelled = labelled || a.restr[c] == a.target;
+            }
+            const uint64_t before = a.wmask[ch];
+            auto own = [&](uint32_t k, uint64_t w) {
+                const uint32_t p = __builtin_amdgcn_readlane(hi, k) & kNoPrev;
+                uint64_t word = w;
+                if (p / kTapeChunk != ch)
+                    word = __hip_atomic_load(&a.wmask[p / kTapeChunk], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return ((word >> (p % kTapeChunk)) & 1ull) != 0;
+            };
+            uint32_t at = 0;
+            const uint64_t w = tape_chunk(s, n, __ballot(valid && kind <= kExit), __ballot(valid && kind == kExit),
+                                          __ballot(valid && kind == kStop), __ballot(valid && (hi & kFirst)),
+                                          __ballot(labelled), __ballot(valid && (hi & kNoPrev) != kNoPrev), own, &at);
+            if (before != w) {
+                diff = true;
+                if (lane == 0)
+                    __hip_atomic_store(&a.wmask[ch], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if ((w >> lane) & 1ull) atomicMin(&out[c], tag << kLineBits | (line - w0));
+            if (at) ended = ord * kTapeChunk + at;
+            ch = next;
+        }
+        if (round == 0 || diff || a.ended[t] != ended) {
+            n_changed++;
+            low = line < low ? line : low;
+            if (lane == 0) a.ended[t] = ended;
+        }
+    }
+    if (lane == 0 && n_changed) {
+        atomicAdd(&changed[round % 3], n_changed);
+        atomicMin(&lowest[round % 3], low);
     }
 }
 
-// A line traced alone, in order (first of its window, footprint beyond the pool).
+// 3. Commit the labels of the lines before `end`, unless round `last` still
+// changed some (check).
+__global__ void __launch_bounds__(kThreads)
+line_commit_kernel(LineArgs a, uint32_t w0, uint32_t end, uint32_t last, bool check) {
+    if (check && a.ctl[kLcChanged + last % 3] != 0) return;
+    const uint32_t cut = window_end(a, end);
+    const uint64_t threads = (uint64_t)gridDim.x * kThreads;
+    for (uint64_t i = saddle_slot(w0, blockIdx.x * kThreads + threadIdx.x); i < cut; i += 7 * threads)
+        a.restr[a.slots[i]] = a.target;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t waves = gridDim.x * (kThreads / 64);
+    const uint32_t n_active = a.ctl[kLcActive];
+    uint32_t n_cut = 0;
+    for (uint32_t t = blockIdx.x * (kThreads / 64) + threadIdx.x / 64; t < n_active; t += waves) {
+        const uint32_t line = __builtin_amdgcn_readfirstlane(a.active[t]);
+        if (line >= cut) continue;
+        const uint32_t ended = a.ended[t];
+        uint32_t ord = 0;
+        for (uint32_t ch = a.head[t]; ch != kNoLine && !(ended && ord * kTapeChunk >= ended); ord++) {
+            const uint64_t e = a.pool.slots[(uint64_t)ch * kTapeChunk + lane];
+            const uint64_t w = a.wmask[ch];
+            if ((w >> lane) & 1ull) a.restr[(uint32_t)e] = a.target;
+            ch = __builtin_amdgcn_readfirstlane((uint32_t)e);
+        }
+        n_cut += ended ? 1u : 0u;
+    }
+    if (lane == 0 && n_cut) atomicAdd(&a.ctl[kLcCut], n_cut);
+}
+
+// A line traced alone, in order (first of its window, its tape beyond the pool).
 __global__ void line_direct_kernel(LineArgs a, uint32_t i) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
     DirectLabels lab{a.restr, a.target};
@@ -307,16 +396,16 @@ __global__ void line_direct_kernel(LineArgs a, uint32_t i) {
 __global__ void line_ctl_init_kernel(uint32_t* ctl, bool all) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         ctl[kLcOverflow] = kNoLine;
-        ctl[kLcFail] = kNoLine;
-        ctl[kLcComps] = 0;
-        ctl[kLcTouched] = 0;
-        ctl[kLcPoolTop] = 0;
+        ctl[kLcActive] = 0;
+        ctl[kLcTop] = 0;
+        for (int k = 0; k < 3; k++) {
+            ctl[kLcChanged + k] = 0;
+            ctl[kLcLowest + k] = kNoLine;
+        }
         if (all) {
             ctl[kLcTraced] = 0;
-            ctl[kLcReplayed] = 0;
             ctl[kLcVoxels] = 0;
-            ctl[kLcWhyTest] = 0;
-            ctl[kLcWhyLabel] = 0;
+            ctl[kLcCut] = 0;
         }
     }
 }
@@ -330,10 +419,11 @@ inline uint32_t blocks_for(uint64_t n) { return (uint32_t)std::max<uint64_t>(1, 
 
 }  // namespace
 
-// Window of lines speculated at once (bounds the footprint scratch).  The
+// Window of lines traced at once (bounds the tapes' scratch; line numbers in
+// the stamps have kLineBits bits).  The
 // environment variable MSCEER_LINE_WINDOW (8 .. 2^20) sets a smaller one,
 // which tests use to exercise many windows on small volumes.
-constexpr uint32_t kWindow = 1u << 20;
+constexpr uint32_t kWindow = 1u << kLineBits;
 
 uint32_t line_window() {
     if (const char* e = getenv("MSCEER_LINE_WINDOW")) {
@@ -343,73 +433,53 @@ uint32_t line_window() {
     return kWindow;
 }
 
-int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t* grad, const double4* gradd,
-              int8_t* restr, bool asc, float gthr, float ethr, int max_iters, LineStats* out) {
+int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t* grad, const MList* saddles,
+              uint32_t n_saddles, const double4* gradd, int8_t* restr, bool asc, float gthr, float ethr, int max_iters,
+              LineStats* out) {
     hipStream_t s = ctx->stream;
     const VGrid g = make_vgrid(d.X, d.Y, d.Z);
     CellGeom m{(int64_t)d.Mx, (int64_t)d.My, (int64_t)d.Mz, (int64_t)d.Mx * (int64_t)d.My};
     if (d.cells >= 0xFFFFFFFFull) return MSCEER_ETOOBIG;
-    uint32_t* ctl = ctl_dev(ctx);
-    uint32_t* count = ctl + kCtlCount;
+    uint32_t* count = ctl_dev(ctx) + kCtlCount;
 
-    // per-cell stamps (lowest speculative labeller, lowest possible labeller,
-    // replay labeller, last speculative labeller), kNoLine between windows
-    CHECK_HIP(ctx->line_stamps.ensure(16 * d.cells));
-    uint32_t* wstamp = ctx->line_stamps.as<uint32_t>();
-    uint32_t* pstamp = wstamp + d.cells;
-    uint32_t* lstamp = pstamp + d.cells;
-    uint32_t* own = lstamp + d.cells;
-    if (!ctx->line_stamps_clear || ctx->line_stamps_cells != d.cells) {
-        hipLaunchKernelGGL(line_fill_kernel, dim3(2048), dim3(kThreads), 0, s, wstamp, 4 * d.cells, kNoLine);
+    uint32_t S = n_saddles;
+    if (!saddles) {
+        // no list of them: count, below gather, by a scan over the cells
+        CHECK_HIP(launch_zero(count, 1, s));
+        hipLaunchKernelGGL(line_saddles_kernel, dim3(2048), dim3(kThreads), 0, s, grad, m, d.X, d.Y, values,
+                           asc ? 2 : 1, asc ? 1 : 0, nullptr, count, 0u);
         CHECK_HIP(hipGetLastError());
-        ctx->line_stamps_cells = d.cells;
+        int rc = read_ctl(ctx, kCtlCount, 1);
+        if (rc) return rc;
+        S = ctx->h_ctl[kCtlCount];
     }
-    ctx->line_stamps_clear = false;  // until every window has cleared its cells
-
-    // saddles: count first, then keys sorted into processing order
-    CHECK_HIP(launch_zero(count, 1, s));
-    hipLaunchKernelGGL(line_saddles_kernel, dim3(2048), dim3(kThreads), 0, s, grad, m, d.X, d.Y, values, asc ? 2 : 1,
-                       asc ? 1 : 0, nullptr, count, 0u);
-    CHECK_HIP(hipGetLastError());
-    int rc = read_ctl(ctx, kCtlCount, 1);
-    if (rc) return rc;
-    const uint32_t S = ctx->h_ctl[kCtlCount];
     out->saddles = S;
-    if (S == 0) {
-        ctx->line_stamps_clear = true;
-        return MSCEER_OK;
-    }
+    if (S == 0) return MSCEER_OK;
     if ((uint64_t)S * 7 >= 0xFFFFFFFFull) return MSCEER_ETOOBIG;
     const uint64_t nslots = 7ull * S;
     const uint32_t W = (uint32_t)std::min<uint64_t>(nslots, line_window());
-    // footprint pool: 256 cells per line of a window on average, at least 2^22
-    // words (a speculative trace runs until committed or its own labels stop
-    // it, so early in a volume it runs to the extremum)
-    const uint32_t pool_cap = (uint32_t)std::min<uint64_t>(
-        std::max<uint64_t>((uint64_t)W * 256, 1u << 22) / kChunk * kChunk, 0x7FFFFFFFull / kChunk * kChunk);
+
+    // two stamps per cell, refilled when they are new or the tags run out
+    if (ctx->line_stamps.bytes < 8 * d.cells) ctx->line_tag = 0;
+    CHECK_HIP(ctx->line_stamps.ensure(8 * d.cells));
+    // tape pool: 128 slots per line of a window (volumes of noise and mixtures
+    // record 20 to 40), at least 2^15 chunks
+    const uint32_t chunks = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(2ull * W, 1u << 15), 1u << 22);
 
     // scratch layout
-    size_t sort_tmp = 0, sort_tmp2 = 0;
-    CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(nullptr, sort_tmp, (const uint64_t*)nullptr,
+    size_t tmp_bytes = 0;
+    CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(nullptr, tmp_bytes, (const uint64_t*)nullptr,
                                                           (uint64_t*)nullptr, (int)S, 0, 64, s));
-    CHECK_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, sort_tmp2, (const uint64_t*)nullptr, (uint64_t*)nullptr,
-                                                (int)W, 0, 64, s));
-    const size_t tmp_bytes = std::max(sort_tmp, sort_tmp2);
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     size_t off = 0;
     const size_t o_keys = off; off += al(8 * (size_t)S);
     const size_t o_sorted = off; off += al(8 * (size_t)S);
     const size_t o_slots = off; off += al(4 * nslots);
-    const size_t o_pool = off; off += al(4 * (size_t)pool_cap);
-    const size_t o_touched = off; off += al(4 * (size_t)pool_cap);
-    const size_t o_fhead = off; off += al((size_t)W * 4);
-    const size_t o_whead = off; off += al((size_t)W * 4);
-    const size_t o_mhead = off; off += al((size_t)W * 4);
-    const size_t o_parent = off; off += al((size_t)W * 4);
-    const size_t o_dep = off; off += al((size_t)W);
-    const size_t o_wkeys = off; off += al((size_t)W * 8);
-    const size_t o_wsorted = off; off += al((size_t)W * 8);
-    const size_t o_starts = off; off += al((size_t)W * 4);
+    const size_t o_pool = off; off += al(8 * (size_t)kTapeChunk * chunks);
+    const size_t o_wmask = off; off += al(8 * (size_t)chunks);
+    const size_t o_active = off; off += al((size_t)W * 4);
+    const size_t o_head = off; off += al((size_t)W * 4);
+    const size_t o_ended = off; off += al((size_t)W * 4);
     const size_t o_lctl = off; off += al(4 * kLcWords);
     const size_t o_tmp = off; off += al(tmp_bytes);
     CHECK_HIP(ctx->lines.ensure(off));
@@ -417,20 +487,18 @@ int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t
     uint64_t* keys = (uint64_t*)(base + o_keys);
     uint64_t* sorted = (uint64_t*)(base + o_sorted);
     uint32_t* slots = (uint32_t*)(base + o_slots);
-    uint32_t* parent = (uint32_t*)(base + o_parent);
-    uint8_t* dep = (uint8_t*)(base + o_dep);
-    uint64_t* wkeys = (uint64_t*)(base + o_wkeys);
-    uint64_t* wsorted = (uint64_t*)(base + o_wsorted);
-    uint32_t* starts = (uint32_t*)(base + o_starts);
     uint32_t* lctl = (uint32_t*)(base + o_lctl);
-    void* tmp = base + o_tmp;
 
-    CHECK_HIP(launch_zero(count, 1, s));
-    hipLaunchKernelGGL(line_saddles_kernel, dim3(2048), dim3(kThreads), 0, s, grad, m, d.X, d.Y, values, asc ? 2 : 1,
-                       asc ? 1 : 0, keys, count, S);
+    if (saddles) {
+        hipLaunchKernelGGL(line_saddle_list_kernel, dim3(std::min<uint32_t>(blocks_for(S), 1024)), dim3(kThreads), 0, s,
+                           *saddles, m, d.X, d.Y, values, asc ? 1 : 0, keys, S);
+    } else {
+        CHECK_HIP(launch_zero(count, 1, s));
+        hipLaunchKernelGGL(line_saddles_kernel, dim3(2048), dim3(kThreads), 0, s, grad, m, d.X, d.Y, values,
+                           asc ? 2 : 1, asc ? 1 : 0, keys, count, S);
+    }
     CHECK_HIP(hipGetLastError());
-    size_t tb = tmp_bytes;
-    CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(tmp, tb, keys, sorted, (int)S, 0, 64, s));
+    CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(base + o_tmp, tmp_bytes, keys, sorted, (int)S, 0, 64, s));
     hipLaunchKernelGGL(line_seeds_kernel, dim3(blocks_for(S)), dim3(kThreads), 0, s, grad, m, sorted, S,
                        asc ? 1 : 0, slots);
     CHECK_HIP(hipGetLastError());
@@ -446,83 +514,85 @@ int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t
     a.gthr = (double)gthr;
     a.ethr = (double)ethr;
     a.max_iters = max_iters;
-    a.wstamp = wstamp;
-    a.pstamp = pstamp;
-    a.lstamp = lstamp;
-    a.own = own;
-    a.pool = Pool{(uint32_t*)(base + o_pool), pool_cap, lctl + kLcPoolTop};
-    a.fhead = (uint32_t*)(base + o_fhead);
-    a.whead = (uint32_t*)(base + o_whead);
-    a.mhead = (uint32_t*)(base + o_mhead);
-    a.touched = (uint32_t*)(base + o_touched);
+    a.pool = TapePool{(uint64_t*)(base + o_pool), chunks, lctl + kLcTop};
+    a.wmask = (uint64_t*)(base + o_wmask);
+    a.active = (uint32_t*)(base + o_active);
+    a.head = (uint32_t*)(base + o_head);
+    a.ended = (uint32_t*)(base + o_ended);
+    a.stamp[0] = ctx->line_stamps.as<uint32_t>();
+    a.stamp[1] = a.stamp[0] + d.cells;
     a.ctl = lctl;
     hipLaunchKernelGGL(line_ctl_init_kernel, dim3(1), dim3(64), 0, s, lctl, true);
     CHECK_HIP(hipGetLastError());
 
     uint32_t h[kLcWords];
+    auto read_back = [&]() -> int {
+        CHECK_HIP(hipMemcpyAsync(h, lctl, sizeof(h), hipMemcpyDeviceToHost, s));
+        CHECK_HIP(hipStreamSynchronize(s));
+        return MSCEER_OK;
+    };
     uint64_t w0 = 0;
     while (w0 < nslots) {
         const uint32_t a0 = (uint32_t)w0;
         const uint32_t w1 = (uint32_t)std::min<uint64_t>(nslots, w0 + W);
         const uint32_t n = w1 - a0;
+        if (ctx->line_tag <= kMaxRounds) {
+            hipLaunchKernelGGL(line_fill_kernel, dim3(2048), dim3(kThreads), 0, s, a.stamp[0],
+                               (uint64_t)(ctx->line_stamps.bytes / 4), kNoLine);
+            CHECK_HIP(hipGetLastError());
+            ctx->line_tag = kTopTag;
+        }
+        const uint32_t wave_blocks = std::min<uint32_t>(blocks_for((uint64_t)n * 64), 2048);
         hipLaunchKernelGGL(line_ctl_init_kernel, dim3(1), dim3(64), 0, s, lctl, false);
-        hipLaunchKernelGGL(line_spec_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, s, a, a0, w1);
+        hipLaunchKernelGGL(line_tape_kernel, dim3((n + kTapeThreads - 1) / kTapeThreads), dim3(kTapeThreads), 0, s, a,
+                           a0, w1);
+        hipLaunchKernelGGL(line_links_kernel, dim3(std::min<uint32_t>(n, 8192)), dim3(kTapeThreads), 0, s, a);
         CHECK_HIP(hipGetLastError());
-        CHECK_HIP(hipMemcpyAsync(h, lctl, sizeof(h), hipMemcpyDeviceToHost, s));
-        CHECK_HIP(hipStreamSynchronize(s));
         out->windows++;
-        if (h[kLcOverflow] == a0) {
-            // the first line's footprint did not fit the pool: it alone, in order
-            hipLaunchKernelGGL(line_clear_kernel, dim3(256), dim3(kThreads), 0, s, a);
-            hipLaunchKernelGGL(line_direct_kernel, dim3(1), dim3(64), 0, s, a, a0);
+        // rounds in groups; the host reads back only whether the last one
+        // still changed a line (then the commit behind it did nothing)
+        uint32_t round = 0;
+        uint32_t cut = 0;
+        while (true) {
+            constexpr uint32_t kGroup = 8;
+            for (uint32_t j = 0; j < kGroup; j++, round++)
+                hipLaunchKernelGGL(line_round_kernel, dim3(wave_blocks), dim3(kThreads), 0, s, a, a0, w1, round,
+                                   ctx->line_tag--);
+            hipLaunchKernelGGL(line_commit_kernel, dim3(wave_blocks), dim3(kThreads), 0, s, a, a0, w1, round - 1, true);
             CHECK_HIP(hipGetLastError());
-            out->direct++;
-            w0 = a0 + 1;
-            continue;
+            int rc = read_back();
+            if (rc) return rc;
+            const uint32_t wc = std::min(h[kLcOverflow], w1);  // lines of this window
+            if (h[kLcChanged + (round - 1) % 3] == 0) {
+                cut = wc;
+                if (wc < w1) out->overflows++;
+                break;
+            }
+            if (round + kGroup > kMaxRounds) {
+                // the lines before the lowest one still changing are exact
+                cut = h[kLcLowest + (round - 1) % 3];
+                hipLaunchKernelGGL(line_commit_kernel, dim3(wave_blocks), dim3(kThreads), 0, s, a, a0, cut, 0u, false);
+                CHECK_HIP(hipGetLastError());
+                out->cuts++;
+                break;
+            }
         }
-        const uint32_t wc = h[kLcOverflow] < w1 ? h[kLcOverflow] : w1;  // lines of this window
-        if (wc < w1) out->overflows++;
-        const uint32_t nc = wc - a0;
-        hipLaunchKernelGGL(line_init_parent_kernel, dim3(blocks_for(nc)), dim3(kThreads), 0, s, parent, nc);
-        hipLaunchKernelGGL(line_union_kernel, dim3(blocks_for(nc)), dim3(kThreads), 0, s, a, a0, wc, parent, dep);
-        hipLaunchKernelGGL(line_keys_kernel, dim3(blocks_for(nc)), dim3(kThreads), 0, s, parent, nc, wkeys);
-        CHECK_HIP(hipGetLastError());
-        tb = tmp_bytes;
-        CHECK_HIP(hipcub::DeviceRadixSort::SortKeys(tmp, tb, wkeys, wsorted, (int)nc, 0, 64, s));
-        hipLaunchKernelGGL(line_starts_kernel, dim3(std::min<uint32_t>(blocks_for(nc), 1024)), dim3(kThreads), 0, s,
-                           wsorted, nc, starts, lctl + kLcComps);
-        hipLaunchKernelGGL(line_replay_kernel, dim3(blocks_for(nc)), dim3(kThreads), 0, s, a, a0, wc, wsorted, starts,
-                           parent, dep);
-        CHECK_HIP(hipGetLastError());
-        CHECK_HIP(hipMemcpyAsync(h, lctl, sizeof(h), hipMemcpyDeviceToHost, s));
-        CHECK_HIP(hipStreamSynchronize(s));
-        const uint32_t cut = h[kLcFail] < wc ? h[kLcFail] : wc;
+        out->rounds += round;
         if (cut == a0) {
-            // (the first line's speculation is exact, so its replay is too;
-            // should it fail all the same, it is traced alone, in order)
-            hipLaunchKernelGGL(line_clear_kernel, dim3(256), dim3(kThreads), 0, s, a);
+            // the first line's tape did not fit the pool: it alone, in order
             hipLaunchKernelGGL(line_direct_kernel, dim3(1), dim3(64), 0, s, a, a0);
             CHECK_HIP(hipGetLastError());
             out->direct++;
             w0 = a0 + 1;
             continue;
         }
-        const uint32_t tb_blocks = std::min<uint32_t>(blocks_for(h[kLcTouched]), 4096);
-        hipLaunchKernelGGL(line_commit_kernel, dim3(tb_blocks), dim3(kThreads), 0, s, a, cut);
-        hipLaunchKernelGGL(line_clear_kernel, dim3(tb_blocks), dim3(kThreads), 0, s, a);
-        CHECK_HIP(hipGetLastError());
-        out->components += h[kLcComps];
-        if (cut < wc) out->cuts++;
         w0 = cut;
     }
-    CHECK_HIP(hipMemcpyAsync(h, lctl, sizeof(h), hipMemcpyDeviceToHost, s));
-    CHECK_HIP(hipStreamSynchronize(s));
-    ctx->line_stamps_clear = true;
+    int rc = read_back();
+    if (rc) return rc;
     out->traced = h[kLcTraced];
-    out->replayed = h[kLcReplayed];
+    out->replayed = h[kLcCut];
     out->voxels = h[kLcVoxels];
-    out->fail_tests = h[kLcWhyTest];
-    out->fail_labels = h[kLcWhyLabel];
     return MSCEER_OK;
 }
 

@@ -172,7 +172,183 @@ struct DirectLabels {
     __device__ void write(uint32_t c) { restr[c] = target; }
     __device__ bool ok() const { return true; }
     __device__ void stop_here(const CellGeom&, const V3<double>&, const V3<double>&, bool) {}
+    __device__ void leave() {}
 };
+
+// ---- tapes -------------------------------------------------------------------
+//
+// The path of a streamline depends on no label: labels only decide where it
+// stops and which of the cells it digitizes it reaches.  A tape is the
+// sequence of what a streamline would ask of the labels if nothing but its own
+// labels stopped it, and what the line does in the reference's order follows
+// from the tape and the labels other lines give alone (tape_chunk), without
+// tracing again.  Entries, 64 bits each: the cell (low word), and in the high
+// word the kind, the first-of-a-list flag and the slot of the line's previous
+// list entry of the same cell.
+//   kStay   a stop test at a step that stays in its voxel; the list of kStop
+//           entries behind it is what a stop there digitizes
+//   kExit   a stop test at the step that leaves a voxel; the kList entries
+//           behind it are digitized whether it stops or not
+//   kList   a digitized cell (in lists: the first labelled cell ends a list)
+//   kStop   as kList, applied only if the kStay test before them stops
+// A test repeated with no list entry of its cell in between asks the same
+// question again and is not recorded.  The first cell of a list carries the
+// target once the list is done (it had it, or takes it), so a test of a cell
+// that was first in an earlier list stops the line whatever other lines do:
+// the tape ends there (history: the last kHistory such cells; an older one
+// only makes the tape longer than it need be).
+// Tapes are chains of chunks of 64 slots: slot 0 holds the next chunk (low
+// word) and the number of entries (high word), slots 1.. the entries.
+constexpr uint32_t kStay = 0, kExit = 1, kList = 2, kStop = 3;
+constexpr int kKindShift = 29;
+constexpr uint32_t kFirst = 0x80000000u;     // first entry of a list
+constexpr uint32_t kNoPrev = 0x1FFFFFFFu;    // no earlier kList entry of the cell
+constexpr uint32_t kTapeChunk = 64;          // slots of a chunk
+constexpr uint32_t kMaxTapeChunks = 1024;    // chunks of one tape (longer lines are traced alone, in order)
+constexpr uint32_t kHistory = 32;
+
+struct TapePool {
+    uint64_t* slots;    // chunks * kTapeChunk
+    uint32_t chunks;
+    uint32_t* top;      // next free chunk
+};
+
+// Recording policy of a trace.  hist: kHistory words, hstride apart.
+struct TapeLabels {
+    const int8_t* restr;
+    int8_t target;
+    bool committed;      // earlier windows have labelled cells: a test of one ends the tape
+    TapePool pool;
+    uint32_t* hist;
+    uint32_t hstride;
+    uint32_t nhist = 0, last = kNoLine;
+    uint32_t head = kNoLine, chunk = kNoLine, fill = 0, nchunks = 0;
+    bool over = false, staying = false, asc = false;
+    const CellGeom* geom = nullptr;
+    V3<double> from{}, to{};
+    __device__ void append(uint32_t kind, uint32_t c) {
+        if (over) return;
+        if (chunk == kNoLine || fill == kTapeChunk - 1) {
+            const uint32_t at = nchunks < kMaxTapeChunks ? atomicAdd(pool.top, 1u) : kNoLine;
+            if (at >= pool.chunks) {
+                over = true;
+                return;
+            }
+            if (chunk == kNoLine) head = at;
+            else pool.slots[(uint64_t)chunk * kTapeChunk] = (uint64_t)fill << 32 | at;
+            chunk = at;
+            fill = 0;
+            nchunks++;
+        }
+        fill++;
+        pool.slots[(uint64_t)chunk * kTapeChunk + fill] = (uint64_t)(kind << kKindShift | kNoPrev) << 32 | c;
+    }
+    // kind: kList or kStop with the first-of-a-list flag folded in by the caller
+    __device__ void append_list(uint32_t kind, uint32_t c, bool first) {
+        append(kind, c);
+        if (first && !over) pool.slots[(uint64_t)chunk * kTapeChunk + fill] |= (uint64_t)kFirst << 32;
+    }
+    __device__ void finish() {
+        if (!over && chunk != kNoLine) pool.slots[(uint64_t)chunk * kTapeChunk] = (uint64_t)fill << 32 | kNoLine;
+    }
+    __device__ void stop_here(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool up) {
+        staying = true;
+        geom = &m;
+        from = a;
+        to = b;
+        asc = up;
+    }
+    __device__ void leave() { staying = false; }
+    __device__ bool test(uint32_t c) {
+        if (c == last) return false;
+        last = c;
+        append(staying ? kStay : kExit, c);
+        if (staying) {
+            uint32_t cells[6];
+            const int n = digitize_cells(*geom, from, to, asc, cells);
+            for (int k = 0; k < n; k++) append_list(kStop, cells[k], k == 0);
+        }
+        bool hit = committed && restr[c] == target;
+        const uint32_t n = nhist < kHistory ? nhist : kHistory;
+        for (uint32_t k = 0; k < n; k++) hit = hit || hist[k * hstride] == c;
+        return hit;
+    }
+    __device__ void list(const uint32_t* cells, int n) {
+        for (int k = 0; k < n; k++) {
+            append_list(kList, cells[k], k == 0);
+            if (cells[k] == last) last = kNoLine;
+        }
+        // an exit without a list: the next test is recorded again, so that no
+        // later list is taken for this exit's
+        if (n > 0) hist[(nhist++ % kHistory) * hstride] = cells[0];
+        else last = kNoLine;
+    }
+    __device__ bool ok() const { return !over; }
+};
+
+__device__ inline void digitize(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool asc, TapeLabels& lab) {
+    uint32_t cells[6];
+    lab.list(cells, digitize_cells(m, a, b, asc, cells));
+}
+
+// What a line does along its tape, chunk by chunk.
+struct TapeState {
+    bool broken = false;   // the list at hand met a labelled cell
+    uint32_t ending = 0;   // a test stopped the line: 1 its kStop list, 2 its kList list remains
+    bool begun = false;    // that list has begun
+};
+
+// Evaluates the entries of one chunk (bit k of a mask: slot k).  test /
+// exitm / stopm / first: kinds (neither test nor stopm: kList); lab: cells
+// that carry the target for this line (committed, or given by an earlier
+// line); prevm: entries with an earlier list entry of the same cell, whose
+// bit own(k, w) returns.  Returns the list entries whose cell carries the
+// target after them -- reached (labelled already, or labelled now) or
+// labelled by the line before; *stop: the slot at which the line ended, 0 if
+// it goes on.
+template <class Own>
+__device__ inline uint64_t tape_chunk(TapeState& s, uint32_t n, uint64_t test, uint64_t exitm, uint64_t stopm,
+                                      uint64_t first, uint64_t lab, uint64_t prevm, Own own, uint32_t* stop) {
+    const uint64_t all = n >= 63 ? ~1ull : ((1ull << (n + 1)) - 2ull);
+    *stop = 0;
+    if (!((lab | prevm) & all) && s.ending == 0 && !s.broken) return all & ~test & ~stopm;
+    uint64_t w = 0;
+    for (uint32_t k = 1; k <= n; k++) {
+        const uint64_t bit = 1ull << k;
+        const bool is_test = (test & bit) != 0, is_stop = (stopm & bit) != 0, is_first = (first & bit) != 0;
+        if (s.ending) {
+            const bool belongs = !is_test && (s.begun ? !is_first : (is_first && is_stop == (s.ending == 1)));
+            if (!belongs) {
+                *stop = k;
+                return w;
+            }
+            s.begun = true;
+        }
+        const bool mine = (prevm & bit) && own(k, w);
+        const bool labelled = (lab & bit) || mine;
+        if (is_test) {
+            if (labelled) {
+                s.ending = (exitm & bit) ? 2u : 1u;
+                s.begun = false;
+            }
+            continue;
+        }
+        if (is_first) s.broken = false;
+        if (is_stop && s.ending != 1) {
+            if (mine) w |= bit;
+            continue;
+        }
+        if (!s.broken || mine) w |= bit;
+        if (labelled) s.broken = true;
+    }
+    return w;
+}
+
+// ---- the window algorithm's label policies -----------------------------------
+//
+// A second realisation of the same order on the same traces (speculation with
+// footprints, replay of the components that interact), run by the host
+// emulation, which checks the tracing and digitizing code with it.
 
 // Footprints: every cell a speculative trace tests or labels, appended (with
 // repeats) to chunks of a shared pool, one chain per line (and a second chain
@@ -272,6 +448,7 @@ struct SpecLabels {
             claim(pstamp, cells[k]);
         }
     }
+    __device__ void leave() {}
     // End marks of the last chunks.
     __device__ void finish() {
         if (over) return;
@@ -362,6 +539,7 @@ struct ReplayLabels {
     }
     __device__ bool ok() const { return !bad; }
     __device__ void stop_here(const CellGeom&, const V3<double>&, const V3<double>&, bool) {}
+    __device__ void leave() {}
 };
 
 // Label the cells of digitize_cells in order; stop at the first one that
@@ -412,6 +590,8 @@ __device__ int advect_voxel(const VGrid& g, const CellGeom& m, Tracer<double>& t
         // instead of the whole voxel segment
         if ((int)t.cur.x == (int)t.old.x && (int)t.cur.y == (int)t.old.y && (int)t.cur.z == (int)t.old.z)
             lab.stop_here(m, start, t.cur, asc);
+        else
+            lab.leave();
         const int64_t cx = asc ? 2 * (int64_t)floor(t.cur.x) + 1 : 2 * (int64_t)floor(t.cur.x + 0.5);
         const int64_t cy = asc ? 2 * (int64_t)floor(t.cur.y) + 1 : 2 * (int64_t)floor(t.cur.y + 0.5);
         const int64_t cz = asc ? 2 * (int64_t)floor(t.cur.z) + 1 : 2 * (int64_t)floor(t.cur.z + 0.5);
