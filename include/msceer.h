@@ -76,7 +76,7 @@ typedef struct msceer_label_stats {
     int64_t reintegrated_fp64;  /* pass-3 re-integrations traced in FP64 (with MSCEER_FP32_FIRST: those escalated) */
     int64_t over_budget_fp64;   /* of those, stopped by the step budget */
     int64_t integrated_vertices;/* vertices the learned mask sent to integration (all if none) */
-    int32_t certain_sweeps;     /* rounds of the certain-region resolution (dependency depth) */
+    int32_t certain_sweeps;     /* sweeps of the certain-region flood enqueued */
     int32_t pass3_rounds;       /* launches of pass 3 (one persistent launch) */
     float ms_lstar;             /* base + constrained lower-star kernels */
     float ms_regions;           /* extremum graph + certain regions */
@@ -102,7 +102,7 @@ typedef struct msceer_label_stats {
     int64_t maxima;             /* needDSC2: critical hexes of the steepest pairing */
     int64_t saddles2;           /* needDSC2: critical quads */
     int64_t regions_dsc;        /* needDSC2: descending certain regions after simplification */
-    int32_t certain_sweeps_dsc; /* needDSC2: certain-region rounds */
+    int32_t certain_sweeps_dsc; /* needDSC2: the same */
     float ms_dsc;               /* needDSC2: the whole descending branch (beside the ascending one with needASC2) */
     float ms_dsc_wait;          /* needDSC2: time its end lies past the ascending branch's */
 } msceer_label_stats;

@@ -119,10 +119,6 @@ __global__ void fill_u8_kernel(uint8_t* p, int64_t n, uint8_t v) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = v;
 }
 
-// ---- certain regions --------------------------------------------------------
-
-// (The certain-region kernels follow the work-list helpers below.)
-
 // ---- streamline integration -------------------------------------------------
 
 // FP64 gradient field, as the reference computes it: FP32 coefficients times
@@ -425,15 +421,15 @@ ers_mark_kernel(VGrid g, const int32_t* __restrict__ label, uint8_t* __restrict_
     if (n) atomicAdd(&counts[3], n);
 }
 
-// ---- certain regions (GridSimplifiedExtremalRegionBuilder::BeginIntegration) ----
+// ---- certain regions of the SameBdry6 rule -----------------------------------
 //
-// A vertex takes the label shared by all of its earlier All6 neighbours if
-// they all carry one (gi_extrema_region_builder.h:806-857); the region seeds
-// are labelled from the start.  On the DAG "earlier neighbour -> vertex" this
-// has one solution, computed here in dependency order: a vertex is resolved
-// once its last unresolved earlier neighbour is, so every vertex is visited
-// once instead of once per sweep of a fixed-point iteration.  cnt[v] counts
-// the unresolved earlier neighbours of a non-seed vertex.
+// (The labelling's certain regions are in certain.hip.)  A vertex takes the
+// label shared by all of its earlier SameBdry6 neighbours if they all carry
+// one and the flood reaches it (below); the extrema are labelled from the
+// start.  On the DAG "earlier neighbour -> vertex" this has one solution,
+// computed here in dependency order: a vertex is resolved once its last
+// unresolved earlier neighbour is.  The reach rule looks at labels, so the
+// chains of certain.hip do not give it.
 //
 // Rounds in dependency order: round r resolves the vertices released in
 // round r - 1 and appends those it releases to a flat list for round r + 1
@@ -448,12 +444,11 @@ constexpr uint32_t kCntMask = 0xFFu;
 constexpr int kEarlierShift = 8, kLaterShift = 16;
 // SameBdry6 (not symmetric: a vertex on a face has no neighbour across it,
 // while the interior vertex beside it counts the face vertex): bits 22-27
-// flag the earlier vertices that count this one as their neighbour, and bit
-// 28 says the test below applies -- the priority flood reaches a vertex only
-// from such a vertex of its region (Enqueue_Later_Neighbors,
+// flag the earlier vertices that count this one as their neighbour: the
+// priority flood reaches a vertex only from such a vertex of its region
+// (Enqueue_Later_Neighbors,
 // gi_numeric_integrator_expanding_region_stop.h:108-123).
 constexpr int kReachShift = 22;
-constexpr uint32_t kAsym = 1u << 28;
 
 __device__ __forceinline__ int64_t dir_offset(const VGrid& g, int j) {
     const int64_t o = j < 2 ? 1 : (j < 4 ? (int64_t)g.X : g.sxy);
@@ -467,12 +462,12 @@ __device__ __forceinline__ uint64_t list_entry(uint32_t v, uint32_t meta) {
 }
 
 // The vertices with no earlier non-seed neighbour start the first list.
-// same_bdry: SameBdry6 neighbours (both along an axis, and only where the
-// vertex is interior along it: gi_regular_grid.h:232-265) instead of All6.
+// SameBdry6 neighbours: both along an axis, and only where the vertex is
+// interior along it (gi_regular_grid.h:232-265).
 __global__ void __launch_bounds__(kThreads)
 certain_init_kernel(const float* __restrict__ f, VGrid g, const uint8_t* __restrict__ seedmask,
                     uint32_t* __restrict__ cnt, uint64_t* __restrict__ out, uint32_t* __restrict__ out_count,
-                    uint32_t capacity, uint32_t* __restrict__ overflow, int same_bdry, int desc) {
+                    uint32_t capacity, uint32_t* __restrict__ overflow) {
     __shared__ uint64_t stage[kStage];
     __shared__ uint32_t s_n, s_base;
     if (threadIdx.x == 0) s_n = 0;
@@ -495,11 +490,11 @@ certain_init_kernel(const float* __restrict__ f, VGrid g, const uint8_t* __restr
         for (int j = 0; j < 6; j++) {
             if (!exists[j]) continue;
             const int a = j >> 1, cu = c3[a] + ((j & 1) ? -1 : 1);
-            const bool mine = !same_bdry || (c3[a] > 0 && c3[a] < n3[a] - 1);   // u is my neighbour
-            const bool theirs = !same_bdry || (cu > 0 && cu < n3[a] - 1);       // I am u's neighbour
+            const bool mine = c3[a] > 0 && c3[a] < n3[a] - 1;   // u is my neighbour
+            const bool theirs = cu > 0 && cu < n3[a] - 1;       // I am u's neighbour
             const int64_t u = v + dir_offset(g, j);
             const bool seed = seedmask[u] != 0;
-            if (ord_before(f, u, v, desc)) {
+            if (before(f, u, v)) {
                 if (mine) earlier |= 1u << j;
                 if (theirs) reach |= 1u << j;
                 if (!seed && (mine || theirs)) c++;
@@ -507,8 +502,7 @@ certain_init_kernel(const float* __restrict__ f, VGrid g, const uint8_t* __restr
                 later |= 1u << j;
             }
         }
-        uint32_t meta = c | earlier << kEarlierShift | later << kLaterShift;
-        if (same_bdry) meta |= reach << kReachShift | kAsym;
+        const uint32_t meta = c | earlier << kEarlierShift | later << kLaterShift | reach << kReachShift;
         cnt[v] = meta;
         if (c == 0) stage[atomicAdd(&s_n, 1u)] = list_entry((uint32_t)v, meta);
     }
@@ -554,7 +548,7 @@ certain_round_kernel(VGrid g, int32_t* __restrict__ label, uint32_t* __restrict_
                 else if (!has) { val = l[j]; has = true; }
                 else if (val != l[j]) ok = false;
             }
-            if (ok && has && (meta & kAsym)) {
+            if (ok && has) {
                 bool reached = false;
                 for (int j = 0; j < 6; j++)
                     if ((meta >> (kReachShift + j)) & 1u) reached = reached || label[v + dir_offset(g, j)] == val;
@@ -1684,10 +1678,10 @@ uint32_t resident_blocks(K kernel) {
 }  // namespace
 hipError_t launch_certain_init(const VGrid& g, const float* values, const uint8_t* seedmask, uint32_t* cnt,
                                uint64_t* out, uint32_t* out_count, uint32_t capacity, uint32_t* overflow,
-                               hipStream_t s, bool same_bdry, bool desc) {
+                               hipStream_t s) {
     const int64_t blocks = (g.verts() + kStage - 1) / kStage;
     hipLaunchKernelGGL(certain_init_kernel, dim3((uint32_t)blocks), dim3(kThreads), 0, s, values, g, seedmask, cnt,
-                       out, out_count, capacity, overflow, same_bdry ? 1 : 0, desc ? 1 : 0);
+                       out, out_count, capacity, overflow);
     return hipGetLastError();
 }
 hipError_t launch_certain_round(const VGrid& g, int32_t* label, uint32_t* cnt, const uint64_t* in,

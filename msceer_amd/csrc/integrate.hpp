@@ -92,8 +92,19 @@ struct WorkQueue {
     uint32_t* first_count;  // items pass 2 queued
 };
 hipError_t launch_pass2(const VGrid& g, const LabelBuffers& b, const WorkQueue& q, hipStream_t s);
-// Certain regions in dependency order (label[v] becomes the label shared by
-// all earlier All6 neighbours of v when they all carry one; seeds are
+// Certain regions by chains and a flood (certain.hip; seeds labelled
+// beforehand, -1 elsewhere): chain labels and bad vertices (parent: one int32
+// per vertex; scratch: certain_scratch_bytes()); one sweep of the flood
+// (sweep 0, 1, ...; active: three words, zero before sweep 0; the flood has
+// ended once sweep k left active[(k + 1) % 3] zero); -1 on what it reached.
+size_t certain_scratch_bytes(const VGrid& g);
+hipError_t launch_certain_chains(const VGrid& g, const float* values, const uint8_t* seedmask, bool desc,
+                                 int32_t* parent, int32_t* label, void* scratch, hipStream_t s);
+hipError_t launch_certain_flood(const VGrid& g, void* scratch, uint32_t sweep, uint32_t* active, hipStream_t s);
+hipError_t launch_certain_finish(const VGrid& g, void* scratch, int32_t* label, hipStream_t s);
+// Certain regions of the SameBdry6 rule in dependency order (label[v] becomes
+// the label shared by all earlier SameBdry6 neighbours of v when they all
+// carry one and one of them reaches v; seeds are
 // labelled beforehand; cnt: one uint32 per vertex; lists of 64-bit entries,
 // capacity entries each).  init lists the vertices
 // with no earlier non-seed neighbour; each round resolves the list `in` and
@@ -101,7 +112,7 @@ hipError_t launch_pass2(const VGrid& g, const LabelBuffers& b, const WorkQueue& 
 // (expected: about how many vertices `in` holds, which sizes the launch).
 hipError_t launch_certain_init(const VGrid& g, const float* values, const uint8_t* seedmask, uint32_t* cnt,
                                uint64_t* out, uint32_t* out_count, uint32_t capacity, uint32_t* overflow,
-                               hipStream_t s, bool same_bdry = false, bool desc = false);
+                               hipStream_t s);
 // NumericIntegratorExpandingRegionStop (minima, downhill): extrema (no
 // SameBdry6 neighbour before the vertex) labelled by their own ids, the rest
 // -1, counts[0] += extrema; stop states from labels (certain: terminal),

@@ -204,15 +204,12 @@ int run_integration(msceer_ctx* ctx, const VGrid& g, const LabelBuffers& b, cons
 
 namespace {
 
-// OnDemandAccurate's accuracy branches: the steepest pairing; the accurate
-// ascending labelling and its MIN boundary (needASC2); the digitized
-// 1-manifolds (needASC1, needDSC1); the conforming lower stars and ldir.
-// Certain regions from the labelled seeds (b.label, b.seedmask): rounds in
-// dependency order (certain_init / certain_round), enqueued in groups; a
-// read-back per group shows whether the next round's list is empty.  Uses
-// the frontier buffers (lists) and b.stamp; same_bdry: SameBdry6 neighbours.
-int run_certain_rounds(msceer_ctx* ctx, const VGrid& g, const float* d_values, const LabelBuffers& b, bool same_bdry,
-                       int* sweeps_out, bool desc = false) {
+// Certain regions of the SameBdry6 rule from the labelled seeds (b.label,
+// b.seedmask): rounds in dependency order (certain_init / certain_round),
+// enqueued in groups; a read-back per group shows whether the next round's
+// list is empty.  Uses the frontier buffers (lists) and b.stamp.
+int run_certain_rounds(msceer_ctx* ctx, const VGrid& g, const float* d_values, const LabelBuffers& b,
+                       int* sweeps_out) {
     hipStream_t s = ctx->stream;
     uint32_t* ctl = ctl_dev(ctx);
     const int64_t V = g.verts();
@@ -222,8 +219,7 @@ int run_certain_rounds(msceer_ctx* ctx, const VGrid& g, const float* d_values, c
     uint32_t* counts = ctl + kCtlRound;  // three rotating count words
     CHECK_HIP(launch_zero(counts, 3, s));
     CHECK_HIP(launch_zero(ctl + kCtlOverflow, 1, s));
-    CHECK_HIP(launch_certain_init(g, d_values, b.seedmask, b.stamp, lists[0], counts, lcap, ctl + kCtlOverflow, s,
-                                  same_bdry, desc));
+    CHECK_HIP(launch_certain_init(g, d_values, b.seedmask, b.stamp, lists[0], counts, lcap, ctl + kCtlOverflow, s));
     rc = read_ctl(ctx, 0, kCtlWords);
     if (rc) return rc;
     int k = 0;
@@ -262,6 +258,31 @@ int run_certain_rounds(msceer_ctx* ctx, const VGrid& g, const float* d_values, c
     if (rc) return rc;
     if (ctx->h_ctl[kCtlOverflow]) return MSCEER_ETOOBIG;
     *sweeps_out = done ? done : k;
+    return MSCEER_OK;
+}
+
+// Certain regions of the All6 rule from the labelled seeds (b.label,
+// b.seedmask): chains and the flood (certain.hip).  Sweeps are enqueued in
+// groups; one read-back per group shows whether the last one left work.  Uses
+// b.label2 and ctx->scan.
+int run_certain_flood(msceer_ctx* ctx, const VGrid& g, const float* d_values, const LabelBuffers& b, int* sweeps_out,
+                      bool desc) {
+    hipStream_t s = ctx->stream;
+    uint32_t* active = ctl_dev(ctx) + kCtlRound;
+    CHECK_HIP(ctx->scan.ensure(certain_scratch_bytes(g)));
+    CHECK_HIP(launch_zero(active, 3, s));
+    CHECK_HIP(launch_certain_chains(g, d_values, b.seedmask, desc, b.label2, b.label, ctx->scan.ptr, s));
+    constexpr uint32_t kFirstGroup = 16, kGroup = 16;
+    uint32_t k = 0;
+    for (uint32_t group = kFirstGroup;; group = kGroup) {
+        for (uint32_t j = 0; j < group; j++, k++) CHECK_HIP(launch_certain_flood(g, ctx->scan.ptr, k, active, s));
+        const int rc = read_ctl(ctx, kCtlRound, 3);
+        if (rc) return rc;
+        if (ctx->h_ctl[kCtlRound + k % 3] == 0) break;
+        if (k > (uint64_t)g.verts() + kGroup) return MSCEER_EHIP;  // every sweep but the last sets a bit
+    }
+    CHECK_HIP(launch_certain_finish(g, ctx->scan.ptr, b.label, s));
+    *sweeps_out = (int)k;
     return MSCEER_OK;
 }
 
@@ -388,7 +409,7 @@ int run_dsc(msceer_ctx* cx, const DscIn& in, msceer_label_stats& st) {
         CHECK_HIP(hipStreamSynchronize(s));  // host vectors go out of scope
     }
     int sweeps = 0;
-    rc = run_certain_rounds(cx, g, in.values, bd, false, &sweeps, true);
+    rc = run_certain_flood(cx, g, in.values, bd, &sweeps, true);
     if (rc) return rc;
     st.certain_sweeps_dsc = sweeps;
     if (!in.stop_r) {
@@ -411,6 +432,10 @@ int run_dsc(msceer_ctx* cx, const DscIn& in, msceer_label_stats& st) {
     return MSCEER_OK;
 }
 
+// OnDemandAccurate's accuracy branches: the steepest pairing; the accurate
+// ascending labelling and its MIN boundary (needASC2), the descending one
+// (needDSC2); the digitized 1-manifolds (needASC1, needDSC1); the conforming
+// lower stars and ldir.
 int ondemand_impl(msceer_ctx* ctx, const float* values, int64_t nx, int64_t ny, int64_t nz, float err_thr,
                   float grad_thr, int32_t max_iters, float presimp, uint32_t need, const uint8_t* integrate_mask,
                   uint8_t* grad_out, int32_t* labels_out, int32_t* labels_dsc_out, int8_t* restriction_out,
@@ -664,9 +689,8 @@ int ondemand_impl(msceer_ctx* ctx, const float* values, int64_t nx, int64_t ny, 
             rc = start_dsc(true);
             if (rc) return rc;
         }
-        // rounds in dependency order
         int sweeps = 0;
-        rc = run_certain_rounds(ctx, g, d_values, b, false, &sweeps);
+        rc = run_certain_flood(ctx, g, d_values, b, &sweeps, false);
         if (rc) return rc;
         st.certain_sweeps = sweeps;
         CHECK_HIP(hipEventRecord(ev[2], s));
@@ -1144,7 +1168,7 @@ extern "C" int msceer_expanding_region_stop(msceer_ctx* ctx, const float* values
     CHECK_HIP(launch_grad_field64(g, nb, s));
     CHECK_HIP(launch_ers_seeds(g, d_values, b.seedmask, b.label, counts, s));
     int sweeps = 0;
-    rc = run_certain_rounds(ctx, g, d_values, b, true, &sweeps);
+    rc = run_certain_rounds(ctx, g, d_values, b, &sweeps);
     if (rc) return rc;
     CHECK_HIP(launch_ers_state(g, b.label, b.dest, counts, s));
     // pass 1: label2 = the certain labels, and the label each streamline reaches
