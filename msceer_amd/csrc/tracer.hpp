@@ -136,6 +136,7 @@ struct Tracer {
     T gm, step;
     int bx, by, bz;
     bool near;
+    bool fresh;  // entered its voxel: the gradient and a fresh step length are due
     int iters;
 };
 
@@ -174,26 +175,36 @@ __device__ __forceinline__ void tracer_begin(Tracer<T, C>& t) {
     t.gr = trilin(t.c, t.cur.x - (T)t.bx, t.cur.y - (T)t.by, t.cur.z - (T)t.bz);
     t.gm = sqrt(t.gr.x * t.gr.x + t.gr.y * t.gr.y + t.gr.z * t.gr.z);
     t.step = (T)kMaxStep / t.gm;
+    t.fresh = false;
 }
 
 // One iteration.  kNone: the streamline goes on (moved: it entered the voxel
 // of vertex `next`); kHitPreassigned (next: the vertex reached), kLowGradient
 // and kOverMax end it; kOutOfVoxel asks the caller to enter the voxel of the
 // position (only a position changed outside a step could lead there).
+//
+// The gradient, its magnitude and the step cap are evaluated at the top of
+// every iteration, whatever the lane did in the one before (entered a voxel,
+// moved inside it, or halved its step, where they come out as they were), so
+// that the lanes of a wave share one evaluation; a gradient evaluated apart
+// for the lanes that entered a voxel and those that moved inside one cost both
+// paths in nearly every iteration (500x380x260 noise: pass 1 16.9 -> 15.8 ms,
+// pass 3 21.7 -> 19.8 ms).
 template <typename T, class C>
 __device__ __forceinline__ int tracer_iterate(const GradSrc<T>& src, const VGrid& g,
                                               const uint8_t* __restrict__ dest, bool stop_on_assigned, T dir,
                                               T gthr, T ethr, Tracer<T, C>& t, int64_t& next, bool& moved) {
     moved = false;
     if (!(t.iters-- > 0)) return kOverMax;
-    if (!(t.old.x == t.cur.x && t.old.y == t.cur.y && t.old.z == t.cur.z)) {
-        if ((int)t.cur.x != (int)t.old.x || (int)t.cur.y != (int)t.old.y || (int)t.cur.z != (int)t.old.z)
-            return kOutOfVoxel;
-        t.gr = trilin(t.c, t.cur.x - (T)t.bx, t.cur.y - (T)t.by, t.cur.z - (T)t.bz);
-        t.gm = sqrt(t.gr.x * t.gr.x + t.gr.y * t.gr.y + t.gr.z * t.gr.z);
-        if (t.gm * t.step > (T)kMaxStep) t.step = (T)kMaxStep / t.gm;
-        t.old = t.cur;
-    }
+    const bool went = !(t.old.x == t.cur.x && t.old.y == t.cur.y && t.old.z == t.cur.z) && !t.fresh;
+    if (went && ((int)t.cur.x != (int)t.old.x || (int)t.cur.y != (int)t.old.y || (int)t.cur.z != (int)t.old.z))
+        return kOutOfVoxel;
+    t.gr = trilin(t.c, t.cur.x - (T)t.bx, t.cur.y - (T)t.by, t.cur.z - (T)t.bz);
+    t.gm = sqrt(t.gr.x * t.gr.x + t.gr.y * t.gr.y + t.gr.z * t.gr.z);
+    const T cap = (T)kMaxStep / t.gm;
+    if (t.fresh || (went && t.gm * t.step > (T)kMaxStep)) t.step = cap;
+    t.fresh = false;
+    t.old = t.cur;
     if (t.gm < gthr) return kLowGradient;
     // dir = -1: ascending manifolds, flow downhill; +1: descending, uphill
     const T s = dir * t.step, hs = (dir * (T)0.5) * t.step;
@@ -209,7 +220,7 @@ __device__ __forceinline__ int tracer_iterate(const GradSrc<T>& src, const VGrid
     }
     t.cur = {t.cur.x + two.x, t.cur.y + two.y, t.cur.z + two.z};
     if (t.near) { t.cur.x = clampc(t.cur.x, g.X); t.cur.y = clampc(t.cur.y, g.Y); t.cur.z = clampc(t.cur.z, g.Z); }
-    const T grow = t.step * (T)1.8, cap = (T)kMaxStep / t.gm;
+    const T grow = t.step * (T)1.8;
     t.step = grow < cap ? grow : cap;
     int nx, ny, nz;
     next = nearest_xyz(g, t.cur, t.near, nx, ny, nz);
@@ -222,7 +233,7 @@ __device__ __forceinline__ int tracer_iterate(const GradSrc<T>& src, const VGrid
     if (d == kCertainTerminal || (stop_on_assigned && d == kAssigned)) return kHitPreassigned;
     if (leave) {
         t.iters--;  // the iteration that leaves the voxel
-        tracer_begin(t);
+        t.fresh = true;
         moved = true;
     }
     return kNone;
@@ -245,7 +256,7 @@ __device__ __forceinline__ void tracer_start(const GradSrc<T>& src, const VGrid&
     t.cur = {(T)x, (T)y, (T)z};
     t.iters = max_iters;
     tracer_load(src, g, t, x, y, z);
-    tracer_begin(t);
+    t.fresh = true;
 }
 
 // ---- FP32 tracer in voxel-local coordinates, with decision margins ---------
