@@ -68,10 +68,18 @@ hipError_t launch_seed_scatter(const int32_t* seed_vert, const int32_t* seed_lab
                                hipStream_t s);
 // dest = UNASSIGNED where label == -1 else CERTAIN_TERMINAL; redo = 0; stamp = no claim.
 hipError_t launch_dest_init(const VGrid& g, const LabelBuffers& b, hipStream_t s);
+// Seeds of one pass-1 level (at least one item of room per vertex), their
+// number and the claim counters of the list's eighths.
+constexpr int kSeedQueues = 8;  // one per XCD
+struct SeedList {
+    uint32_t* items;
+    uint32_t* count;
+    uint32_t* heads;  // kSeedQueues
+};
 // Pass 1 at one level of the coarse-to-fine order (sign -1: flow downhill to
 // minima, +1: uphill to maxima; the same for pass 3).
-hipError_t launch_pass1(const VGrid& g, const LabelBuffers& b, int stride, bool first_level, float gthr, float ethr,
-                        int max_iters, int sign, hipStream_t s);
+hipError_t launch_pass1(const VGrid& g, const LabelBuffers& b, const SeedList& seeds, int stride, bool first_level,
+                        float gthr, float ethr, int max_iters, int sign, hipStream_t s);
 // End of a pass-1 level: its seeds and claimed path vertices become assigned
 // (claims in b.stamp, all kNoClaim on entry; reset to zero after the last
 // level for passes 2 and 3).

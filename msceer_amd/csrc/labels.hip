@@ -152,9 +152,11 @@ int run_integration(msceer_ctx* ctx, const VGrid& g, const LabelBuffers& b, cons
     int top = 1;
     while (top * 2 <= kPass1TopStride && top * 2 < max_dim) top *= 2;
     CHECK_HIP(hipEventRecord(ctx->ev[12], s));
+    const SeedList seeds{ctx->front1.as<uint32_t>(), ctl + kCtlRound, ctl + kCtlRound + 1};
+    if (ctx->front1.bytes < sizeof(uint32_t) * (size_t)V) return MSCEER_EHIP;  // (never: it holds 2 V words)
     for (int stride = top; stride >= 1; stride /= 2) {
-        CHECK_HIP(launch_pass1(g, b, stride, stride == top, grad_thr, err_thr, std::min(max_iters, kPass1Budget),
-                               sign, s));
+        CHECK_HIP(launch_pass1(g, b, seeds, stride, stride == top, grad_thr, err_thr,
+                               std::min(max_iters, kPass1Budget), sign, s));
         CHECK_HIP(launch_pass1_finish(g, b, stride, stride == top, stride == 1, s));
     }
     CHECK_HIP(hipEventRecord(ctx->ev[13], s));
