@@ -59,3 +59,16 @@ def test_device_pointers_and_one_output(ctx):
     hipmem.synchronize()
     m = dm.download(np.int32, f.size).reshape(f.shape)
     assert (m == mounts).all()
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 2), (2, 2, 70), (2, 70, 2), (70, 2, 2), (5, 4, 65), (4, 9, 64), (6, 5, 129)])
+def test_tile_edges_against_oracle(ctx, shape):
+    # paths followed inside 64x4x4 tiles, extents of one hex (coinciding strides) among them
+    f = synth.Stream(44).normal(int(np.prod(shape))).reshape(shape).astype(np.float32)
+    g = oracle_lib.steepest_grad(f)
+    print(shape, flush=True)
+    b, m, c = msc.msc_base(g, shape, ctx=ctx)
+    rb, rm, rc = oracle_lib.msc_base(g, shape)
+    assert (c == rc).all()
+    assert (b == rb).all(), int((b != rb).sum())
+    assert (m == rm).all(), int((m != rm).sum())
