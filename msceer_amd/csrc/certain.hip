@@ -203,8 +203,13 @@ __global__ void __launch_bounds__(kThreads)
 flood_kernel(Geo g, Planes p, uint32_t* __restrict__ dirty, uint32_t sweep, uint32_t* __restrict__ active) {
     // active: three rotating words; this sweep reads active[sweep % 3]
     if (blockIdx.x == 0 && threadIdx.x == 0) active[(sweep + 2) % 3] = 0;
-    if (sweep > 0 && (active[sweep % 3] == 0 || dirty[blockIdx.x] != sweep)) return;
     __shared__ uint64_t rows[2][kThreads];
+    // one lane decides for the work-group: a neighbour of the same sweep may be
+    // writing the mark, and waves that read it apart could part ways here
+    __shared__ int s_run;
+    if (threadIdx.x == 0) s_run = sweep == 0 || (active[sweep % 3] != 0 && dirty[blockIdx.x] == sweep);
+    __syncthreads();
+    if (!s_run) return;
     const int w = (int)(blockIdx.x % (uint32_t)g.words);
     const int q = (int)(blockIdx.x / (uint32_t)g.words);
     const int ty = q % g.ty, tz = q / g.ty;
