@@ -62,7 +62,7 @@ typedef struct msceer_timing {
     float lstar_ms;        /* lower-star pairing kernel */
     float ldir_ms;         /* ascending-manifold-dimension (ldir) passes */
     float total_ms;        /* whole device-side call */
-    int32_t ldir_rounds;   /* frontier rounds used by the ldir passes */
+    int32_t ldir_rounds;   /* flood sweeps launched by the ldir passes */
     int64_t critical[4];   /* critical cells by dimension */
 } msceer_timing;
 
@@ -145,7 +145,7 @@ int msceer_lstar_grad(msceer_ctx* ctx, const float* values, int64_t nx, int64_t 
  * reference: for callers that cannot allocate device memory (tight serving
  * loops, harnesses that forbid hipMalloc).  Device pointers only (values in,
  * grad_out out); every scratch buffer (control words, critical-cell lists,
- * frontiers, ldir records) comes from one static 48 MiB array per GPU, so a
+ * ldir planes and bits) comes from one static 48 MiB array per GPU, so a
  * volume whose scratch would exceed it returns MSCEER_ETOOBIG (up to about
  * 1.3 million vertices fit, e.g. 128x128x64).  The lower-star brick shape is
  * the one an earlier msceer_lstar_grad tuned for this x extent, else 64x2x2;
@@ -287,10 +287,9 @@ int msceer_batch(msceer_ctx* ctx, msceer_volume* vols, int32_t n, int32_t stream
  * volumes form groups of fewer than 2^32 - 1 cells in all and, if
  * max_group_verts > 0, at most that many vertices (a single larger volume is
  * a group of its own).  Each group runs as one launch per stage for all its
- * volumes (lower star, ldir records, the two ldir passes' frontier rounds on
- * two streams, finish), captured once in a hipGraph and replayed on later
- * calls with the same shapes (and, with device pointers, the same
- * addresses); the lower-star launch (brick shape; a work-group per brick, or
+ * volumes (lower star, ldir planes, flood sweeps, finish), captured once in a
+ * hipGraph and replayed on later calls with the same shapes (and, with device
+ * pointers, the same addresses); the lower-star launch (brick shape; a work-group per brick, or
  * persistent work-groups claiming bricks from per-XCD queues in chunks) is
  * tuned on a group's first call unless msceer_set_autotune fixed the shape.
  * One host synchronisation per group.  Flags: MSCEER_DEVICE_PTRS (values and
@@ -305,11 +304,11 @@ typedef struct msceer_batch_stats {
     int32_t groups;        /* groups the last call ran */
     int32_t replays;       /* graph launches */
     int32_t captures;      /* graphs captured (first calls, or after a plan changed) */
-    int32_t eager_rounds;  /* frontier rounds and sweeps run after a replay left work */
+    int32_t eager_rounds;  /* flood sweeps run after a replay left work */
     int32_t shape;         /* lower-star brick shape (last group), as msceer_lstar_brick */
     int32_t blocks;        /* persistent work-groups, 0: a work-group per brick */
     int32_t chunk;         /* bricks per queue claim */
-    int32_t rounds;        /* frontier rounds per pass in the graph */
+    int32_t rounds;        /* flood sweeps in the graph */
     int64_t critical[4];   /* critical cells by dimension, all volumes */
     float ms_gpu;          /* device time of the groups (events around each replay and what followed) */
 } msceer_batch_stats;

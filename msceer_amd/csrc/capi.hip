@@ -52,65 +52,6 @@ MList front_list(msceer_ctx* ctx, const ListCaps& c, int k) {
     return MList{buf, ctl_dev(ctx) + kCtlRound + (k % 3) * kCountWords, c.front_sub, c.front_spill};
 }
 
-// One ldir pass (1: from the critical edges, 2: from the critical quads).
-// Rounds are enqueued in groups without host synchronisation (each reads its
-// counts on the device); after each group one read-back shows whether the
-// frontier emptied.  The first group is short: the start round's work-groups
-// usually finish their whole manifolds, and the round after it the rest.  A sweep rebuilds the frontier after any overflow of the
-// start list or of a frontier.
-int ldir_pass(msceer_ctx* ctx, const Dims& d, uint8_t* grad, const LdirScratch& ls, int pass, const MList& start,
-              bool start_valid, const ListCaps& caps, int* rounds) {
-    uint32_t* ctl = ctl_dev(ctx);
-    uint32_t* overflow = ctl + kCtlOverflow;
-    void* scratch = ctx->ldir.ptr;
-    auto front = [&](int k) { return front_list(ctx, caps, k); };
-    auto host_total = [&](int k) { return list_total(ctx->h_ctl + kCtlRound + (k % 3) * kCountWords, front(k)); };
-    constexpr int kFirstGroup = 2, kGroup = 8;
-    int group = kFirstGroup;
-    MList in = start;
-    bool is_start = true;
-    int k = 0;
-    bool need_sweep = !start_valid;
-    CHECK_HIP(launch_zero(front(0).counts, kCountWords, ctx->stream));
-    CHECK_HIP(launch_zero(overflow, 1, ctx->stream));
-    for (int guard = 0; guard < 100000; guard++) {
-        if (need_sweep) {
-            CHECK_HIP(launch_zero(front(k).counts, kCountWords, ctx->stream));
-            CHECK_HIP(launch_zero(overflow, 1, ctx->stream));
-            CHECK_HIP(launch_ldir_sweep(d, grad, scratch, ls, pass, front(k), overflow, ctx->stream));
-            int rc = read_ctl(ctx, 0, kCtlWords);
-            if (rc) return rc;
-            need_sweep = ctx->h_ctl[kCtlOverflow] != 0;
-            (*rounds)++;
-            const uint64_t n = host_total(k);
-            if (n == 0 && !need_sweep) return MSCEER_OK;
-            CHECK_HIP(launch_zero(overflow, 1, ctx->stream));
-            in = front(k);
-            is_start = false;
-            k++;
-            CHECK_HIP(launch_zero(front(k).counts, kCountWords, ctx->stream));
-        }
-        for (int j = 0; j < group; j++) {
-            const MList out = front(k);
-            CHECK_HIP(launch_ldir_round(d, scratch, ls, pass, is_start, in, out, front(k + 1).counts, overflow,
-                                        ctx->stream));
-            (*rounds)++;
-            in = out;
-            is_start = false;
-            k++;
-        }
-        group = kGroup;
-        int rc = read_ctl(ctx, 0, kCtlWords);
-        if (rc) return rc;
-        if (ctx->h_ctl[kCtlOverflow]) {
-            need_sweep = true;
-            continue;
-        }
-        if (host_total(k - 1) == 0) return MSCEER_OK;
-    }
-    return MSCEER_EHIP;
-}
-
 // Critical lists: a quarter of the vertices per sub-list set, spill for as
 // many again as there are vertices; frontiers: the vertex count in sub-lists
 // and as much again in spill.  Entries are cell ids (< 2^32).
@@ -184,27 +125,35 @@ int ensure_lists(msceer_ctx* ctx, const Dims& d, ListCaps* caps) {
     return MSCEER_OK;
 }
 
-int run_ldir(msceer_ctx* ctx, const Dims& d, uint8_t* grad, const ListCaps& caps, bool lists_ok, int* rounds) {
+// The sweeps are enqueued in groups with the finish behind them, which does
+// nothing while the floods are not done; one read-back per group shows whether
+// the last sweep left work for another.
+int run_ldir(msceer_ctx* ctx, const Dims& d, uint8_t* grad, int* rounds) {
+    hipStream_t s = ctx->stream;
     LdirScratch ls{};
     CHECK_HIP(ctx->ldir.ensure(ldir_scratch_bytes(d, &ls)));
-    CHECK_HIP(launch_ldir_records(d, grad, ctx->ldir.ptr, ls, ctx->stream));
-    int rc = ldir_pass(ctx, d, grad, ls, 1, crit_list(ctx, caps, 0), lists_ok, caps, rounds);
-    if (rc) return rc;
-    rc = ldir_pass(ctx, d, grad, ls, 2, crit_list(ctx, caps, 1), lists_ok, caps, rounds);
-    if (rc) return rc;
-    CHECK_HIP(launch_ldir_finish(d, grad, ctx->ldir.ptr, ls, ctx->stream));
-    return MSCEER_OK;
+    uint32_t* active = ctl_dev(ctx) + kCtlRound;
+    CHECK_HIP(launch_ldir_planes(d, grad, ctx->ldir.ptr, ls, active, s));
+    constexpr uint32_t kGroup = 12;
+    for (uint32_t k = 0;;) {
+        for (uint32_t j = 0; j < kGroup; j++, k++) CHECK_HIP(launch_ldir_flood(d, ctx->ldir.ptr, ls, k, active, s));
+        CHECK_HIP(launch_ldir_finish(d, grad, ctx->ldir.ptr, ls, k, active, s));
+        const int rc = read_ctl(ctx, 0, kCtlWords);
+        if (rc) return rc;
+        *rounds = (int)k;
+        if (ctx->h_ctl[kCtlRound + k % 3] == 0) return MSCEER_OK;
+        if (k > 6 * d.verts + kGroup) return MSCEER_EHIP;  // every sweep but the last sets a bit
+    }
 }
 
 int lstar_grad_device(msceer_ctx* ctx, const Dims& d, const float* d_values, uint8_t* d_grad, uint8_t* host_out,
                       uint32_t flags) {
     const bool timing = flags & MSCEER_TIMING;
     hipStream_t s = ctx->stream;
-    // critical-cell lists and frontiers: sized to the volume, capped; any
-    // overflow falls back to a sweep
-    ListCaps caps{};
-    int rc = ensure_lists(ctx, d, &caps);
-    if (rc) return rc;
+    // critical-cell lists, which the lower-star kernel fills: sized to the volume
+    const ListCaps caps = list_caps(d);
+    CHECK_HIP(ctx->lists.ensure(list_bytes(caps)));
+    int rc = MSCEER_OK;
     uint32_t* ctl = ctl_dev(ctx);
     const MList list1 = crit_list(ctx, caps, 0), list2 = crit_list(ctx, caps, 1);
 
@@ -221,24 +170,19 @@ int lstar_grad_device(msceer_ctx* ctx, const Dims& d, const float* d_values, uin
     if (timing) CHECK_HIP(hipEventRecord(ctx->ev[1], s));
     CHECK_HIP(launch_lstar(d, b, s, shape));
     if (timing) CHECK_HIP(hipEventRecord(ctx->ev[2], s));
-    rc = read_ctl(ctx, 0, kCtlWords);
-    if (rc) return rc;
     msceer_timing t{};
-    for (int i = 0; i < kSubs; i++)
-        for (int k = 0; k < 4; k++) t.critical[k] += ctx->h_ctl[kCtlStats + 4 * i + k];
-    const bool lists_ok = ctx->h_ctl[kCtlOverflow] == 0;
-
     int rounds = 0;
     if (timing) CHECK_HIP(hipEventRecord(ctx->ev[3], s));
-    if (flags & MSCEER_TILED_LAYOUT) {
-        CHECK_HIP(launch_clear_ldir_bits(d_grad, (int64_t)d.cells, s));
-    } else if (!(flags & MSCEER_SKIP_LDIR)) {
-        rc = run_ldir(ctx, d, d_grad, caps, lists_ok, &rounds);
-        if (rc) return rc;
-    }
+    const bool ldir = !(flags & (MSCEER_TILED_LAYOUT | MSCEER_SKIP_LDIR));
+    if (flags & MSCEER_TILED_LAYOUT) CHECK_HIP(launch_clear_ldir_bits(d_grad, (int64_t)d.cells, s));
+    if (ldir) rc = run_ldir(ctx, d, d_grad, &rounds);
+    else rc = read_ctl(ctx, 0, kCtlWords);
+    if (rc) return rc;
+    for (int i = 0; i < kSubs; i++)
+        for (int k = 0; k < 4; k++) t.critical[k] += ctx->h_ctl[kCtlStats + 4 * i + k];
     if (timing) CHECK_HIP(hipEventRecord(ctx->ev[4], s));
     if (host_out) CHECK_HIP(hipMemcpyAsync(host_out, d_grad, d.cells, hipMemcpyDeviceToHost, s));
-    CHECK_HIP(hipStreamSynchronize(s));
+    if (host_out || timing) CHECK_HIP(hipStreamSynchronize(s));  // (the read-back waited for the rest)
     if (timing) {
         CHECK_HIP(hipEventElapsedTime(&t.lstar_ms, ctx->ev[1], ctx->ev[2]));
         CHECK_HIP(hipEventElapsedTime(&t.ldir_ms, ctx->ev[3], ctx->ev[4]));

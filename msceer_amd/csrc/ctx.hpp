@@ -155,8 +155,6 @@ int ensure_lists(msceer_ctx* ctx, const Dims& d, ListCaps* caps);
 MList crit_list(msceer_ctx* ctx, const ListCaps& c, int which);
 // Frontier k of a chain of rounds: buffer k % 2, count array k % 3.
 MList front_list(msceer_ctx* ctx, const ListCaps& c, int k);
-int ldir_pass(msceer_ctx* ctx, const Dims& d, uint8_t* grad, const LdirScratch& ls, int pass, const MList& start,
-              bool start_valid, const ListCaps& caps, int* rounds);
 // Brick shape for the lower-star kernel on this volume: tuned on first use of
 // an x extent (times every shape on the given buffers; call before the
 // control block is cleared for the real launch).
@@ -166,8 +164,9 @@ int tuned_shape(msceer_ctx* ctx, const Dims& d, int fallback);
 // Resolves the device address of the allocation-free entry point's scratch
 // array on `device` (current), once per device.
 int noalloc_setup(int device);
-// ldir passes on a .grad whose lstar pass filled the critical lists.
-int run_ldir(msceer_ctx* ctx, const Dims& d, uint8_t* grad, const ListCaps& caps, bool lists_ok, int* rounds);
+// ldir passes on a .grad in device memory; ends with a read-back of the whole
+// control block (h_ctl), with all that was enqueued before it done.
+int run_ldir(msceer_ctx* ctx, const Dims& d, uint8_t* grad, int* rounds);
 // Capacities of the critical lists and frontiers of a volume, and the bytes
 // ensure_lists gives them (two lists, two frontiers).
 ListCaps list_caps(const Dims& d);

@@ -3,18 +3,16 @@
 // hipGraph and replayed.
 //
 // A group is a run of consecutive volumes with fewer than 2^32 - 1 cells in
-// all (frontier items are 32-bit), optionally capped in vertices.  Its
+// all (listed cells are 32-bit), optionally capped in vertices.  Its
 // pipeline: clear the control block; lower-star bricks of every volume (one
 // launch: a work-group per brick, or persistent work-groups over the claim
-// queues, whichever the tuner measured faster); the ldir records of every
-// volume (one launch); pass 1 and pass 2 of the ldir walks as two chains of R
-// frontier rounds on two streams (the passes are independent until the
-// finish); the finish of every volume (one launch).  A round whose frontier
-// is empty returns at once, so R rounds cover every walk that ends within R.
-// After a replay one read-back of the control block shows whether a list
-// overflowed or a frontier is left; then the pass goes on eagerly (rounds,
-// sweeps after an overflow) and the finish runs again (it writes every ldir
-// bit from the visited bitmaps alone), and the next capture takes more rounds.
+// queues, whichever the tuner measured faster); the ldir planes of every
+// volume (one launch); R sweeps of the ldir floods; the finish of every volume
+// (one launch).  A sweep after one that changed nothing returns at once, so R
+// sweeps cover every flood that ends within R.  After a replay one read-back of
+// the control block shows whether a flood is left; then sweeps go on eagerly
+// and the finish (which does nothing while a flood is left) is launched again,
+// and the next capture takes more sweeps.
 //
 // Per group and call: the captured graph, keyed by the group's volume shapes,
 // buffer addresses and launch parameters; the tuning (brick shape, persistent
@@ -43,15 +41,15 @@ namespace {
 enum GCtl : int {
     kGList1 = 0,                           // count arrays of the critical lists
     kGList2 = kCountWords,
-    kGRound = 2 * kCountWords,             // 3 count arrays per pass (pass p at kGRound + 3 (p - 1) kCountWords)
-    kGStats = 8 * kCountWords,             // kSubs * 4 critical counts
-    kGOverflow = 8 * kCountWords + 4 * kSubs,  // lists, pass 1, pass 2
+    kGActive = 2 * kCountWords,            // three rotating words of the floods
+    kGStats = 2 * kCountWords + 4,         // kSubs * 4 critical counts
+    kGOverflow = kGStats + 4 * kSubs,      // a critical list ran out of room
     kGQueue = kGOverflow + 4,              // kQueues claim counters
     kGWords = kGQueue + kQueues
 };
 
-constexpr uint32_t kMaxItems = 0xFFFFFFFEu;  // cells of a group (kNoItem is 0xFFFFFFFF)
-constexpr int kDefaultRounds = 3;
+constexpr uint32_t kMaxItems = 0xFFFFFFFEu;  // cells of a group
+constexpr int kDefaultRounds = 12;           // sweeps in a first capture
 constexpr int kMaxPlans = 4;
 
 __global__ void times_init_kernel(unsigned long long* t, uint32_t n) {
@@ -73,9 +71,8 @@ struct GroupLayout {
     int first, count;  // volumes [first, first + count)
     uint64_t verts, cells;
     // host copies of the unit tables
-    std::vector<uint32_t> brick_first[kLstarBricks], tile_first, item_first;
-    size_t ldir_bytes = 0, bits_offset = 0;  // ldir scratch: records, then every volume's bitmaps
-    uint64_t bit_words = 0;
+    std::vector<uint32_t> brick_first[kLstarBricks], tile_first, flood_first, item_first;
+    size_t ldir_bytes = 0, dirty_off = 0;  // ldir scratch: every volume's planes and bits, then the tile marks
     std::vector<LdirScratch> ls;          // per volume, offsets from the group's ldir buffer
     std::vector<size_t> vals_off, grad_off;  // packed host-staging offsets (bytes)
     size_t vals_bytes = 0, grad_bytes = 0;
@@ -95,9 +92,8 @@ struct GroupPlan {
 }  // namespace
 
 struct BatchState {
-    hipStream_t side = nullptr;  // second stream (pass 2)
-    hipEvent_t fork = nullptr, join = nullptr, t0 = nullptr, t1 = nullptr;
-    DevBuf vals, grad, ldir, lists, fronts, ctl, times;
+    hipEvent_t t0 = nullptr, t1 = nullptr;
+    DevBuf vals, grad, ldir, lists, ctl, times;
     uint64_t generation = 0;  // bumped whenever a shared buffer moves (captured graphs then stale)
     std::list<GroupPlan> plans;  // most recent first
     std::map<std::string, LaunchTune> tunes;
@@ -148,14 +144,6 @@ MList glist(BatchState& s, const ListCaps& c, int which) {
                  c.list_spill};
 }
 
-// Frontier k of pass p: buffer (p - 1) * 2 + k % 2, count array k % 3.
-MList gfront(BatchState& s, const ListCaps& c, int pass, int k) {
-    const size_t per = (size_t)c.front_sub * kSubs + c.front_spill;
-    uint32_t* buf = s.fronts.as<uint32_t>() + ((size_t)(pass - 1) * 2 + (size_t)(k % 2)) * per;
-    return MList{buf, s.ctl.as<uint32_t>() + kGRound + (3 * (pass - 1) + k % 3) * kCountWords, c.front_sub,
-                 c.front_spill};
-}
-
 std::string shapes_key(const msceer_volume* v, const GroupLayout& g) {
     std::string k;
     char buf[64];
@@ -171,12 +159,12 @@ void layout(const msceer_volume* vols, GroupLayout& g) {
     const int n = g.count;
     for (int sh = 0; sh < kLstarBricks; sh++) g.brick_first[sh].assign(n + 1, 0);
     g.tile_first.assign(n + 1, 0);
+    g.flood_first.assign(n + 1, 0);
     g.item_first.assign(n + 1, 0);
     g.ls.resize(n);
     g.vals_off.resize(n);
     g.grad_off.resize(n);
-    size_t rec = 0, bits = 0, vo = 0, go = 0;
-    std::vector<size_t> bits_at(n);
+    size_t at = 0, vo = 0, go = 0;
     for (int i = 0; i < n; i++) {
         const msceer_volume& v = vols[g.first + i];
         const Dims d = make_dims(v.nx, v.ny, v.nz);
@@ -186,37 +174,24 @@ void layout(const msceer_volume* vols, GroupLayout& g) {
             const uint64_t nb = (uint64_t)((d.X + bx - 1) / bx) * ((d.Y + by - 1) / by) * ((d.Z + bz - 1) / bz);
             g.brick_first[sh][i + 1] = g.brick_first[sh][i] + (uint32_t)nb;
         }
-        uint32_t ntx, nty, nt;
-        ldir_tiles(d, &ntx, &nty, &nt);
-        g.tile_first[i + 1] = g.tile_first[i] + nt;
+        g.tile_first[i + 1] = g.tile_first[i] + ldir_tiles(d);
+        g.flood_first[i + 1] = g.flood_first[i] + ldir_flood_tiles(d);
         g.item_first[i + 1] = g.item_first[i] + (uint32_t)d.cells;
         LdirScratch one{};
         const size_t total = ldir_scratch_bytes(d, &one);
-        const size_t bw = total - one.bits2_off;  // bytes of one bitmap (padded)
-        // records of the volume at `rec`, its two bitmaps at `bits` (placed after all records)
-        g.ls[i].rec1_off = rec + one.rec1_off;
-        g.ls[i].rec2_off = rec + one.rec2_off;
-        g.ls[i].bit_words = one.bit_words;
-        bits_at[i] = bits;
-        rec += one.bits1_off;
-        bits += 2 * bw;
+        g.ls[i] = one;
+        g.ls[i].rec1_off += at;
+        g.ls[i].rec2_off += at;
+        g.ls[i].bits1_off += at;
+        g.ls[i].bits2_off += at;
+        at += total;
         g.vals_off[i] = vo;
         g.grad_off[i] = go;
         vo += (sizeof(float) * d.verts + 255) & ~(size_t)255;
         go += (d.cells + 255) & ~(size_t)255;
     }
-    g.bits_offset = rec;
-    for (int i = 0; i < n; i++) {
-        const msceer_volume& v = vols[g.first + i];
-        const Dims d = make_dims(v.nx, v.ny, v.nz);
-        LdirScratch one{};
-        const size_t total = ldir_scratch_bytes(d, &one);
-        const size_t bw = total - one.bits2_off;
-        g.ls[i].bits1_off = rec + bits_at[i];
-        g.ls[i].bits2_off = rec + bits_at[i] + bw;
-    }
-    g.bit_words = bits / 4;
-    g.ldir_bytes = rec + bits;
+    g.dirty_off = at;
+    g.ldir_bytes = at + 2 * sizeof(uint32_t) * (size_t)g.flood_first[n];
     g.vals_bytes = vo;
     g.grad_bytes = go;
 }
@@ -233,20 +208,18 @@ int upload_tables(msceer_ctx* ctx, BatchState& s, const msceer_volume* vols, con
         GVol& o = gv[i];
         o.values = dev ? v.values : reinterpret_cast<const float*>(s.vals.as<uint8_t>() + g.vals_off[i]);
         o.grad = dev ? v.grad_out : s.grad.as<uint8_t>() + g.grad_off[i];
-        o.rec1 = reinterpret_cast<uint16_t*>(lbase + g.ls[i].rec1_off);
-        o.rec2 = lbase + g.ls[i].rec2_off;
-        o.bits1 = reinterpret_cast<uint32_t*>(lbase + g.ls[i].bits1_off);
-        o.bits2 = reinterpret_cast<uint32_t*>(lbase + g.ls[i].bits2_off);
+        o.rec1 = reinterpret_cast<uint64_t*>(lbase + g.ls[i].rec1_off);
+        o.rec2 = reinterpret_cast<uint64_t*>(lbase + g.ls[i].rec2_off);
+        o.bits1 = reinterpret_cast<uint64_t*>(lbase + g.ls[i].bits1_off);
+        o.bits2 = reinterpret_cast<uint64_t*>(lbase + g.ls[i].bits2_off);
         o.cells = d.cells;
-        o.bit_words = g.ls[i].bit_words;
+        o.ldir = ldir_geom(d);
         o.X = d.X;
         o.Y = d.Y;
         o.Z = d.Z;
         o.Mx = d.Mx;
         o.My = d.My;
         o.Mz = d.Mz;
-        uint32_t nt;
-        ldir_tiles(d, &o.ntx, &o.nty, &nt);
     }
     // pack: GVol[n] | per table: first[n + 1], bucket[]
     std::vector<uint8_t> host;
@@ -268,7 +241,7 @@ int upload_tables(msceer_ctx* ctx, BatchState& s, const msceer_volume* vols, con
     };
     T tb[kLstarBricks];
     for (int sh = 0; sh < kLstarBricks; sh++) tb[sh] = table(g.brick_first[sh]);
-    const T tt = table(g.tile_first), ti = table(g.item_first);
+    const T tt = table(g.tile_first), tf = table(g.flood_first), ti = table(g.item_first);
     CHECK_HIP(p.tables.ensure(host.size()));
     CHECK_HIP(hipMemcpyAsync(p.tables.ptr, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream));
     CHECK_HIP(hipStreamSynchronize(ctx->stream));  // `host` goes out of scope
@@ -282,6 +255,7 @@ int upload_tables(msceer_ctx* ctx, BatchState& s, const msceer_volume* vols, con
     p.batch.nvols = (uint32_t)n;
     for (int sh = 0; sh < kLstarBricks; sh++) p.bricks[sh] = units(tb[sh]);
     p.batch.tiles = units(tt);
+    p.batch.floods = units(tf);
     p.batch.items = units(ti);
     p.batch.queue = s.ctl.as<uint32_t>() + kGQueue;
     return MSCEER_OK;
@@ -388,8 +362,25 @@ int tune_group(msceer_ctx* ctx, BatchState& s, GroupPlan& p, const ListCaps& cap
     return MSCEER_OK;
 }
 
+// The group's tables with its tuned lower-star bricks.
+GBatch group_batch(BatchState& s, const GroupPlan& p, bool timing) {
+    GBatch b = p.batch;
+    b.bricks = p.bricks[p.tune.shape];
+    b.times = timing ? s.times.as<unsigned long long>() : nullptr;
+    return b;
+}
+
+// Sweeps [k, end) of the group's floods.
+int enqueue_sweeps(msceer_ctx* ctx, BatchState& s, const GroupPlan& p, const GroupLayout& g, int k, int end) {
+    uint32_t* dirty = reinterpret_cast<uint32_t*>(s.ldir.as<uint8_t>() + g.dirty_off);
+    for (; k < end; k++)
+        CHECK_HIP(launch_ldir_flood_group(group_batch(s, p, false), dirty, (uint32_t)k,
+                                          s.ctl.as<uint32_t>() + kGActive, ctx->stream));
+    return MSCEER_OK;
+}
+
 // Enqueue the group's pipeline (captured or not): clear, lower star,
-// records, R rounds of each pass on two streams, finish.
+// planes, R sweeps, finish.
 int enqueue_group(msceer_ctx* ctx, BatchState& s, GroupPlan& p, const GroupLayout& g, const ListCaps& caps, int R,
                   bool timing) {
     hipStream_t st = ctx->stream;
@@ -401,26 +392,11 @@ int enqueue_group(msceer_ctx* ctx, BatchState& s, GroupPlan& p, const GroupLayou
         CHECK_HIP(hipGetLastError());
     }
     CHECK_HIP(lstar_stage(s, p, caps, p.tune, timing ? s.times.as<unsigned long long>() : nullptr, st));
-    GBatch b = p.batch;
-    b.bricks = p.bricks[p.tune.shape];
-    b.times = timing ? s.times.as<unsigned long long>() : nullptr;
-    CHECK_HIP(launch_ldir_records_group(b, reinterpret_cast<uint32_t*>(s.ldir.as<uint8_t>() + g.bits_offset),
-                                        g.bit_words, st));
-    CHECK_HIP(hipEventRecord(s.fork, st));
-    CHECK_HIP(hipStreamWaitEvent(s.side, s.fork, 0));
-    for (int pass = 1; pass <= 2; pass++) {
-        hipStream_t ps = pass == 1 ? st : s.side;
-        MList in = glist(s, caps, pass - 1);
-        for (int k = 0; k < R; k++) {
-            const MList out = gfront(s, caps, pass, k);
-            CHECK_HIP(launch_ldir_round_group(b, pass, k == 0, in, out, gfront(s, caps, pass, k + 1).counts,
-                                              ctl + kGOverflow + pass, ps));
-            in = out;
-        }
-    }
-    CHECK_HIP(hipEventRecord(s.join, s.side));
-    CHECK_HIP(hipStreamWaitEvent(st, s.join, 0));
-    CHECK_HIP(launch_ldir_finish_group(b, st));
+    const GBatch b = group_batch(s, p, timing);
+    CHECK_HIP(launch_ldir_planes_group(b, ctl + kGActive, st));
+    const int rc = enqueue_sweeps(ctx, s, p, g, 0, R);
+    if (rc) return rc;
+    CHECK_HIP(launch_ldir_finish_group(b, (uint32_t)R, ctl + kGActive, st));
     return MSCEER_OK;
 }
 
@@ -430,67 +406,11 @@ int read_gctl(msceer_ctx* ctx, BatchState& s) {
     return MSCEER_OK;
 }
 
-// Finish a pass eagerly after the captured rounds: from frontier R - 1 (or a
-// sweep of every volume after an overflow) until the frontier is empty.
-int continue_pass(msceer_ctx* ctx, BatchState& s, GroupPlan& p, const GroupLayout& g, const msceer_volume* vols,
-                  bool dev, const ListCaps& caps, int pass, int R, bool need_sweep, int* extra) {
-    uint32_t* ctl = s.ctl.as<uint32_t>();
-    uint32_t* overflow = ctl + kGOverflow + pass;
-    GBatch b = p.batch;
-    b.bricks = p.bricks[p.tune.shape];
-    int k = R;
-    MList in = R > 0 ? gfront(s, caps, pass, R - 1) : glist(s, caps, pass - 1);
-    auto total = [&](int kk) {
-        return list_total(s.h_ctl + kGRound + (3 * (pass - 1) + kk % 3) * kCountWords, gfront(s, caps, pass, kk));
-    };
-    for (int guard = 0; guard < 100000; guard++) {
-        if (need_sweep) {
-            const MList out = gfront(s, caps, pass, k);
-            CHECK_HIP(launch_zero(out.counts, kCountWords, ctx->stream));
-            CHECK_HIP(launch_zero(overflow, 1, ctx->stream));
-            uint8_t* lbase = s.ldir.as<uint8_t>();
-            for (int i = 0; i < g.count; i++) {
-                const msceer_volume& v = vols[g.first + i];
-                const Dims d = make_dims(v.nx, v.ny, v.nz);
-                const uint8_t* grad = dev ? v.grad_out : s.grad.as<uint8_t>() + g.grad_off[i];
-                CHECK_HIP(launch_ldir_sweep(d, grad, lbase, g.ls[i], pass, out, overflow, ctx->stream,
-                                            g.item_first[i]));
-            }
-            int rc = read_gctl(ctx, s);
-            if (rc) return rc;
-            need_sweep = s.h_ctl[kGOverflow + pass] != 0;
-            (*extra)++;
-            if (total(k) == 0 && !need_sweep) return MSCEER_OK;
-            CHECK_HIP(launch_zero(overflow, 1, ctx->stream));
-            in = out;
-            k++;
-            CHECK_HIP(launch_zero(gfront(s, caps, pass, k).counts, kCountWords, ctx->stream));
-        } else if (total(k - 1) == 0) {
-            return MSCEER_OK;
-        }
-        for (int j = 0; j < 4; j++) {
-            const MList out = gfront(s, caps, pass, k);
-            CHECK_HIP(launch_ldir_round_group(b, pass, false, in, out, gfront(s, caps, pass, k + 1).counts, overflow,
-                                              ctx->stream));
-            (*extra)++;
-            in = out;
-            k++;
-        }
-        int rc = read_gctl(ctx, s);
-        if (rc) return rc;
-        if (s.h_ctl[kGOverflow + pass]) need_sweep = true;
-    }
-    return MSCEER_EHIP;
-}
-
 int ensure_state(msceer_ctx* ctx) {
     if (ctx->gbatch) return MSCEER_OK;
     BatchState* s = new (std::nothrow) BatchState();
     if (!s) return MSCEER_ENOMEM;
     ctx->gbatch = s;
-    CHECK_HIP(hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking));
-    CHECK_HIP(hipEventCreateWithFlags(&s->fork, hipEventDisableTiming));
-    CHECK_HIP(hipEventCreateWithFlags(&s->join, hipEventDisableTiming));
     CHECK_HIP(hipEventCreate(&s->t0));
     CHECK_HIP(hipEventCreate(&s->t1));
     CHECK_HIP(hipHostMalloc((void**)&s->h_ctl, sizeof(uint32_t) * kGWords, hipHostMallocDefault));
@@ -505,9 +425,7 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
               msceer_batch_stats& st) {
     const ListCaps caps = group_caps(g.verts);
     const size_t lbytes = sizeof(uint32_t) * 2 * ((size_t)caps.list_sub * kSubs + caps.list_spill);
-    const size_t fbytes = sizeof(uint32_t) * 4 * ((size_t)caps.front_sub * kSubs + caps.front_spill);
     CHECK_HIP(grow(s, s.lists, lbytes));
-    CHECK_HIP(grow(s, s.fronts, fbytes));
     CHECK_HIP(grow(s, s.ctl, sizeof(uint32_t) * kGWords));
     CHECK_HIP(grow(s, s.ldir, g.ldir_bytes));
     CHECK_HIP(grow(s, s.times, sizeof(unsigned long long) * 2 * (size_t)g.count));
@@ -538,9 +456,8 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
         s.plans.emplace_front();
         it = s.plans.begin();
         it->key = key;
-        // frontier rounds per pass in a first capture (later captures take
-        // what the calls needed)
-        // (0: none, each pass then starts from a sweep after the replay)
+        // sweeps in a first capture (later captures take what the calls
+        // needed; 0: none, all run after the replay)
         if (const char* e = getenv("MSCEER_BATCH_ROUNDS")) it->rounds = std::max(0, std::min(64, atoi(e)));
         int rc = upload_tables(ctx, s, vols, g, dev, *it);
         if (rc) return rc;
@@ -594,36 +511,24 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
     st.replays++;
     int rc = read_gctl(ctx, s);
     if (rc) return rc;
-    const bool lists_lost = s.h_ctl[kGOverflow] != 0;
-    int extra = 0, grow_by = 0;
-    bool redo = false;
-    for (int pass = 1; pass <= 2; pass++) {
-        const int R = p.rounds;
-        const bool left =
-            R > 0 && list_total(s.h_ctl + kGRound + (3 * (pass - 1) + (R - 1) % 3) * kCountWords,
-                                gfront(s, caps, pass, R - 1)) != 0;
-        const bool sweep = R == 0 || lists_lost || s.h_ctl[kGOverflow + pass] != 0;
-        if (!left && !sweep) continue;
-        int used = 0;
-        rc = continue_pass(ctx, s, p, g, vols, dev, caps, pass, R, sweep, &used);
+    int k = p.rounds;
+    const uint64_t most = 6 * g.verts + 64;  // every sweep but the last sets a bit
+    while (k == 0 || s.h_ctl[kGActive + k % 3] != 0) {
+        if ((uint64_t)k > most) return MSCEER_EHIP;
+        rc = enqueue_sweeps(ctx, s, p, g, k, k + 4);
         if (rc) return rc;
-        extra += used;
-        // more captured rounds help a walk that was still going, not an overflow
-        if (!sweep || R == 0) grow_by = std::max(grow_by, used);
-        redo = true;
+        k += 4;
+        rc = read_gctl(ctx, s);
+        if (rc) return rc;
     }
-    if (redo) {
-        GBatch b = p.batch;
-        b.bricks = p.bricks[p.tune.shape];
-        b.times = timing ? s.times.as<unsigned long long>() : nullptr;
-        CHECK_HIP(launch_ldir_finish_group(b, ctx->stream));
-        // the next capture of this plan takes the rounds this call needed
-        if (grow_by > 0) {
-            if (p.exec) (void)hipGraphExecDestroy(p.exec);
-            p.exec = nullptr;
-            p.rounds = std::min(p.rounds + grow_by, 64);
-        }
-        st.eager_rounds += extra;
+    if (k > p.rounds) {
+        st.eager_rounds += k - p.rounds;
+        CHECK_HIP(launch_ldir_finish_group(group_batch(s, p, timing), (uint32_t)k, s.ctl.as<uint32_t>() + kGActive,
+                                           ctx->stream));
+        // the next capture of this plan takes the sweeps this call needed
+        if (p.exec) (void)hipGraphExecDestroy(p.exec);
+        p.exec = nullptr;
+        p.rounds = std::min(k, 64);
     }
     CHECK_HIP(hipEventRecord(s.t1, ctx->stream));
     if (!dev) {
@@ -673,13 +578,12 @@ void batch_state_free(msceer_ctx* ctx) {
         if (p.exec) (void)hipGraphExecDestroy(p.exec);
         p.tables.release();
     }
-    DevBuf* bufs[] = {&s->vals, &s->grad, &s->ldir, &s->lists, &s->fronts, &s->ctl, &s->times};
+    DevBuf* bufs[] = {&s->vals, &s->grad, &s->ldir, &s->lists, &s->ctl, &s->times};
     for (DevBuf* b : bufs) b->release();
     if (s->h_ctl) (void)hipHostFree(s->h_ctl);
-    hipEvent_t evs[] = {s->fork, s->join, s->t0, s->t1};
+    hipEvent_t evs[] = {s->t0, s->t1};
     for (hipEvent_t e : evs)
         if (e) (void)hipEventDestroy(e);
-    if (s->side) (void)hipStreamDestroy(s->side);
     delete s;
     ctx->gbatch = nullptr;
 }

@@ -1,19 +1,19 @@
 // Batched lower-star .grad: many volumes in one launch per stage.
 //
 // A group of volumes is laid out as one index space per kind of work unit:
-// lower-star bricks, ldir tiles and frontier items (cells) of volume v are
+// lower-star bricks, ldir tiles, flood tiles and cells of volume v are
 // numbered from first[v] on, first[] an ascending table with first[n] the
 // total.  Work-groups are mapped to units so that every XCD takes a
 // contiguous eighth of them (bricks that share halos and partly written
 // cache lines of the .grad then meet in that XCD's L2): either one
 // work-group per unit, dealt out by the hardware, or persistent work-groups
 // that claim units from eight queues, one per XCD, and take units from the
-// other queues once their own is empty.  Frontier items are the volume's
-// cell id plus its first[], found again through a coarse bucket table.
+// other queues once their own is empty.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "internal.hpp"
 #include "mlist.hpp"
 
 namespace msceer {
@@ -22,15 +22,14 @@ namespace msceer {
 struct GVol {
     const float* values;  // X*Y*Z
     uint8_t* grad;        // cells
-    uint16_t* rec1;       // ldir records and visited bitmaps of the volume
-    uint8_t* rec2;
-    uint32_t* bits1;
-    uint32_t* bits2;
+    uint64_t* rec1;       // ldir planes and reached bits of the volume
+    uint64_t* rec2;
+    uint64_t* bits1;
+    uint64_t* bits2;
     uint64_t cells;
-    uint32_t bit_words;  // words of one bitmap
     int X, Y, Z;
     uint32_t Mx, My, Mz;
-    uint32_t ntx, nty;  // ldir tiles along x and y
+    LdirGeom ldir;
 };
 
 constexpr int kQueues = 8;  // claim queues, one per XCD
@@ -50,8 +49,9 @@ struct GBatch {
     const GVol* vols;
     uint32_t nvols;
     GUnits bricks;  // lower-star bricks of the launch's brick shape
-    GUnits tiles;   // ldir tiles
-    GUnits items;   // frontier items: the volume's cells
+    GUnits tiles;   // work-groups of the ldir streaming passes
+    GUnits floods;  // ldir flood tiles
+    GUnits items;   // the volume's cells
     uint32_t* queue;            // kQueues claim counters (persistent launches; zeroed before each)
     unsigned long long* times;  // 2 per volume: first brick started, last tile finished (wall clock); or null
     uint32_t chunk;             // units per claim

@@ -54,42 +54,44 @@ hipError_t launch_lstar_batch(const GBatch& g, const LstarBuffers& b, uint32_t b
 // Persistent work-groups of the batched lower-star kernel one CU holds at once.
 int lstar_batch_occupancy(int shape);
 
-// ldir (ascending-manifold dimension) passes, see ldir.hip.  Scratch: edge
-// and quad walk records and the two visited bitmaps, at these byte offsets of
-// one device buffer of ldir_scratch_bytes().
+// ldir (ascending-manifold dimension) passes, see ldir.hip.  Geometry of the
+// bit planes: the words' axis, then the other two (axis[], with the vertices
+// n[] and the .grad strides cs[] along them); 64-bit words per row; flood
+// tiles (16 rows each) along the rows' two axes.
+struct LdirGeom {
+    int axis[3];
+    int n[3];
+    uint32_t cs[3];
+    int words, ty, tz;
+};
+LdirGeom ldir_geom(const Dims& d);
+// Scratch: edge and quad planes, the bits reached, the tile marks, at these
+// byte offsets of one device buffer of ldir_scratch_bytes().
 struct LdirScratch {
-    size_t rec1_off, rec2_off, bits1_off, bits2_off;
-    uint32_t bit_words;  // words of one bitmap
+    size_t rec1_off, rec2_off, bits1_off, bits2_off, dirty_off;
 };
 size_t ldir_scratch_bytes(const Dims& d, LdirScratch* s);
 // Clears the ascending-manifold dimension bits (5-7) of n .grad bytes.
 hipError_t launch_clear_ldir_bits(uint8_t* grad, int64_t n, hipStream_t st);
-// Records of the walks (from the lower-star bytes) and cleared bitmaps.
-hipError_t launch_ldir_records(const Dims& d, const uint8_t* grad, void* scratch, const LdirScratch& s,
-                               hipStream_t st);
-// One frontier round of pass 1 (edges) or 2 (quads): expands the items of
-// `in` (critical cells, claimed first, when `start`), appends what is left to
-// `out` (start items it did not reach claimed first) and zeroes
-// `clear_counts` for the next round.  overflow |= 1 when an item did not fit
-// `out`.
-hipError_t launch_ldir_round(const Dims& d, void* scratch, const LdirScratch& s, int pass, bool start, const MList& in,
-                             const MList& out, uint32_t* clear_counts, uint32_t* overflow, hipStream_t st);
-// Rebuild a frontier from the bitmaps and records alone (after an overflow).
-// (The frontier entries are the cell ids plus item0.)
-hipError_t launch_ldir_sweep(const Dims& d, const uint8_t* grad, void* scratch, const LdirScratch& s, int pass,
-                             const MList& out, uint32_t* overflow, hipStream_t st, uint32_t item0 = 0);
-// Every cell's ldir from what the two passes reached.
-hipError_t launch_ldir_finish(const Dims& d, uint8_t* grad, void* scratch, const LdirScratch& s, hipStream_t st);
-// Tiles of the ldir streaming passes of a volume (along x, y, in all).
-void ldir_tiles(const Dims& d, uint32_t* ntx, uint32_t* nty, uint32_t* tiles);
-// The same passes over a group of volumes (one launch each; records and
-// bitmaps of every volume in its table entry): records, clearing bit_words
-// words of the group's bitmaps from `bits`; one round of pass 1 or 2 over
-// frontier items of the group; the ldir bits of every volume.
-hipError_t launch_ldir_records_group(const GBatch& b, uint32_t* bits, uint64_t bit_words, hipStream_t st);
-hipError_t launch_ldir_round_group(const GBatch& b, int pass, bool start, const MList& in, const MList& out,
-                                   uint32_t* clear_counts, uint32_t* overflow, hipStream_t st);
-hipError_t launch_ldir_finish_group(const GBatch& b, hipStream_t st);
+// Planes and start bits from the lower-star bytes; zeroes active[0..2].
+hipError_t launch_ldir_planes(const Dims& d, const uint8_t* grad, void* scratch, const LdirScratch& s,
+                              uint32_t* active, hipStream_t st);
+// Sweep 0, 1, ... of both floods; they have ended once sweep k left
+// active[(k + 1) % 3] zero (further sweeps do nothing).
+hipError_t launch_ldir_flood(const Dims& d, void* scratch, const LdirScratch& s, uint32_t sweep, uint32_t* active,
+                             hipStream_t st);
+// Every cell's ldir from what the floods reached, if they ended within `sweeps`
+// sweeps (else nothing is written).
+hipError_t launch_ldir_finish(const Dims& d, uint8_t* grad, void* scratch, const LdirScratch& s, uint32_t sweeps,
+                              uint32_t* active, hipStream_t st);
+// Work-groups of the streaming passes of a volume, and flood tiles.
+uint32_t ldir_tiles(const Dims& d);
+uint32_t ldir_flood_tiles(const Dims& d);
+// The same over a group of volumes, one launch each (buffers of every volume
+// in its table entry; dirty: two words per flood tile of the group).
+hipError_t launch_ldir_planes_group(const GBatch& b, uint32_t* active, hipStream_t st);
+hipError_t launch_ldir_flood_group(const GBatch& b, uint32_t* dirty, uint32_t sweep, uint32_t* active, hipStream_t st);
+hipError_t launch_ldir_finish_group(const GBatch& b, uint32_t sweeps, uint32_t* active, hipStream_t st);
 // Zero n words.
 hipError_t launch_zero(uint32_t* p, uint32_t n, hipStream_t s);
 

@@ -785,10 +785,8 @@ int ondemand_impl(msceer_ctx* ctx, const float* values, int64_t nx, int64_t ny, 
         LstarBuffers cb{d_values, d_grad, restr, &list1, &list2, ctl + kCtlStats, ctl + kCtlOverflow};
         CHECK_HIP(launch_lstar(d, cb, s, shape));
         CHECK_HIP(hipEventRecord(ev[6], s));
-        rc = read_ctl(ctx, kCtlOverflow, 1);
-        if (rc) return rc;
         int ldir_rounds = 0;
-        rc = run_ldir(ctx, d, d_grad, caps, ctx->h_ctl[kCtlOverflow] == 0, &ldir_rounds);
+        rc = run_ldir(ctx, d, d_grad, &ldir_rounds);
         if (rc) return rc;
         if (!dev) CHECK_HIP(hipMemcpyAsync(grad_out, d_grad, C, hipMemcpyDeviceToHost, s));
     } else {
@@ -1029,10 +1027,8 @@ extern "C" int msceer_constrained_lstar(msceer_ctx* ctx, const float* values, in
     CHECK_HIP(launch_zero(ctl, kCtlWords, s));
     CHECK_HIP(launch_lstar(d, cb, s, shape));
     if (!(flags & MSCEER_SKIP_LDIR)) {
-        rc = read_ctl(ctx, kCtlOverflow, 1);
-        if (rc) return rc;
         int rounds = 0;
-        rc = run_ldir(ctx, d, d_grad, caps, ctx->h_ctl[kCtlOverflow] == 0, &rounds);
+        rc = run_ldir(ctx, d, d_grad, &rounds);
         if (rc) return rc;
     }
     if (!dev) CHECK_HIP(hipMemcpyAsync(grad_inout, d_grad, d.cells, hipMemcpyDeviceToHost, s));

@@ -277,7 +277,7 @@ __global__ void __launch_bounds__(kThreads) lstar_kernel(LstarArgs a) {
 
         // Copy the stage out, four cells a lane at a time along the rows; a zero
         // byte is a cell no brick vertex owns.  Critical cells (pair code 7) are
-        // counted by dimension and the 1- and 2-cells listed for the ldir passes.
+        // counted by dimension and the 1- and 2-cells listed (for the line tracers).
         // Cell parity: stage x offset 4 j + b is .grad x 2 x0 - 1 + 4 j + b (odd
         // for even b), stage row (j, k) is y 2 y0 - 1 + j, z 2 z0 - 1 + k.
         uint32_t* const lst = reinterpret_cast<uint32_t*>(smem);
