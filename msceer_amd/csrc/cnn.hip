@@ -50,37 +50,75 @@ __device__ __forceinline__ int tap_dx(int t) { return t % 3 - 1; }
 __device__ __forceinline__ int tap_dy(int t) { return (t / 3) % 3 - 1; }
 __device__ __forceinline__ int tap_dz(int t) { return t / 9 - 1; }
 
+// Tile of a work-group: tiles along x, then y, then z; work-groups are dealt to
+// the eight XCDs round robin, so each takes a contiguous run of the tiles and
+// neighbours share their halos in one L2.  A launch takes at most kMaxTiles of
+// them (a grid holds fewer than 2^32 threads), from `first` on.
+struct Tiles {
+    uint32_t first, n, x, y;  // of this launch; along x and y
+};
+struct Tile {
+    int x, y, z;
+};
+constexpr uint32_t kMaxTiles = 1u << 22;
+__device__ __forceinline__ Tile tile_of(const Tiles& a) {
+    const uint32_t per = a.n / 8u, rem = a.n % 8u, xcd = blockIdx.x % 8u, k = blockIdx.x / 8u;
+    const uint32_t t = a.first + (xcd < rem ? xcd * (per + 1u) + k : rem * (per + 1u) + (xcd - rem) * per + k);
+    const uint32_t q = t / a.x;
+    return Tile{(int)(t % a.x), (int)(q % a.y), (int)(q / a.y)};
+}
+
 // ---- local normalisation (separable 9-wide box sums in FP64) ----------------
 
-__global__ void __launch_bounds__(kT) norm_x_kernel(const float* __restrict__ f, Geo g, double2* __restrict__ out) {
-    const int64_t n = g.verts();
-    for (int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x; v < n; v += (int64_t)gridDim.x * kT) {
-        const int x = (int)(v % g.X);
+// Sums along x, then along y, for a tile of 64x16 vertices of one layer: values
+// and x sums in LDS.  Absent vertices add zeros, in the order of the window, so
+// the sums are those of the present ones alone.  Bound by LDS reads (9 values
+// and 3 pairs of doubles per vertex) and the 16 B/vertex written: 41 us at
+// 256x192x128; as two passes over memory, with each pair of sums read 9 times
+// and coordinates by 64-bit division, 182.
+constexpr int kNormX = 64, kNormY = 16;
+__global__ void __launch_bounds__(kT) norm_xy_kernel(const float* __restrict__ f, Geo g, Tiles tiles,
+                                                     double2* __restrict__ out) {
+    __shared__ float sv[kNormY + 8][kNormX + 8];
+    __shared__ double2 sx[kNormY + 8][kNormX];
+    const Tile t = tile_of(tiles);
+    const int x0 = t.x * kNormX, y0 = t.y * kNormY;
+    const float* const layer = f + (int64_t)t.z * g.sxy;
+    for (int i = threadIdx.x; i < (kNormY + 8) * (kNormX + 8); i += kT) {
+        const int ly = i / (kNormX + 8), lx = i % (kNormX + 8), x = x0 + lx - 4, y = y0 + ly - 4;
+        const bool in = x >= 0 && x < g.X && y >= 0 && y < g.Y;
+        sv[ly][lx] = in ? layer[(int64_t)y * g.X + x] : 0.f;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < (kNormY + 8) * kNormX; i += kT) {
+        const int ly = i / kNormX, lx = i % kNormX;
         double s1 = 0.0, s2 = 0.0;
-        for (int d = -4; d <= 4; d++) {
-            const int xx = x + d;
-            if (xx < 0 || xx >= g.X) continue;
-            const double a = (double)f[v + d];
+#pragma unroll
+        for (int d = 0; d < 9; d++) {
+            const double a = (double)sv[ly][lx + d];
             s1 += a;
             s2 += a * a;
         }
-        out[v] = make_double2(s1, s2);
+        sx[ly][lx] = make_double2(s1, s2);
     }
-}
-
-__global__ void __launch_bounds__(kT) norm_y_kernel(const double2* __restrict__ in, Geo g, double2* __restrict__ out) {
-    const int64_t n = g.verts();
-    for (int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x; v < n; v += (int64_t)gridDim.x * kT) {
-        const int y = (int)((v / g.X) % g.Y);
+    __syncthreads();
+    constexpr int kRows = kNormY * kNormX / kT;  // rows per thread
+    const int lx = threadIdx.x % kNormX, ly = threadIdx.x / kNormX * kRows, x = x0 + lx;
+    double2 col[kRows + 8];
+#pragma unroll
+    for (int d = 0; d < kRows + 8; d++) col[d] = sx[ly + d][lx];
+    if (x >= g.X) return;
+#pragma unroll
+    for (int j = 0; j < kRows; j++) {
+        const int y = y0 + ly + j;
+        if (y >= g.Y) break;
         double s1 = 0.0, s2 = 0.0;
-        for (int d = -4; d <= 4; d++) {
-            const int yy = y + d;
-            if (yy < 0 || yy >= g.Y) continue;
-            const double2 a = in[v + (int64_t)d * g.X];
-            s1 += a.x;
-            s2 += a.y;
+#pragma unroll
+        for (int d = 0; d < 9; d++) {
+            s1 += col[j + d].x;
+            s2 += col[j + d].y;
         }
-        out[v] = make_double2(s1, s2);
+        out[(int64_t)t.z * g.sxy + (int64_t)y * g.X + x] = make_double2(s1, s2);
     }
 }
 
@@ -89,20 +127,35 @@ __device__ __forceinline__ int win_count(int c, int n) {
     return hi - lo + 1;
 }
 
+// Sums along z and the normalised value, kNormZ vertices up per thread: 16 sums
+// read for 8 vertices.  Bound by the FP64 division and square root: 43 us at
+// 256x192x128 (63 with 9 reads a vertex).
+constexpr int kNormZ = 8;
 __global__ void __launch_bounds__(kT)
-norm_z_kernel(const double2* __restrict__ in, const float* __restrict__ f, Geo g, float* __restrict__ out) {
-    const int64_t n = g.verts();
-    for (int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x; v < n; v += (int64_t)gridDim.x * kT) {
-        const int x = (int)(v % g.X), y = (int)((v / g.X) % g.Y), z = (int)(v / g.sxy);
+norm_z_kernel(const double2* __restrict__ in, const float* __restrict__ f, Geo g, Tiles tiles, float* __restrict__ out) {
+    const Tile t = tile_of(tiles);
+    const int x = t.x * 64 + (int)(threadIdx.x & 63u), y = t.y * (kT / 64) + (int)(threadIdx.x >> 6), z0 = t.z * kNormZ;
+    if (x >= g.X || y >= g.Y) return;
+    const int64_t v0 = (int64_t)z0 * g.sxy + (int64_t)y * g.X + x;
+    double2 col[kNormZ + 8];
+#pragma unroll
+    for (int d = 0; d < kNormZ + 8; d++) {
+        const int z = z0 + d - 4;
+        col[d] = z >= 0 && z < g.Z ? in[v0 + (int64_t)(d - 4) * g.sxy] : make_double2(0.0, 0.0);
+    }
+    const double cxy = (double)win_count(x, g.X) * win_count(y, g.Y);
+#pragma unroll
+    for (int j = 0; j < kNormZ; j++) {
+        const int z = z0 + j;
+        if (z >= g.Z) break;
         double s1 = 0.0, s2 = 0.0;
-        for (int d = -4; d <= 4; d++) {
-            const int zz = z + d;
-            if (zz < 0 || zz >= g.Z) continue;
-            const double2 a = in[v + (int64_t)d * g.sxy];
-            s1 += a.x;
-            s2 += a.y;
+#pragma unroll
+        for (int d = 0; d < 9; d++) {
+            s1 += col[j + d].x;
+            s2 += col[j + d].y;
         }
-        const double cnt = (double)win_count(x, g.X) * win_count(y, g.Y) * win_count(z, g.Z);
+        const int64_t v = v0 + (int64_t)j * g.sxy;
+        const double cnt = cxy * win_count(z, g.Z);
         const double mean = s1 / cnt;
         double var = s2 / cnt - mean * mean;
         if (var < 0.0) var = 0.0;
@@ -110,41 +163,76 @@ norm_z_kernel(const double2* __restrict__ in, const float* __restrict__ f, Geo g
     }
 }
 
+// Two values to BF16, nearest even (no NaN reaches it).
+__device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
+    return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)lo) |
+           (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)hi) << 16;
+}
+__device__ __forceinline__ float relu(float v) { return v > 0.f ? v : 0.f; }  // (of NaN: 0)
+
 // ---- conv1: 1 -> 16, ReLU (VALU) --------------------------------------------
 
+// A wave takes 64 vertices along x by 4 rows: each tap's 16 weights, read from
+// LDS by all lanes at once, serve the four.  Bound by VALU issue, 432 FMAs a
+// vertex: 95 us at 256x192x128.  With one vertex per lane and each weight read
+// for it alone it was bound by the LDS reads, 466; with the weights of two rows
+// by scalar loads, which the compiler moves to the front and spills, 169.
+constexpr int kC1Rows = 4;
 __global__ void __launch_bounds__(kT)
-conv1_kernel(const float* __restrict__ xin, Geo g, const float* __restrict__ w1 /*[27][16] bf16-rounded*/,
+conv1_kernel(const float* __restrict__ xin, Geo g, Tiles tiles, const float* __restrict__ w1 /*[27][16] bf16-rounded*/,
              const float* __restrict__ b1, uint16_t* __restrict__ a1) {
-    __shared__ float sw[27 * 16 + 16];
+    __shared__ __attribute__((aligned(16))) float sw[27 * 16];
     for (int i = threadIdx.x; i < 27 * 16; i += kT) sw[i] = w1[i];
-    if (threadIdx.x < 16) sw[27 * 16 + threadIdx.x] = b1[threadIdx.x];
     __syncthreads();
-    const int64_t n = g.verts();
-    for (int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x; v < n; v += (int64_t)gridDim.x * kT) {
-        const int x = (int)(v % g.X), y = (int)((v / g.X) % g.Y), z = (int)(v / g.sxy);
-        float nv[27];
+    const Tile t = tile_of(tiles);
+    const int x = t.x * 64 + (int)(threadIdx.x & 63u), y0 = t.y * kC1Rows;
+    const int z = t.z * (kT / 64) + (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (z >= g.Z) return;
+    const int xc = min(x, g.X - 1), xl = max(xc - 1, 0), xr = min(xc + 1, g.X - 1);
+    const bool okl = x > 0, okr = x + 1 < g.X;
+    float acc[kC1Rows][16];
 #pragma unroll
-        for (int t = 0; t < 27; t++) {
-            const int xx = x + tap_dx(t), yy = y + tap_dy(t), zz = z + tap_dz(t);
-            const bool ok = xx >= 0 && xx < g.X && yy >= 0 && yy < g.Y && zz >= 0 && zz < g.Z;
-            nv[t] = ok ? xin[v + tap_dx(t) + (int64_t)tap_dy(t) * g.X + (int64_t)tap_dz(t) * g.sxy] : 0.f;
+    for (int c = 0; c < 16; c++)
+#pragma unroll
+        for (int j = 0; j < kC1Rows; j++) acc[j][c] = b1[c];
+#pragma unroll 1
+    for (int dz = 0; dz < 3; dz++) {
+        const int zz = z + dz - 1;
+        const bool zok = zz >= 0 && zz < g.Z;
+        const float* const layer = xin + (int64_t)(zok ? zz : z) * g.sxy;
+        float nv[kC1Rows + 2][3];
+#pragma unroll
+        for (int i = 0; i < kC1Rows + 2; i++) {
+            const int yy = y0 + i - 1;
+            const bool yok = yy >= 0 && yy < g.Y, ok = zok && yok;  // the same in every lane
+            const float* const row = layer + (int64_t)(yok ? yy : y0) * g.X;
+            const float l = row[xl], c = row[xc], r = row[xr];
+            nv[i][0] = ok && okl ? l : 0.f;
+            nv[i][1] = ok ? c : 0.f;
+            nv[i][2] = ok && okr ? r : 0.f;
         }
-        uint32_t packed[8];
 #pragma unroll
-        for (int c = 0; c < 16; c += 2) {
-            float z0 = sw[27 * 16 + c], z1 = sw[27 * 16 + c + 1];
+        for (int k = 0; k < 9; k++) {
+            const float4* const wk = reinterpret_cast<const float4*>(sw + (dz * 9 + k) * 16);
+            const float4 w0 = wk[0], w4 = wk[1], w8 = wk[2], wc = wk[3];
+            const float w[16] = {w0.x, w0.y, w0.z, w0.w, w4.x, w4.y, w4.z, w4.w,
+                                 w8.x, w8.y, w8.z, w8.w, wc.x, wc.y, wc.z, wc.w};
 #pragma unroll
-            for (int t = 0; t < 27; t++) {
-                z0 = fmaf(sw[t * 16 + c], nv[t], z0);
-                z1 = fmaf(sw[t * 16 + c + 1], nv[t], z1);
-            }
-            z0 = z0 > 0.f ? z0 : 0.f;
-            z1 = z1 > 0.f ? z1 : 0.f;
-            packed[c / 2] = (uint32_t)f2bf(z0) | ((uint32_t)f2bf(z1) << 16);
+            for (int c = 0; c < 16; c++)
+#pragma unroll
+                for (int j = 0; j < kC1Rows; j++) acc[j][c] = fmaf(w[c], nv[j + k / 3][k % 3], acc[j][c]);
         }
-        uint4* o = reinterpret_cast<uint4*>(a1 + v * 16);
-        o[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-        o[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
+    }
+    if (x >= g.X) return;
+#pragma unroll
+    for (int j = 0; j < kC1Rows; j++) {
+        if (y0 + j >= g.Y) break;
+        uint32_t p[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) p[c] = pack_bf(relu(acc[j][2 * c]), relu(acc[j][2 * c + 1]));
+        uint4* o = reinterpret_cast<uint4*>(a1 + ((int64_t)z * g.sxy + (int64_t)(y0 + j) * g.X + x) * 16);
+        o[0] = make_uint4(p[0], p[1], p[2], p[3]);
+        o[1] = make_uint4(p[4], p[5], p[6], p[7]);
     }
 }
 
@@ -161,123 +249,256 @@ __device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
     return __builtin_bit_cast(bf16x8, u);
 }
 
-// conv 16 -> 32: one wave computes 32 consecutive x-voxels x 32 output
-// channels with one 32x32x16 MFMA per tap.  Operand layouts (wave64):
+// Two values of a gradient to BF16 where the activations are positive.
+__device__ __forceinline__ uint32_t gated(uint32_t gate, float lo, float hi) {
+    return (bf2f((uint16_t)gate) > 0.f ? (uint32_t)f2bf(lo) : 0u) |
+           (bf2f((uint16_t)(gate >> 16)) > 0.f ? (uint32_t)f2bf(hi) : 0u) << 16;
+}
+
+// Both convolutions: a work-group computes 32x16 vertices of `layers` layers,
+// each wave several rows along y of one x tile.  It runs up the input layers:
+// 34x18 vertices of one are staged in LDS (the next one's loads are in flight
+// meanwhile) and serve the three output layers they are taps of, two of which
+// a wave keeps between steps.  Per layer of taps a wave holds its 9 weight
+// operands and runs over the input rows; an input row (three LDS reads, one per
+// dx) serves the up to three output rows it is a tap of.  So every output still
+// sums its taps in order.  The weights are the A operand and the vertices the
+// columns: a lane then holds several channels of one vertex, and stores (or
+// sums, for the head) them together.  Bound by LDS reads and MFMA, about even,
+// with the memory traffic behind them (256x192x128: 0.6 GB for 16 -> 32, 0.4 GB
+// for 32 -> 16): 164 and 178 us, of which the MFMAs alone take 69 each.  Without
+// the run along z, three layers staged per output layer: 248 and 265; without
+// LDS, bound by the cache's accesses: 345 and 345; a wave per row with a load per
+// tap and MFMA, vertices as rows and 2-byte stores: 553 and 835.
+constexpr int kCx = 32, kCy = 16;
+
+// One layer of a tile with its rim for the work-group: kC channels, zero where
+// there is no vertex.
+template <int kC>
+struct Stage {
+    static constexpr int kPer = kC / 8, kAll = (kCx + 2) * (kCy + 2) * kPer, kK = (kAll + kT - 1) / kT;
+    int32_t at[kK];  // 16-byte pieces from the layer's tile origin, -1: none
+    uint4 u[kK];
+    __device__ Stage(const Geo& g, int x0, int y0) {
+#pragma unroll
+        for (int k = 0; k < kK; k++) {
+            const int i = (int)threadIdx.x + k * kT, v = i / kPer, x = x0 + v % (kCx + 2) - 1, y = y0 + v / (kCx + 2) - 1;
+            const bool in = i < kAll && x >= 0 && x < g.X && y >= 0 && y < g.Y;
+            at[k] = in ? ((y - max(y0 - 1, 0)) * g.X + x) * kPer + i % kPer : -1;  // (< 18 * 2^16 * 4)
+        }
+    }
+    // tile: the layer's row max(y0 - 1, 0); ok: the layer is there
+    __device__ __forceinline__ void load(const uint4* __restrict__ tile, bool ok) {
+#pragma unroll
+        for (int k = 0; k < kK; k++) {
+            u[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (ok && at[k] >= 0) u[k] = tile[at[k]];
+        }
+    }
+    __device__ __forceinline__ void store(uint4* lds) const {
+#pragma unroll
+        for (int k = 0; k < kK; k++) {
+            const int i = (int)threadIdx.x + k * kT;
+            if (i < kAll) lds[i] = u[k];
+        }
+    }
+};
+
+// conv 16 -> 32, a wave 32 vertices x kC2Rows rows, MFMA 32x32x16 (wave64):
 // A[row = lane%32][k = 8*(lane/32) .. +8], B[k = 8*(lane/32) .. +8][col = lane%32],
-// D[i]: row 8*(i/4) + 4*(lane/32) + i%4, col lane%32.
+// D[i]: row 8*(i/4) + 4*(lane/32) + i%4, col lane%32.  Row m of A is output
+// channel 16*((m/4)%2) + 4*(m/8) + m%4, so D[i] is channel 16*(lane/32) + i.
+constexpr int kC2Rows = 4;  // of 16 for four waves
 template <int kMode>
 __global__ void __launch_bounds__(kT)
-conv16to32_kernel(const uint16_t* __restrict__ in, Geo g, const uint16_t* __restrict__ w /*[27][32][16]*/,
+conv16to32_kernel(const uint16_t* __restrict__ in, Geo g, Tiles tiles, int layers, const uint16_t* __restrict__ w /*[27][32][16]*/,
                   const float* __restrict__ bias, const uint16_t* __restrict__ gate, uint16_t* __restrict__ out) {
     __shared__ __attribute__((aligned(16))) uint16_t sw[27 * 32 * 16];
+    __shared__ __attribute__((aligned(16))) uint16_t sv[(kCx + 2) * (kCy + 2) * 16];
     __shared__ float sb[32];
+    if (kMode == kFwd && threadIdx.x < 32) sb[threadIdx.x] = bias[threadIdx.x];
     for (int i = threadIdx.x; i < 27 * 32 * 16 / 8; i += kT)
         reinterpret_cast<uint4*>(sw)[i] = reinterpret_cast<const uint4*>(w)[i];
-    if (kMode == kFwd && threadIdx.x < 32) sb[threadIdx.x] = bias[threadIdx.x];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = lane & 31, h = lane >> 5;
-    const int tiles_x = (g.X + 31) / 32;
-    const int64_t ntiles = (int64_t)tiles_x * g.Y * g.Z;
-    for (int64_t tile = (int64_t)blockIdx.x * 4 + wave; tile < ntiles; tile += (int64_t)gridDim.x * 4) {
-        const int x0 = (int)(tile % tiles_x) * 32;
-        const int y = (int)((tile / tiles_x) % g.Y), z = (int)(tile / ((int64_t)tiles_x * g.Y));
-        f32x16 acc = {};
-        const int x = x0 + r;
-#pragma unroll 3
-        for (int t = 0; t < 27; t++) {
-            const int xx = x + tap_dx(t), yy = y + tap_dy(t), zz = z + tap_dz(t);
-            const bool ok = x < g.X && xx >= 0 && xx < g.X && yy >= 0 && yy < g.Y && zz >= 0 && zz < g.Z;
-            bf16x8 a = {};
-            if (ok) a = load8(in + ((int64_t)xx + (int64_t)yy * g.X + (int64_t)zz * g.sxy) * 16 + 8 * h);
-            const bf16x8 b = load8(sw + (t * 32 + r) * 16 + 8 * h);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-        }
-        const int co = r;
+    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+    const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Tile t = tile_of(tiles);
+    const int x = t.x * kCx + r, y0 = t.y * kCy + wave * kC2Rows;
+    const int z0 = t.z * layers, z1 = min(z0 + layers, g.Z);
+    const uint16_t* const wl = sw + (16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3)) * 16 + 8 * h;
+    const uint16_t* const vl = sv + (wave * kC2Rows * (kCx + 2) + r) * 16 + 8 * h;
+    Stage<16> stage(g, t.x * kCx, t.y * kCy);
+    const uint4* const tile = reinterpret_cast<const uint4*>(in + (int64_t)max(t.y * kCy - 1, 0) * g.X * 16);
+    auto load = [&](int z) { stage.load(tile + (int64_t)z * g.sxy * 2, z >= 0 && z < g.Z); };
+    // adds the taps of layer dz that lie in the staged input layer
+    auto taps = [&](f32x16 acc[kC2Rows], int dz) {
+        bf16x8 wt[9];
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int row = 8 * (i / 4) + 4 * h + (i % 4);
-            const int xo = x0 + row;
-            if (xo >= g.X) continue;
-            const int64_t vo = (int64_t)xo + (int64_t)y * g.X + (int64_t)z * g.sxy;
-            float val = acc[i];
-            if (kMode == kFwd) {
-                val += sb[co];
-                val = val > 0.f ? val : 0.f;
-            } else {
-                if (!(bf2f(gate[vo * 32 + co]) > 0.f)) val = 0.f;
+        for (int k = 0; k < 9; k++) wt[k] = load8(wl + (dz * 9 + k) * 512);
+#pragma unroll
+        for (int i = 0; i < kC2Rows + 2; i++)
+#pragma unroll
+            for (int dx = 0; dx < 3; dx++) {
+                const bf16x8 v = load8(vl + (i * (kCx + 2) + dx) * 16);
+#pragma unroll
+                for (int dy = 0; dy < 3; dy++)
+                    if (i - dy >= 0 && i - dy < kC2Rows)
+                        acc[i - dy] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wt[3 * dy + dx], v, acc[i - dy], 0, 0, 0);
             }
-            out[vo * 32 + co] = f2bf(val);
+    };
+    auto emit = [&](const f32x16 acc[kC2Rows], int z) {
+        if (x >= g.X) return;
+#pragma unroll
+        for (int j = 0; j < kC2Rows; j++) {
+            if (y0 + j >= g.Y) break;
+            const int64_t at = ((int64_t)z * g.sxy + (int64_t)(y0 + j) * g.X + x) * 32 + 16 * h;
+            uint32_t p[8];
+            if (kMode == kFwd) {
+                const float* const b = sb + 16 * h;
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    p[i] = pack_bf(relu(acc[j][2 * i] + b[2 * i]), relu(acc[j][2 * i + 1] + b[2 * i + 1]));
+            } else {
+                const uint4 g0 = reinterpret_cast<const uint4*>(gate + at)[0], g1 = reinterpret_cast<const uint4*>(gate + at)[1];
+                const uint32_t gs[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+#pragma unroll
+                for (int i = 0; i < 8; i++) p[i] = gated(gs[i], acc[j][2 * i], acc[j][2 * i + 1]);
+            }
+            uint4* const o = reinterpret_cast<uint4*>(out + at);
+            o[0] = make_uint4(p[0], p[1], p[2], p[3]);
+            o[1] = make_uint4(p[4], p[5], p[6], p[7]);
+        }
+    };
+    f32x16 a[kC2Rows] = {}, b[kC2Rows] = {};  // of the layers below and at the input layer
+    load(z0 - 1);
+#pragma unroll 1
+    for (int z = z0 - 1; z <= z1; z++) {
+        __syncthreads();
+        stage.store(reinterpret_cast<uint4*>(sv));
+        if (z < z1) load(z + 1);
+        __syncthreads();
+        if (z > z0) {
+            taps(a, 2);
+            emit(a, z - 1);
+        }
+        if (z >= z0 && z < z1) {
+#pragma unroll
+            for (int j = 0; j < kC2Rows; j++) a[j] = b[j];
+            taps(a, 1);
+        }
+        if (z + 1 < z1) {
+#pragma unroll
+            for (int j = 0; j < kC2Rows; j++) b[j] = f32x16{};
+            taps(b, 0);
         }
     }
 }
 
-// conv 32 -> 16: one wave computes 64 consecutive x-voxels (four 16-voxel
-// sub-tiles) x 16 output channels, one 16x16x32 MFMA per sub-tile and tap.
+// conv 32 -> 16, a wave 16 vertices x kC3Rows rows, MFMA 16x16x32:
 // A[row = lane%16][k = 8*(lane/16) .. +8], B[k = 8*(lane/16) .. +8][col = lane%16],
-// D[i]: row 4*(lane/16) + i, col lane%16.
+// D[i]: row (channel) 4*(lane/16) + i, col (vertex) lane%16.
+constexpr int kC3Rows = 8;  // four waves: 2 x 2
 template <int kMode>
 __global__ void __launch_bounds__(kT)
-conv32to16_kernel(const uint16_t* __restrict__ in, Geo g, const uint16_t* __restrict__ w /*[27][16][32]*/,
+conv32to16_kernel(const uint16_t* __restrict__ in, Geo g, Tiles tiles, int layers, const uint16_t* __restrict__ w /*[27][16][32]*/,
                   const float* __restrict__ bias, const float* __restrict__ head /*[16] + bias*/,
                   const uint16_t* __restrict__ gate, uint16_t* __restrict__ out, float* __restrict__ prob) {
     __shared__ __attribute__((aligned(16))) uint16_t sw[27 * 16 * 32];
-    __shared__ float sb[16], sh[17];
+    __shared__ __attribute__((aligned(16))) uint16_t sv[(kCx + 2) * (kCy + 2) * 32];
     for (int i = threadIdx.x; i < 27 * 16 * 32 / 8; i += kT)
         reinterpret_cast<uint4*>(sw)[i] = reinterpret_cast<const uint4*>(w)[i];
-    if (kMode != kBwd && threadIdx.x < 16) sb[threadIdx.x] = bias[threadIdx.x];
-    if (kMode == kFwdHead && threadIdx.x < 17) sh[threadIdx.x] = head[threadIdx.x];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = lane & 15, q = lane >> 4;
-    const int tiles_x = (g.X + 63) / 64;
-    const int64_t ntiles = (int64_t)tiles_x * g.Y * g.Z;
-    for (int64_t tile = (int64_t)blockIdx.x * 4 + wave; tile < ntiles; tile += (int64_t)gridDim.x * 4) {
-        const int x0 = (int)(tile % tiles_x) * 64;
-        const int y = (int)((tile / tiles_x) % g.Y), z = (int)(tile / ((int64_t)tiles_x * g.Y));
-        f32x4 acc[4] = {};
-#pragma unroll 3
-        for (int t = 0; t < 27; t++) {
-            const bf16x8 b = load8(sw + (t * 16 + r) * 32 + 8 * q);
-            const int yy = y + tap_dy(t), zz = z + tap_dz(t);
-            const bool rowok = yy >= 0 && yy < g.Y && zz >= 0 && zz < g.Z;
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Tile t = tile_of(tiles);
+    const int lx = (wave & 1) * 16, ly = (wave >> 1) * kC3Rows;
+    const int x = t.x * kCx + lx + r, y0 = t.y * kCy + ly;
+    const int z0 = t.z * layers, z1 = min(z0 + layers, g.Z);
+    const uint16_t* const wl = sw + r * 32 + 8 * q;
+    const uint16_t* const vl = sv + (ly * (kCx + 2) + lx + r) * 32 + 8 * q;
+    Stage<32> stage(g, t.x * kCx, t.y * kCy);
+    const uint4* const tile = reinterpret_cast<const uint4*>(in + (int64_t)max(t.y * kCy - 1, 0) * g.X * 32);
+    auto load = [&](int z) { stage.load(tile + (int64_t)z * g.sxy * 4, z >= 0 && z < g.Z); };
+    float bv[4], hv[4], hb = 0.f;
 #pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const int x = x0 + 16 * s + r, xx = x + tap_dx(t);
-                bf16x8 a = {};
-                if (rowok && x < g.X && xx >= 0 && xx < g.X)
-                    a = load8(in + ((int64_t)xx + (int64_t)yy * g.X + (int64_t)zz * g.sxy) * 32 + 8 * q);
-                acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[s], 0, 0, 0);
+    for (int i = 0; i < 4; i++) {
+        bv[i] = kMode != kBwd ? bias[4 * q + i] : 0.f;
+        hv[i] = kMode == kFwdHead ? head[4 * q + i] : 0.f;
+    }
+    if (kMode == kFwdHead) hb = head[16];
+    auto taps = [&](f32x4 acc[kC3Rows], int dz) {
+        bf16x8 wt[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) wt[k] = load8(wl + (dz * 9 + k) * 512);
+#pragma unroll
+        for (int i = 0; i < kC3Rows + 2; i++)
+#pragma unroll
+            for (int dx = 0; dx < 3; dx++) {
+                const bf16x8 v = load8(vl + (i * (kCx + 2) + dx) * 32);
+#pragma unroll
+                for (int dy = 0; dy < 3; dy++)
+                    if (i - dy >= 0 && i - dy < kC3Rows)
+                        acc[i - dy] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[3 * dy + dx], v, acc[i - dy], 0, 0, 0);
             }
+    };
+    auto emit = [&](const f32x4 acc[kC3Rows], int z) {
+        const int64_t v0 = (int64_t)z * g.sxy + (int64_t)y0 * g.X + x;
+        if (kMode == kFwdHead) {
+            // head: a vertex's channels are in four lanes; lane q then finishes rows q, q + 4, ..
+            float logit[kC3Rows / 4];
+#pragma unroll
+            for (int j = 0; j < kC3Rows; j++) {
+                float p[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) p[i] = hv[i] * bf2f((uint16_t)pack_bf(relu(acc[j][i] + bv[i]), 0.f));
+                float s = (p[0] + p[1]) + (p[2] + p[3]);
+                s += __shfl_xor(s, 16);
+                s += __shfl_xor(s, 32);
+                if (j % 4 == 0 || q == j % 4) logit[j / 4] = s;
+            }
+#pragma unroll
+            for (int k = 0; k < kC3Rows / 4; k++) {
+                const int j = 4 * k + q;
+                if (x < g.X && y0 + j < g.Y) prob[v0 + (int64_t)j * g.X] = 1.f / (1.f + expf(-(logit[k] + hb)));
+            }
+            return;
         }
-        const int co = r;
+        if (x >= g.X) return;
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int xo = x0 + 16 * s + 4 * q + i;
-                const bool in_range = xo < g.X;
-                const int64_t vo = (int64_t)xo + (int64_t)y * g.X + (int64_t)z * g.sxy;
-                float val = acc[s][i];
-                if (kMode == kBwd) {
-                    if (in_range && !(bf2f(gate[vo * 16 + co]) > 0.f)) val = 0.f;
-                    if (in_range) out[vo * 16 + co] = f2bf(val);
-                } else {
-                    val += sb[co];
-                    val = val > 0.f ? val : 0.f;
-                    if (kMode == kFwd) {
-                        if (in_range) out[vo * 16 + co] = f2bf(val);
-                    } else {
-                        // head: the 16 channels of a voxel sit in 16 consecutive lanes
-                        float p = sh[co] * bf2f(f2bf(val));
-                        p += __shfl_xor(p, 1);
-                        p += __shfl_xor(p, 2);
-                        p += __shfl_xor(p, 4);
-                        p += __shfl_xor(p, 8);
-                        if (in_range && co == 0) prob[vo] = 1.f / (1.f + expf(-(p + sh[16])));
-                    }
-                }
+        for (int j = 0; j < kC3Rows; j++) {
+            if (y0 + j >= g.Y) break;
+            const int64_t at = (v0 + (int64_t)j * g.X) * 16 + 4 * q;
+            uint2 p;
+            if (kMode == kFwd) {
+                p.x = pack_bf(relu(acc[j][0] + bv[0]), relu(acc[j][1] + bv[1]));
+                p.y = pack_bf(relu(acc[j][2] + bv[2]), relu(acc[j][3] + bv[3]));
+            } else {
+                const uint2 gs = *reinterpret_cast<const uint2*>(gate + at);
+                p.x = gated(gs.x, acc[j][0], acc[j][1]);
+                p.y = gated(gs.y, acc[j][2], acc[j][3]);
             }
+            *reinterpret_cast<uint2*>(out + at) = p;
+        }
+    };
+    f32x4 a[kC3Rows] = {}, b[kC3Rows] = {};  // of the layers below and at the input layer
+    load(z0 - 1);
+#pragma unroll 1
+    for (int z = z0 - 1; z <= z1; z++) {
+        __syncthreads();
+        stage.store(reinterpret_cast<uint4*>(sv));
+        if (z < z1) load(z + 1);
+        __syncthreads();
+        if (z > z0) {
+            taps(a, 2);
+            emit(a, z - 1);
+        }
+        if (z >= z0 && z < z1) {
+#pragma unroll
+            for (int j = 0; j < kC3Rows; j++) a[j] = b[j];
+            taps(a, 1);
+        }
+        if (z + 1 < z1) {
+#pragma unroll
+            for (int j = 0; j < kC3Rows; j++) b[j] = f32x4{};
+            taps(b, 0);
         }
     }
 }
@@ -546,6 +767,27 @@ __global__ void count_kernel(const uint8_t* __restrict__ m, int64_t n, unsigned 
     if ((threadIdx.x & 63) == 0 && c) atomicAdd(out, (unsigned long long)c);
 }
 
+// launch(grid, tiles) for all x * y * z tiles of the volume (fewer than 2^30: a
+// volume has at most 2^34 vertices and sides of 2^16, a tile 4 rows or more).
+template <class Launch>
+void for_tiles(const Geo& g, int x, int y, int z, Launch launch) {
+    auto along = [](int n, int side) { return (uint32_t)((n + side - 1) / side); };
+    Tiles t{0, 0, along(g.X, x), along(g.Y, y)};
+    const uint32_t all = t.x * t.y * along(g.Z, z);
+    for (; t.first < all; t.first += t.n) {
+        t.n = std::min(all - t.first, kMaxTiles);
+        launch(dim3(t.n), t);
+    }
+}
+// Layers a work-group of a convolution runs up: the more, the fewer layers are
+// read twice and the fewer weights staged, as long as there are two work-groups
+// per CU.
+inline int conv_layers(const Geo& g) {
+    const int64_t tiles = (int64_t)((g.X + kCx - 1) / kCx) * ((g.Y + kCy - 1) / kCy);
+    int n = 8;
+    while (n > 1 && tiles * ((g.Z + n - 1) / n) < 512) n /= 2;
+    return n;
+}
 inline uint32_t blocks_for(int64_t n, uint32_t cap = 16384) {
     const int64_t b = (n + kT - 1) / kT;
     return (uint32_t)(b < 1 ? 1 : (b > cap ? cap : b));
@@ -589,8 +831,7 @@ std::vector<float> cnn_initial_params(uint64_t seed) {
 hipError_t CnnState::ensure_volume(int64_t verts) {
     if (verts <= vol_cap) return hipSuccess;
     hipError_t e;
-    if ((e = tmp1.ensure(sizeof(double2) * verts)) != hipSuccess) return e;
-    if ((e = tmp2.ensure(sizeof(double2) * verts)) != hipSuccess) return e;
+    if ((e = tmp.ensure(sizeof(double2) * verts)) != hipSuccess) return e;
     if ((e = xin.ensure(sizeof(float) * verts)) != hipSuccess) return e;
     if ((e = a1.ensure(2 * 16 * verts)) != hipSuccess) return e;
     if ((e = a2.ensure(2 * 32 * verts)) != hipSuccess) return e;
@@ -611,7 +852,7 @@ hipError_t CnnState::ensure_train(int64_t verts) {
 }
 
 void CnnState::release_all() {
-    DevBuf* all[] = {&params, &grads, &m, &v, &pk, &parts, &loss, &tmp1, &tmp2, &xin, &a1, &a2, &a3,
+    DevBuf* all[] = {&params, &grads, &m, &v, &pk, &parts, &loss, &tmp, &xin, &a1, &a2, &a3,
                      &prob, &m0, &m1, &dz3, &dz2, &dz1};
     for (DevBuf* b : all) b->release();
     vol_cap = 0;
@@ -638,26 +879,31 @@ hipError_t cnn_pack(CnnState& s, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t cnn_forward(CnnState& s, const float* values, int X, int Y, int Z, bool keep_a3, hipStream_t st) {
+hipError_t cnn_forward(CnnState& s, const float* values, int X, int Y, int Z, bool keep_a3, float* prob, hipStream_t st) {
     const Geo g{X, Y, Z, (int64_t)X * Y};
-    const int64_t n = g.verts();
     const CnnPacked k = s.packed();
-    hipLaunchKernelGGL(norm_x_kernel, dim3(blocks_for(n)), dim3(kT), 0, st, values, g, s.tmp1.as<double2>());
-    hipLaunchKernelGGL(norm_y_kernel, dim3(blocks_for(n)), dim3(kT), 0, st, s.tmp1.as<double2>(), g, s.tmp2.as<double2>());
-    hipLaunchKernelGGL(norm_z_kernel, dim3(blocks_for(n)), dim3(kT), 0, st, s.tmp2.as<double2>(), values, g,
-                       s.xin.as<float>());
-    hipLaunchKernelGGL(conv1_kernel, dim3(blocks_for(n)), dim3(kT), 0, st, s.xin.as<float>(), g, k.w1, k.b1,
-                       s.a1.as<uint16_t>());
-    const int64_t t32 = (int64_t)((X + 31) / 32) * Y * Z, t64 = (int64_t)((X + 63) / 64) * Y * Z;
-    const uint32_t b32 = (uint32_t)std::min<int64_t>((t32 + 3) / 4, 65536), b64 = (uint32_t)std::min<int64_t>((t64 + 3) / 4, 65536);
-    hipLaunchKernelGGL(conv16to32_kernel<kFwd>, dim3(b32), dim3(kT), 0, st, s.a1.as<uint16_t>(), g, k.w2, k.b2,
-                       (const uint16_t*)nullptr, s.a2.as<uint16_t>());
-    if (keep_a3)
-        hipLaunchKernelGGL(conv32to16_kernel<kFwd>, dim3(b64), dim3(kT), 0, st, s.a2.as<uint16_t>(), g, k.w3, k.b3,
-                           k.head, (const uint16_t*)nullptr, s.a3.as<uint16_t>(), (float*)nullptr);
-    else
-        hipLaunchKernelGGL(conv32to16_kernel<kFwdHead>, dim3(b64), dim3(kT), 0, st, s.a2.as<uint16_t>(), g, k.w3,
-                           k.b3, k.head, (const uint16_t*)nullptr, (uint16_t*)nullptr, s.prob.as<float>());
+    const int layers = conv_layers(g);
+    for_tiles(g, kNormX, kNormY, 1, [&](dim3 n, Tiles t) {
+        hipLaunchKernelGGL(norm_xy_kernel, n, dim3(kT), 0, st, values, g, t, s.tmp.as<double2>());
+    });
+    for_tiles(g, 64, kT / 64, kNormZ, [&](dim3 n, Tiles t) {
+        hipLaunchKernelGGL(norm_z_kernel, n, dim3(kT), 0, st, s.tmp.as<double2>(), values, g, t, s.xin.as<float>());
+    });
+    for_tiles(g, 64, kC1Rows, kT / 64, [&](dim3 n, Tiles t) {
+        hipLaunchKernelGGL(conv1_kernel, n, dim3(kT), 0, st, s.xin.as<float>(), g, t, k.w1, k.b1, s.a1.as<uint16_t>());
+    });
+    for_tiles(g, kCx, kCy, layers, [&](dim3 n, Tiles t) {
+        hipLaunchKernelGGL(conv16to32_kernel<kFwd>, n, dim3(kT), 0, st, s.a1.as<uint16_t>(), g, t, layers, k.w2, k.b2,
+                           (const uint16_t*)nullptr, s.a2.as<uint16_t>());
+    });
+    for_tiles(g, kCx, kCy, layers, [&](dim3 n, Tiles t) {
+        if (keep_a3)
+            hipLaunchKernelGGL(conv32to16_kernel<kFwd>, n, dim3(kT), 0, st, s.a2.as<uint16_t>(), g, t, layers, k.w3, k.b3, k.head,
+                               (const uint16_t*)nullptr, s.a3.as<uint16_t>(), (float*)nullptr);
+        else
+            hipLaunchKernelGGL(conv32to16_kernel<kFwdHead>, n, dim3(kT), 0, st, s.a2.as<uint16_t>(), g, t, layers, k.w3, k.b3,
+                               k.head, (const uint16_t*)nullptr, (uint16_t*)nullptr, prob);
+    });
     return hipGetLastError();
 }
 
@@ -674,15 +920,18 @@ hipError_t cnn_backward(CnnState& s, int X, int Y, int Z, const uint8_t* target,
     hipLaunchKernelGGL(reduce_parts_kernel, dim3(1), dim3(kT), 0, st, s.parts.as<float>(), (int)hb, kHeadPart,
                        loss);
     hipLaunchKernelGGL(reorder_head_kernel, dim3(1), dim3(32), 0, st, loss, grad);
-    const int64_t t32 = (int64_t)((X + 31) / 32) * Y * Z, t64 = (int64_t)((X + 63) / 64) * Y * Z;
-    const uint32_t b32 = (uint32_t)std::min<int64_t>((t32 + 3) / 4, 65536), b64 = (uint32_t)std::min<int64_t>((t64 + 3) / 4, 65536);
     // dz2 = (dz3 conv^T W3) * (a2 > 0): a 16 -> 32 convolution with W3T
-    hipLaunchKernelGGL(conv16to32_kernel<kBwd>, dim3(b32), dim3(kT), 0, st, s.dz3.as<uint16_t>(), g, k.w3t,
-                       (const float*)nullptr, s.a2.as<uint16_t>(), s.dz2.as<uint16_t>());
+    const int layers = conv_layers(g);
+    for_tiles(g, kCx, kCy, layers, [&](dim3 n, Tiles t) {
+        hipLaunchKernelGGL(conv16to32_kernel<kBwd>, n, dim3(kT), 0, st, s.dz3.as<uint16_t>(), g, t, layers, k.w3t,
+                           (const float*)nullptr, s.a2.as<uint16_t>(), s.dz2.as<uint16_t>());
+    });
     // dz1 = (dz2 conv^T W2) * (a1 > 0): a 32 -> 16 convolution with W2T
-    hipLaunchKernelGGL(conv32to16_kernel<kBwd>, dim3(b64), dim3(kT), 0, st, s.dz2.as<uint16_t>(), g, k.w2t,
-                       (const float*)nullptr, (const float*)nullptr, s.a1.as<uint16_t>(), s.dz1.as<uint16_t>(),
-                       (float*)nullptr);
+    for_tiles(g, kCx, kCy, layers, [&](dim3 n, Tiles t) {
+        hipLaunchKernelGGL(conv32to16_kernel<kBwd>, n, dim3(kT), 0, st, s.dz2.as<uint16_t>(), g, t, layers, k.w2t,
+                           (const float*)nullptr, (const float*)nullptr, s.a1.as<uint16_t>(), s.dz1.as<uint16_t>(),
+                           (float*)nullptr);
+    });
     const int64_t nseg = (int64_t)((X + 63) / 64) * Y * Z;
     const int wb = (int)std::min<int64_t>(nseg, kGradBlocks);
     hipLaunchKernelGGL((wgrad_kernel<32, 16>), dim3(wb), dim3(kT), 0, st, s.a2.as<uint16_t>(), s.dz3.as<uint16_t>(), g,

@@ -35,7 +35,7 @@ struct CnnPacked {
 
 struct CnnState {
     DevBuf params, grads, m, v, pk, parts, loss;
-    DevBuf tmp1, tmp2, xin, a1, a2, a3, prob, m0, m1;
+    DevBuf tmp, xin, a1, a2, a3, prob, m0, m1;
     DevBuf dz3, dz2, dz1;
     int step = 0;
     int64_t vol_cap = 0;
@@ -48,8 +48,8 @@ struct CnnState {
 std::vector<float> cnn_initial_params(uint64_t seed);
 hipError_t cnn_pack(CnnState& s, hipStream_t st);
 // Normalisation + convolutions; keep_a3: store conv3's activations (training)
-// instead of the head's probabilities.
-hipError_t cnn_forward(CnnState& s, const float* values, int X, int Y, int Z, bool keep_a3, hipStream_t st);
+// instead of the head's probabilities, which go to prob.
+hipError_t cnn_forward(CnnState& s, const float* values, int X, int Y, int Z, bool keep_a3, float* prob, hipStream_t st);
 // Loss and gradient of the last forward(keep_a3) into s.grads (loss in s.loss[0]).
 hipError_t cnn_backward(CnnState& s, int X, int Y, int Z, const uint8_t* target, float pos_w, hipStream_t st);
 hipError_t cnn_adam(CnnState& s, float lr, hipStream_t st);

@@ -121,9 +121,9 @@ int msceer_cnn_predict(msceer_ctx* ctx, msceer_cnn* net, const float* values, in
     const float* d_values = nullptr;
     rc = stage(ctx, ctx->values, values, (size_t)V, dev, &d_values);
     if (rc) return rc;
-    CHECK_HIP(cnn_forward(s, d_values, (int)nx, (int)ny, (int)nz, false, ctx->stream));
-    CHECK_HIP(hipMemcpyAsync(prob_out, s.prob.ptr, sizeof(float) * V, dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost,
-                             ctx->stream));
+    CHECK_HIP(cnn_forward(s, d_values, (int)nx, (int)ny, (int)nz, false, dev ? prob_out : s.prob.as<float>(),
+                          ctx->stream));
+    if (!dev) CHECK_HIP(hipMemcpyAsync(prob_out, s.prob.ptr, sizeof(float) * V, hipMemcpyDeviceToHost, ctx->stream));
     CHECK_HIP(hipStreamSynchronize(ctx->stream));
     return MSCEER_OK;
 }
@@ -147,7 +147,7 @@ int msceer_cnn_gradient(msceer_ctx* ctx, msceer_cnn* net, const float* values, i
     const uint8_t* d_target = nullptr;
     rc = stage(ctx, ctx->mask, target, (size_t)V, dev, &d_target);
     if (rc) return rc;
-    CHECK_HIP(cnn_forward(s, d_values, (int)nx, (int)ny, (int)nz, true, ctx->stream));
+    CHECK_HIP(cnn_forward(s, d_values, (int)nx, (int)ny, (int)nz, true, nullptr, ctx->stream));
     CHECK_HIP(cnn_backward(s, (int)nx, (int)ny, (int)nz, d_target, pos_weight, ctx->stream));
     if (loss_out) CHECK_HIP(hipMemcpyAsync(loss_out, s.loss.ptr, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     if (grad_out)
@@ -186,7 +186,7 @@ int msceer_cnn_mask(msceer_ctx* ctx, msceer_cnn* net, const float* values, int64
     }
     unsigned long long* d_count = reinterpret_cast<unsigned long long*>(s.loss.as<float>() + 24);
     CHECK_HIP(hipMemsetAsync(d_count, 0, sizeof(unsigned long long), ctx->stream));
-    CHECK_HIP(cnn_forward(s, d_values, (int)nx, (int)ny, (int)nz, false, ctx->stream));
+    CHECK_HIP(cnn_forward(s, d_values, (int)nx, (int)ny, (int)nz, false, s.prob.as<float>(), ctx->stream));
     CHECK_HIP(cnn_mask(s, (int)nx, (int)ny, (int)nz, threshold, dilation, d_mask, d_count, ctx->stream));
     if (!dev) CHECK_HIP(hipMemcpyAsync(mask_out, d_mask, V, hipMemcpyDeviceToHost, ctx->stream));
     unsigned long long cnt = 0;
