@@ -290,11 +290,6 @@ pass1_kernel(GradSrc<float> src, VGrid g, LabelBuffers b, SeedList seeds, float 
             if (active && ev == kNone) {
                 bool moved = false;
                 ev = tracer_iterate(src, g, b.dest, true, dir, gthr, ethr, tr, next, moved);
-                if (ev == kOutOfVoxel) {
-                    next = tracer_reenter(src, g, tr);
-                    moved = true;
-                    ev = kNone;
-                }
                 if (kClaims && moved && np < kPath) path[(np++) * kThreads] = (int32_t)next;
             }
             if (__popcll(__ballot(ev != kNone)) >= enough) break;
@@ -477,10 +472,6 @@ ers_trace_kernel(GradSrc<double> src, VGrid g, const uint8_t* __restrict__ dest,
         int64_t next = 0;
         bool moved = false;
         int ev = tracer_iterate(src, g, dest, false, -1.0, gthr, ethr, tr, next, moved);
-        if (ev == kOutOfVoxel) {
-            next = tracer_reenter(src, g, tr);
-            ev = kNone;
-        }
         if (ev == kNone) continue;
         active = false;
         if (ev != kHitPreassigned) next = nearest(g, tr.cur, tr.near);
@@ -1032,10 +1023,6 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
                         }
                     } else {
                         ev = tracer_iterate(srcd, g, b.dest, false, dird, gthrd, ethrd, tr.d, next, moved);
-                        if (ev == kOutOfVoxel) {
-                            tracer_reenter(srcd, g, tr.d);
-                            ev = kNone;
-                        }
                     }
                 }
                 if (__popcll(__ballot(ev != kNone)) >= enough) break;

@@ -31,18 +31,12 @@ struct GradSrc<float> {
     const float* f;
     const uint8_t* seedmask;
     VGrid g;
-    __device__ __forceinline__ V3<float> at(int64_t v) const {
-        const float4 r = gradf[v];
-        return {r.x, r.y, r.z};
-    }
+    __device__ __forceinline__ const float4* field() const { return gradf; }
 };
 template <>
 struct GradSrc<double> {
     const double4* gradd;
-    __device__ __forceinline__ V3<double> at(int64_t v) const {
-        const double4 r = gradd[v];
-        return {r.x, r.y, r.z};
-    }
+    __device__ __forceinline__ const double4* field() const { return gradd; }
 };
 
 template <typename T>
@@ -92,6 +86,11 @@ __device__ __forceinline__ T clampc(T p, int n) {
 // boundary as Inbounds does).
 __device__ __forceinline__ int clampi(int v, int n) { return v < 0 ? 0 : (v >= n ? n - 1 : v); }
 
+// Index of a vertex (fewer than 2^31 in a volume).
+__device__ __forceinline__ uint32_t vertex_index(const VGrid& g, int x, int y, int z) {
+    return (uint32_t)x + (uint32_t)g.X * ((uint32_t)y + (uint32_t)g.Y * (uint32_t)z);
+}
+
 // (Away from the boundary the position lies inside the grid and the final
 // index clamp changes nothing; it only keeps a corrupt position in bounds.)
 template <typename T>
@@ -101,7 +100,7 @@ __device__ __forceinline__ int64_t nearest_xyz(const VGrid& g, const V3<T>& p, b
     x = clampi((int)qx, g.X);
     y = clampi((int)qy, g.Y);
     z = clampi((int)qz, g.Z);
-    return (int64_t)x + (int64_t)g.X * ((int64_t)y + (int64_t)g.Y * (int64_t)z);
+    return (int64_t)vertex_index(g, x, y, z);
 }
 
 template <typename T>
@@ -114,6 +113,40 @@ __device__ __forceinline__ int dist_to_boundary(const VGrid& g, int x, int y, in
     int m = min(x, g.X - 1 - x);
     m = min(m, min(y, g.Y - 1 - y));
     return min(m, min(z, g.Z - 1 - z));
+}
+
+// The 8 corner gradients of the voxel at (bx, by, bz); near the boundary its
+// upper corners may be clamped onto the lower ones.  One index (a volume has
+// fewer than 2^31 vertices) and the corners' distances from it: an index per
+// corner, from its coordinates in 64 bits, took about 70 more instructions per
+// step of a wave.
+template <typename T, class C>
+__device__ __forceinline__ void load_corners(const GradSrc<T>& src, const VGrid& g, C& c, int bx, int by, int bz,
+                                             bool near) {
+    int xs[2] = {bx, bx + 1}, ys[2] = {by, by + 1}, zs[2] = {bz, bz + 1};
+    if (near) {
+        if (bx >= g.X - 1) xs[0] = xs[1] = g.X - 1;
+        if (by >= g.Y - 1) ys[0] = ys[1] = g.Y - 1;
+        if (bz >= g.Z - 1) zs[0] = zs[1] = g.Z - 1;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        xs[k] = clampi(xs[k], g.X);
+        ys[k] = clampi(ys[k], g.Y);
+        zs[k] = clampi(zs[k], g.Z);
+    }
+    const auto* const p = src.field() + vertex_index(g, xs[0], ys[0], zs[0]);
+    const uint32_t ox = xs[1] > xs[0] ? 1u : 0u, oy = ys[1] > ys[0] ? (uint32_t)g.X : 0u;
+    const uint32_t oz = zs[1] > zs[0] ? (uint32_t)g.sxy : 0u;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const auto* q = p;
+        if (k & 1) q += ox;
+        if (k & 2) q += oy;
+        if (k & 4) q += oz;
+        const auto r = *q;
+        c.set(k, V3<T>{r.x, r.y, r.z});
+    }
 }
 
 // Adaptive Euler with step doubling (gi_adaptive_euler_advector.h:51-305) in
@@ -151,21 +184,7 @@ __device__ __forceinline__ void tracer_load(const GradSrc<T>& src, const VGrid& 
     t.bx = (int)b0.x;
     t.by = (int)b0.y;
     t.bz = (int)b0.z;
-    int xs[2] = {t.bx, t.bx + 1}, ys[2] = {t.by, t.by + 1}, zs[2] = {t.bz, t.bz + 1};
-    if (t.near) {
-        if (t.bx >= g.X - 1) xs[0] = xs[1] = g.X - 1;
-        if (t.by >= g.Y - 1) ys[0] = ys[1] = g.Y - 1;
-        if (t.bz >= g.Z - 1) zs[0] = zs[1] = g.Z - 1;
-    }
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        xs[k] = clampi(xs[k], g.X);
-        ys[k] = clampi(ys[k], g.Y);
-        zs[k] = clampi(zs[k], g.Z);
-    }
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-        t.c.set(k, src.at((int64_t)xs[k & 1] + (int64_t)g.X * ((int64_t)ys[(k >> 1) & 1] + (int64_t)g.Y * zs[k >> 2])));
+    load_corners(src, g, t.c, t.bx, t.by, t.bz, t.near);
 }
 
 // Voxel entry: gradient at the position and a fresh step length.
@@ -180,8 +199,10 @@ __device__ __forceinline__ void tracer_begin(Tracer<T, C>& t) {
 
 // One iteration.  kNone: the streamline goes on (moved: it entered the voxel
 // of vertex `next`); kHitPreassigned (next: the vertex reached), kLowGradient
-// and kOverMax end it; kOutOfVoxel asks the caller to enter the voxel of the
-// position (only a position changed outside a step could lead there).
+// and kOverMax end it.  (A step that leaves the voxel enters the next one at
+// once, so the reference's test at the top of its loop, whether the position
+// has left the voxel, is never true here; nor does a step length kept from an
+// iteration that did not move exceed the cap.)
 //
 // The gradient, its magnitude and the step cap are evaluated at the top of
 // every iteration, whatever the lane did in the one before (entered a voxel,
@@ -196,15 +217,11 @@ __device__ __forceinline__ int tracer_iterate(const GradSrc<T>& src, const VGrid
                                               T gthr, T ethr, Tracer<T, C>& t, int64_t& next, bool& moved) {
     moved = false;
     if (!(t.iters-- > 0)) return kOverMax;
-    const bool went = !(t.old.x == t.cur.x && t.old.y == t.cur.y && t.old.z == t.cur.z) && !t.fresh;
-    if (went && ((int)t.cur.x != (int)t.old.x || (int)t.cur.y != (int)t.old.y || (int)t.cur.z != (int)t.old.z))
-        return kOutOfVoxel;
     t.gr = trilin(t.c, t.cur.x - (T)t.bx, t.cur.y - (T)t.by, t.cur.z - (T)t.bz);
     t.gm = sqrt(t.gr.x * t.gr.x + t.gr.y * t.gr.y + t.gr.z * t.gr.z);
     const T cap = (T)kMaxStep / t.gm;
-    if (t.fresh || (went && t.gm * t.step > (T)kMaxStep)) t.step = cap;
+    if (t.fresh || t.gm * t.step > (T)kMaxStep) t.step = cap;
     t.fresh = false;
-    t.old = t.cur;
     if (t.gm < gthr) return kLowGradient;
     // dir = -1: ascending manifolds, flow downhill; +1: descending, uphill
     const T s = dir * t.step, hs = (dir * (T)0.5) * t.step;
@@ -218,6 +235,7 @@ __device__ __forceinline__ int tracer_iterate(const GradSrc<T>& src, const VGrid
         t.step = t.step * (T)0.5;
         return kNone;
     }
+    const V3<T> old = t.cur;
     t.cur = {t.cur.x + two.x, t.cur.y + two.y, t.cur.z + two.z};
     if (t.near) { t.cur.x = clampc(t.cur.x, g.X); t.cur.y = clampc(t.cur.y, g.Y); t.cur.z = clampc(t.cur.z, g.Z); }
     const T grow = t.step * (T)1.8;
@@ -228,7 +246,7 @@ __device__ __forceinline__ int tracer_iterate(const GradSrc<T>& src, const VGrid
     // the next iteration would leave the voxel: gather the next voxel's
     // corners while the destination byte is in flight
     const bool leave = t.iters > 0 &&
-                       ((int)t.cur.x != (int)t.old.x || (int)t.cur.y != (int)t.old.y || (int)t.cur.z != (int)t.old.z);
+                       ((int)t.cur.x != (int)old.x || (int)t.cur.y != (int)old.y || (int)t.cur.z != (int)old.z);
     if (leave) tracer_load(src, g, t, nx, ny, nz);
     if (d == kCertainTerminal || (stop_on_assigned && d == kAssigned)) return kHitPreassigned;
     if (leave) {
@@ -239,7 +257,7 @@ __device__ __forceinline__ int tracer_iterate(const GradSrc<T>& src, const VGrid
     return kNone;
 }
 
-// Enter the voxel of the position after kOutOfVoxel; returns the vertex nearest to it.
+// Enter the voxel of a position changed outside a step; returns the vertex nearest to it.
 template <typename T, class C>
 __device__ __forceinline__ int64_t tracer_reenter(const GradSrc<T>& src, const VGrid& g, Tracer<T, C>& t) {
     int x, y, z;
@@ -308,7 +326,7 @@ __device__ __forceinline__ int64_t nearest_l(const VGrid& g, const TracerL<C>& t
     x = clampi(t.bx + (int)floorf(t.cur.x + 0.5f), g.X);
     y = clampi(t.by + (int)floorf(t.cur.y + 0.5f), g.Y);
     z = clampi(t.bz + (int)floorf(t.cur.z + 0.5f), g.Z);
-    return (int64_t)x + (int64_t)g.X * ((int64_t)y + (int64_t)g.Y * (int64_t)z);
+    return (int64_t)vertex_index(g, x, y, z);
 }
 template <class C>
 __device__ __forceinline__ int64_t tracer_nearest(const VGrid& g, const TracerL<C>& t) {
@@ -344,21 +362,7 @@ __device__ __forceinline__ void tracer_load(const GradSrc<float>& src, const VGr
     t.bx = nbx;
     t.by = nby;
     t.bz = nbz;
-    int xs[2] = {t.bx, t.bx + 1}, ys[2] = {t.by, t.by + 1}, zs[2] = {t.bz, t.bz + 1};
-    if (t.near) {
-        if (t.bx >= g.X - 1) xs[0] = xs[1] = g.X - 1;
-        if (t.by >= g.Y - 1) ys[0] = ys[1] = g.Y - 1;
-        if (t.bz >= g.Z - 1) zs[0] = zs[1] = g.Z - 1;
-    }
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        xs[k] = clampi(xs[k], g.X);
-        ys[k] = clampi(ys[k], g.Y);
-        zs[k] = clampi(zs[k], g.Z);
-    }
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-        t.c.set(k, src.at((int64_t)xs[k & 1] + (int64_t)g.X * ((int64_t)ys[(k >> 1) & 1] + (int64_t)g.Y * zs[k >> 2])));
+    load_corners(src, g, t.c, t.bx, t.by, t.bz, t.near);
 }
 
 template <class C>
