@@ -98,6 +98,7 @@ struct WorkQueue {
     uint32_t* ahead_on;     // set once pass 3 traces vertices ahead
     uint32_t* chunk_head;   // next chunk of the items pass 2 queued
     uint32_t* first_count;  // items pass 2 queued
+    uint32_t* busy;         // pass-3 waves that hold anything but traces ahead
 };
 hipError_t launch_pass2(const VGrid& g, const LabelBuffers& b, const WorkQueue& q, hipStream_t s);
 // Certain regions by chains and a flood (certain.hip; seeds labelled

@@ -166,9 +166,10 @@ int run_integration(msceer_ctx* ctx, const VGrid& g, const LabelBuffers& b, cons
     // frontier buffer (at least V words; items beyond it report overflow)
     const uint64_t qcap = std::min<uint64_t>(std::min<uint64_t>(ctx->front0.bytes / 4, 2 * (uint64_t)V), 0xFFFFFFFFull);
     const WorkQueue q{ctx->front0.as<uint32_t>(), (uint32_t)qcap, ctl + kCtlCursor, ctl + kCtlCursor + 1,
-                      ctl + kCtlOverflow, ctl + kCtlCursor + 2, ctl + kCtlCursor + 3, ctl + kCtlCursor + 4};
+                      ctl + kCtlOverflow, ctl + kCtlCursor + 2, ctl + kCtlCursor + 3, ctl + kCtlCursor + 4,
+                      ctl + kCtlCursor + 5};
     CHECK_HIP(launch_fill_u32(q.items, (int64_t)qcap, 0xFFFFFFFFu, s));
-    CHECK_HIP(launch_zero(ctl + kCtlCursor, 5, s));
+    CHECK_HIP(launch_zero(ctl + kCtlCursor, 6, s));
     CHECK_HIP(launch_zero(ctl + kCtlOverflow, 1, s));
     CHECK_HIP(launch_pass2(g, b, q, s));
     // the labels pass 3 reads for its results
