@@ -258,6 +258,7 @@ int msceer_destroy(msceer_ctx* ctx) {
     ctx->aux = nullptr;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     batch_state_free(ctx);
     ctx->values.release();
     ctx->grad.release();
@@ -268,12 +269,14 @@ int msceer_destroy(msceer_ctx* ctx) {
     ctx->ldir.release();
     DevBuf* label_bufs[] = {&ctx->gradf, &ctx->gradd, &ctx->scan, &ctx->label, &ctx->label2, &ctx->dest, &ctx->seedmask, &ctx->redo,
                             &ctx->stamp, &ctx->rep, &ctx->rep2, &ctx->restriction, &ctx->host_io, &ctx->mask,
-                            &ctx->label_dsc, &ctx->seedmask2, &ctx->line_stamps, &ctx->lines};
+                            &ctx->label_dsc, &ctx->seedmask2, &ctx->line_stamps, &ctx->lines, &ctx->lines2};
     for (DevBuf* b : label_bufs) b->release();
     ctx->host_stage.release();
     if (ctx->h_ctl) (void)hipHostFree(ctx->h_ctl);
     for (int i = 0; i < msceer_ctx::kEvents; i++)
         if (ctx->ev[i]) (void)hipEventDestroy(ctx->ev[i]);
+    if (ctx->side_ev) (void)hipEventDestroy(ctx->side_ev);
+    if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->own) (void)hipStreamDestroy(ctx->own);
     delete ctx;
     return MSCEER_OK;

@@ -125,7 +125,7 @@ struct msceer_ctx {
     msceer::DevBuf gradf, gradd, scan, label, label2, dest, seedmask, redo, stamp, rep, rep2, restriction, host_io, mask;
     // accurate 1-manifolds: per-cell line stamps (two words, older tags are
     // ignored) with the next tag, and the saddle / window scratch
-    msceer::DevBuf line_stamps, lines;
+    msceer::DevBuf line_stamps, lines, lines2;
     uint32_t line_tag = 0;
     // descending 3-manifolds: their labels and seed mask
     msceer::DevBuf label_dsc, seedmask2;
@@ -139,6 +139,8 @@ struct msceer_ctx {
     msceer_label_stats last_labels{};
     std::shared_ptr<msceer::Tuning> tuning = std::make_shared<msceer::Tuning>();
     std::vector<msceer_ctx*> workers;  // contexts of msceer_batch's worker threads
+    hipStream_t side = nullptr;        // second stream of the 1-manifolds (default priority)
+    hipEvent_t side_ev = nullptr;      // its fork and join
     msceer_ctx* aux = nullptr;         // the descending labelling's own stream and buffers
     msceer::BatchState* gbatch = nullptr;  // msceer_batch_grad: buffers, plans and graphs
 };

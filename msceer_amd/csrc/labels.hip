@@ -744,7 +744,6 @@ int ondemand_impl(msceer_ctx* ctx, const float* values, int64_t nx, int64_t ny, 
             }
             // after needDSC2 the descending branch's field, zeroed at both families' seeds
             const double4* field = dsc2 ? ctx->aux->gradd.as<double4>() : b.gradd;
-            LineStats la, ld;
             // the saddles are the base pass's critical quads and edges, where
             // its lists had room for them (the labellings return before here
             // otherwise)
@@ -753,16 +752,19 @@ int ondemand_impl(msceer_ctx* ctx, const float* values, int64_t nx, int64_t ny, 
             const bool listed = asc2 || dsc2 || ctx->h_ctl[kCtlOverflow] == 0;
             const uint32_t n_edges = (uint32_t)list_total(ctx->h_ctl + kCtlList1, list1);
             const uint32_t n_quads = (uint32_t)list_total(ctx->h_ctl + kCtlList2, list2);
-            if (need & MSCEER_NEED_ASC1) {
-                rc = run_lines(ctx, d, d_values, d_grad, listed ? &list2 : nullptr, n_quads, field, restr, true,
-                               grad_thr, err_thr, max_iters, &la);
-                if (rc) return rc;
-            }
-            if (need & MSCEER_NEED_DSC1) {
-                rc = run_lines(ctx, d, d_values, d_grad, listed ? &list1 : nullptr, n_edges, field, restr, false,
-                               grad_thr, err_thr, max_iters, &ld);
-                if (rc) return rc;
-            }
+            LineFamily families[2];
+            int n_families = 0;
+            auto add = [&](bool asc, const MList* list, uint32_t n) {
+                families[n_families++] = LineFamily{d, d_values, d_grad, listed ? list : nullptr, n, field, restr, asc,
+                                                    grad_thr, err_thr, max_iters};
+            };
+            if (need & MSCEER_NEED_ASC1) add(true, &list2, n_quads);
+            if (need & MSCEER_NEED_DSC1) add(false, &list1, n_edges);
+            LineStats ls[2];
+            rc = run_lines(ctx, families, n_families, ls);
+            if (rc) return rc;
+            const LineStats la = (need & MSCEER_NEED_ASC1) ? ls[0] : LineStats{};
+            const LineStats ld = (need & MSCEER_NEED_DSC1) ? ls[n_families - 1] : LineStats{};
             st.lines_asc = (int64_t)la.traced;
             st.lines_dsc = (int64_t)ld.traced;
             st.lines_replayed = (int64_t)(la.replayed + ld.replayed);

@@ -433,35 +433,53 @@ uint32_t line_window() {
     return kWindow;
 }
 
-int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t* grad, const MList* saddles,
-              uint32_t n_saddles, const double4* gradd, int8_t* restr, bool asc, float gthr, float ethr, int max_iters,
-              LineStats* out) {
-    hipStream_t s = ctx->stream;
-    const VGrid g = make_vgrid(d.X, d.Y, d.Z);
-    CellGeom m{(int64_t)d.Mx, (int64_t)d.My, (int64_t)d.Mz, (int64_t)d.Mx * (int64_t)d.My};
-    if (d.cells >= 0xFFFFFFFFull) return MSCEER_ETOOBIG;
-    uint32_t* count = ctl_dev(ctx) + kCtlCount;
+namespace {
 
-    uint32_t S = n_saddles;
-    if (!saddles) {
-        // no list of them: count, below gather, by a scan over the cells
-        CHECK_HIP(launch_zero(count, 1, s));
-        hipLaunchKernelGGL(line_saddles_kernel, dim3(2048), dim3(kThreads), 0, s, grad, m, d.X, d.Y, values,
-                           asc ? 2 : 1, asc ? 1 : 0, nullptr, count, 0u);
-        CHECK_HIP(hipGetLastError());
-        int rc = read_ctl(ctx, kCtlCount, 1);
-        if (rc) return rc;
-        S = ctx->h_ctl[kCtlCount];
-    }
-    out->saddles = S;
-    if (S == 0) return MSCEER_OK;
-    if ((uint64_t)S * 7 >= 0xFFFFFFFFull) return MSCEER_ETOOBIG;
+// A family's lines: their seeds and scratch, the first window's tapes enqueued.
+struct LineJob {
+    uint64_t nslots = 0;
+    uint32_t W = 0;
+    LineArgs a{};
+};
+
+// Lines [w0, w1): tapes and links.
+int enqueue_tapes(const LineArgs& a, uint32_t w0, uint32_t w1, hipStream_t s) {
+    const uint32_t n = w1 - w0;
+    hipLaunchKernelGGL(line_ctl_init_kernel, dim3(1), dim3(64), 0, s, a.ctl, false);
+    hipLaunchKernelGGL(line_tape_kernel, dim3((n + kTapeThreads - 1) / kTapeThreads), dim3(kTapeThreads), 0, s, a, w0, w1);
+    hipLaunchKernelGGL(line_links_kernel, dim3(std::min<uint32_t>(n, 8192)), dim3(kTapeThreads), 0, s, a);
+    CHECK_HIP(hipGetLastError());
+    return MSCEER_OK;
+}
+
+// Number of lines' saddles: of the list, else counted by a scan over the cells.
+int count_saddles(msceer_ctx* ctx, const LineFamily& f, const CellGeom& m, uint32_t* S) {
+    *S = f.n_saddles;
+    if (f.saddles) return MSCEER_OK;
+    hipStream_t s = ctx->stream;
+    CHECK_HIP(launch_zero(ctl_dev(ctx) + kCtlCount, 1, s));
+    hipLaunchKernelGGL(line_saddles_kernel, dim3(2048), dim3(kThreads), 0, s, f.grad, m, f.d.X, f.d.Y, f.values,
+                       f.asc ? 2 : 1, f.asc ? 1 : 0, nullptr, ctl_dev(ctx) + kCtlCount, 0u);
+    CHECK_HIP(hipGetLastError());
+    int rc = read_ctl(ctx, kCtlCount, 1);
+    if (rc) return rc;
+    *S = ctx->h_ctl[kCtlCount];
+    return MSCEER_OK;
+}
+
+CellGeom cell_geom(const Dims& d) {
+    return CellGeom{(int64_t)d.Mx, (int64_t)d.My, (int64_t)d.Mz, (int64_t)d.Mx * (int64_t)d.My};
+}
+
+// Seeds and the first window's tapes of a family with S saddles, on stream s
+// (the seeds by a scan, where the saddles are not listed, use the context's
+// counter: then s is its stream).  The tapes of the first window read no label.
+int begin_lines(msceer_ctx* ctx, const LineFamily& f, uint32_t S, DevBuf& buf, hipStream_t s, LineJob* job) {
+    const VGrid g = make_vgrid(f.d.X, f.d.Y, f.d.Z);
+    const CellGeom m = cell_geom(f.d);
+    uint32_t* count = ctl_dev(ctx) + kCtlCount;
     const uint64_t nslots = 7ull * S;
     const uint32_t W = (uint32_t)std::min<uint64_t>(nslots, line_window());
-
-    // two stamps per cell, refilled when they are new or the tags run out
-    if (ctx->line_stamps.bytes < 8 * d.cells) ctx->line_tag = 0;
-    CHECK_HIP(ctx->line_stamps.ensure(8 * d.cells));
     // tape pool: 128 slots per line of a window (volumes of noise and mixtures
     // record 20 to 40), at least 2^15 chunks
     const uint32_t chunks = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(2ull * W, 1u << 15), 1u << 22);
@@ -482,52 +500,63 @@ int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t
     const size_t o_ended = off; off += al((size_t)W * 4);
     const size_t o_lctl = off; off += al(4 * kLcWords);
     const size_t o_tmp = off; off += al(tmp_bytes);
-    CHECK_HIP(ctx->lines.ensure(off));
-    char* base = ctx->lines.as<char>();
+    CHECK_HIP(buf.ensure(off));
+    char* base = buf.as<char>();
     uint64_t* keys = (uint64_t*)(base + o_keys);
     uint64_t* sorted = (uint64_t*)(base + o_sorted);
     uint32_t* slots = (uint32_t*)(base + o_slots);
     uint32_t* lctl = (uint32_t*)(base + o_lctl);
 
-    if (saddles) {
+    if (f.saddles) {
         hipLaunchKernelGGL(line_saddle_list_kernel, dim3(std::min<uint32_t>(blocks_for(S), 1024)), dim3(kThreads), 0, s,
-                           *saddles, m, d.X, d.Y, values, asc ? 1 : 0, keys, S);
+                           *f.saddles, m, f.d.X, f.d.Y, f.values, f.asc ? 1 : 0, keys, S);
     } else {
         CHECK_HIP(launch_zero(count, 1, s));
-        hipLaunchKernelGGL(line_saddles_kernel, dim3(2048), dim3(kThreads), 0, s, grad, m, d.X, d.Y, values,
-                           asc ? 2 : 1, asc ? 1 : 0, keys, count, S);
+        hipLaunchKernelGGL(line_saddles_kernel, dim3(2048), dim3(kThreads), 0, s, f.grad, m, f.d.X, f.d.Y, f.values,
+                           f.asc ? 2 : 1, f.asc ? 1 : 0, keys, count, S);
     }
     CHECK_HIP(hipGetLastError());
     CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(base + o_tmp, tmp_bytes, keys, sorted, (int)S, 0, 64, s));
-    hipLaunchKernelGGL(line_seeds_kernel, dim3(blocks_for(S)), dim3(kThreads), 0, s, grad, m, sorted, S,
-                       asc ? 1 : 0, slots);
+    hipLaunchKernelGGL(line_seeds_kernel, dim3(blocks_for(S)), dim3(kThreads), 0, s, f.grad, m, sorted, S,
+                       f.asc ? 1 : 0, slots);
     CHECK_HIP(hipGetLastError());
 
-    LineArgs a{};
-    a.src = GradSrc<double>{gradd};
+    LineArgs& a = job->a;
+    a.src = GradSrc<double>{f.gradd};
     a.g = g;
     a.m = m;
     a.slots = slots;
-    a.restr = restr;
-    a.target = asc ? 4 : 5;
-    a.asc = asc;
-    a.gthr = (double)gthr;
-    a.ethr = (double)ethr;
-    a.max_iters = max_iters;
+    a.restr = f.restr;
+    a.target = f.asc ? 4 : 5;
+    a.asc = f.asc;
+    a.gthr = (double)f.gthr;
+    a.ethr = (double)f.ethr;
+    a.max_iters = f.max_iters;
     a.pool = TapePool{(uint64_t*)(base + o_pool), chunks, lctl + kLcTop};
     a.wmask = (uint64_t*)(base + o_wmask);
     a.active = (uint32_t*)(base + o_active);
     a.head = (uint32_t*)(base + o_head);
     a.ended = (uint32_t*)(base + o_ended);
     a.stamp[0] = ctx->line_stamps.as<uint32_t>();
-    a.stamp[1] = a.stamp[0] + d.cells;
+    a.stamp[1] = a.stamp[0] + f.d.cells;
     a.ctl = lctl;
     hipLaunchKernelGGL(line_ctl_init_kernel, dim3(1), dim3(64), 0, s, lctl, true);
     CHECK_HIP(hipGetLastError());
 
+    job->nslots = nslots;
+    job->W = W;
+    return enqueue_tapes(a, 0, (uint32_t)std::min<uint64_t>(nslots, W), s);
+}
+
+// The rest of a family's lines, on the context's stream.
+int finish_lines(msceer_ctx* ctx, const LineJob& job, LineStats* out) {
+    hipStream_t s = ctx->stream;
+    const LineArgs& a = job.a;
+    const uint64_t nslots = job.nslots;
+    const uint32_t W = job.W;
     uint32_t h[kLcWords];
     auto read_back = [&]() -> int {
-        CHECK_HIP(hipMemcpyAsync(h, lctl, sizeof(h), hipMemcpyDeviceToHost, s));
+        CHECK_HIP(hipMemcpyAsync(h, a.ctl, sizeof(h), hipMemcpyDeviceToHost, s));
         CHECK_HIP(hipStreamSynchronize(s));
         return MSCEER_OK;
     };
@@ -543,11 +572,10 @@ int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t
             ctx->line_tag = kTopTag;
         }
         const uint32_t wave_blocks = std::min<uint32_t>(blocks_for((uint64_t)n * 64), 2048);
-        hipLaunchKernelGGL(line_ctl_init_kernel, dim3(1), dim3(64), 0, s, lctl, false);
-        hipLaunchKernelGGL(line_tape_kernel, dim3((n + kTapeThreads - 1) / kTapeThreads), dim3(kTapeThreads), 0, s, a,
-                           a0, w1);
-        hipLaunchKernelGGL(line_links_kernel, dim3(std::min<uint32_t>(n, 8192)), dim3(kTapeThreads), 0, s, a);
-        CHECK_HIP(hipGetLastError());
+        if (w0 > 0) {
+            int rc = enqueue_tapes(a, a0, w1, s);
+            if (rc) return rc;
+        }
         out->windows++;
         // rounds in groups; the host reads back only whether the last one
         // still changed a line (then the commit behind it did nothing)
@@ -593,6 +621,68 @@ int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t
     out->traced = h[kLcTraced];
     out->replayed = h[kLcCut];
     out->voxels = h[kLcVoxels];
+    return MSCEER_OK;
+}
+
+
+}  // namespace
+
+// A second family's tapes are traced on another stream beside the first's: the
+// tape kernels last as long as their longest streamlines and leave most of the
+// chip idle (256^3 mixture: 2.4 and 3.0 ms one after the other).  The labels
+// are still resolved one family after the other.  Without memory for a second
+// set of tapes the families take turns with one.
+int run_lines(msceer_ctx* ctx, const LineFamily* families, int n, LineStats* out) {
+    hipStream_t s = ctx->stream;
+    LineJob jobs[2];
+    uint32_t S[2] = {0, 0};
+    bool begun[2] = {false, false};
+    for (int i = 0; i < n; i++) {
+        const Dims& d = families[i].d;
+        if (d.cells >= 0xFFFFFFFFull) return MSCEER_ETOOBIG;
+        int rc = count_saddles(ctx, families[i], cell_geom(d), &S[i]);
+        if (rc) return rc;
+        out[i].saddles = S[i];
+        if ((uint64_t)S[i] * 7 >= 0xFFFFFFFFull) return MSCEER_ETOOBIG;
+        // two stamps per cell, refilled when they are new or the tags run out
+        if (ctx->line_stamps.bytes < 8 * d.cells) ctx->line_tag = 0;
+        if (S[i]) CHECK_HIP(ctx->line_stamps.ensure(8 * d.cells));
+    }
+    // whatever happens, nothing is left running on the second stream
+    struct Join {
+        msceer_ctx* ctx;
+        bool on = false;
+        ~Join() {
+            if (on) (void)hipStreamSynchronize(ctx->side);
+        }
+    } join{ctx};
+    if (n == 2 && S[0] && S[1] && families[1].saddles) {
+        if (!ctx->side) CHECK_HIP(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
+        if (!ctx->side_ev) CHECK_HIP(hipEventCreateWithFlags(&ctx->side_ev, hipEventDisableTiming));
+        CHECK_HIP(hipEventRecord(ctx->side_ev, s));
+        CHECK_HIP(hipStreamWaitEvent(ctx->side, ctx->side_ev, 0));
+        join.on = true;
+        begun[1] = begin_lines(ctx, families[1], S[1], ctx->lines2, ctx->side, &jobs[1]) == MSCEER_OK;
+        if (!begun[1]) {
+            (void)hipGetLastError();
+            CHECK_HIP(hipStreamSynchronize(ctx->side));
+            jobs[1] = LineJob{};
+        }
+    }
+    for (int i = 0; i < n; i++) {
+        if (S[i] == 0) continue;
+        int rc;
+        if (begun[i]) {
+            CHECK_HIP(hipEventRecord(ctx->side_ev, ctx->side));
+            CHECK_HIP(hipStreamWaitEvent(s, ctx->side_ev, 0));
+        } else {
+            rc = begin_lines(ctx, families[i], S[i], ctx->lines, s, &jobs[i]);
+            if (rc) return rc;
+        }
+        rc = finish_lines(ctx, jobs[i], &out[i]);
+        if (rc) return rc;
+    }
+    join.on = false;  // (the context's stream has waited for it)
     return MSCEER_OK;
 }
 

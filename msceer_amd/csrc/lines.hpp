@@ -21,14 +21,27 @@ struct LineStats {
     uint64_t overflows = 0;   // windows cut short where the tape pool ran out
 };
 
-// The digitized 1-manifolds of one family added onto `restr` (device, one
-// int8 per cell): asc = from the 2-saddles up (value 4), else from the
-// 1-saddles down (value 5).  grad: the steepest .grad (pairs of the lower-star
-// pass); saddles (may be null: the cells are scanned): its list of the
-// critical cells of that dimension, n_saddles of them; gradd: the FP64
-// gradient field the streamlines follow.
-int run_lines(msceer_ctx* ctx, const Dims& d, const float* values, const uint8_t* grad, const MList* saddles,
-              uint32_t n_saddles, const double4* gradd, int8_t* restr, bool asc, float gthr, float ethr, int max_iters,
-              LineStats* out);
+// One family of 1-manifolds: asc = from the 2-saddles up (value 4), else from
+// the 1-saddles down (value 5).  grad: the steepest .grad (pairs of the
+// lower-star pass); saddles (may be null: the cells are scanned): its list of
+// the critical cells of that dimension, n_saddles of them; gradd: the FP64
+// gradient field the streamlines follow; restr: the labels (device, one int8
+// per cell) the lines are digitized into.
+struct LineFamily {
+    Dims d;
+    const float* values;
+    const uint8_t* grad;
+    const MList* saddles;
+    uint32_t n_saddles;
+    const double4* gradd;
+    int8_t* restr;
+    bool asc;
+    float gthr, ethr;
+    int max_iters;
+};
+
+// The lines of n (at most two) families of one volume, one family after the
+// other; out: n.
+int run_lines(msceer_ctx* ctx, const LineFamily* families, int n, LineStats* out);
 
 }  // namespace msceer
