@@ -183,6 +183,7 @@ __global__ void __launch_bounds__(kTapeThreads) line_tape_kernel(LineArgs a, uin
     uint32_t first = kNoLine;
     if (c != kNoLine) {
         TapeLabels lab{a.restr, a.target, w0 > 0, a.pool, hist + threadIdx.x, (uint32_t)kTapeThreads};
+        lab.geom = a.m;
         uint32_t vox = 0;
         trace_line(a.src, a.g, a.m, c, a.asc, a.gthr, a.ethr, a.max_iters, lab, &vox);
         lab.finish();

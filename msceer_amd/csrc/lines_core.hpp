@@ -33,7 +33,20 @@ struct CellGeom {
     __device__ bool inside(int64_t x, int64_t y, int64_t z) const {
         return x >= 0 && y >= 0 && z >= 0 && x < Mx && y < My && z < Mz;
     }
+    // the same for coordinates from cell_floor (an id has 32 bits, an extent 17)
+    __device__ __forceinline__ uint32_t id32(int x, int y, int z) const {
+        return (uint32_t)x + (uint32_t)Mx * ((uint32_t)y + (uint32_t)My * (uint32_t)z);
+    }
+    __device__ __forceinline__ bool inside32(int x, int y, int z) const {
+        return (uint32_t)x < (uint32_t)Mx && (uint32_t)y < (uint32_t)My && (uint32_t)z < (uint32_t)Mz;
+    }
 };
+
+// floor(v), cut off far outside any volume so that twice it fits an int.
+__device__ __forceinline__ int cell_floor(double v) {
+    const int f = (int)floor(v);
+    return f < -(1 << 29) ? -(1 << 29) : (f > (1 << 29) ? 1 << 29 : f);
+}
 
 // Order key of a float: monotone, -0 and +0 equal (as float comparison has them).
 __device__ __forceinline__ uint32_t value_key(float f) {
@@ -60,63 +73,91 @@ __device__ __forceinline__ double comp(const V3<double>& v, int a) { return a ==
 // in order (cell, face, cell, face, ...: at most six) without looking at any
 // label; digitize labels them in that order and stops at the first one that
 // already carries the target.
-__device__ inline int digitize_cells(const CellGeom& m, V3<double> a, V3<double> b, bool asc, uint32_t* out) {
+__device__ __forceinline__ int digitize_cells(const CellGeom& m, V3<double> a, V3<double> b, bool asc, uint32_t* out) {
     if (!asc) {
         a = {a.x + 0.5, a.y + 0.5, a.z + 0.5};
         b = {b.x + 0.5, b.y + 0.5, b.z + 0.5};
     }
     const V3<double> ab{b.x - a.x, b.y - a.y, b.z - a.z};
-    uint32_t face[3];
-    double tc[3];
+    // the faces crossed, at most one per axis; every index below is known when
+    // compiled, so they stay in registers, and the faces' coordinates are kept
+    // (from the id they cost two divisions each)
+    uint32_t face[3] = {};
+    double tc[3] = {};
+    int p[3][3] = {};
     int n = 0;
+#pragma unroll
     for (int d = 0; d < 3; d++) {
         const double av = comp(a, d), bv = comp(b, d);
         const int va = (int)floor(av), vb = (int)floor(bv);
         if (va == vb) continue;
         const int plane = va > vb ? va : vb;
         const double t = ((double)plane - av) / (bv - av);
-        tc[n] = t;
         if (t < 0 || t > 1) return 0;
-        int64_t fc[3];
+        int fc[3];
+#pragma unroll
         for (int k = 0; k < 3; k++)
-            fc[k] = 2 * (int64_t)floor(comp(ab, k) * t + comp(a, k)) + (k == d ? 0 : 1) - (asc ? 0 : 1);
-        if (!m.inside(fc[0], fc[1], fc[2])) return 0;
-        face[n++] = m.id(fc[0], fc[1], fc[2]);
+            fc[k] = 2 * cell_floor(comp(ab, k) * t + comp(a, k)) + (k == d ? 0 : 1) - (asc ? 0 : 1);
+        if (!m.inside32(fc[0], fc[1], fc[2])) return 0;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (i == n) {
+                tc[i] = t;
+                face[i] = m.id32(fc[0], fc[1], fc[2]);
+                for (int k = 0; k < 3; k++) p[i][k] = fc[k];
+            }
+        n++;
     }
     if (n == 0) return 0;
-    for (int i = 0; i < n; i++)
-        for (int j = i; j < n; j++)
-            if (tc[i] > tc[j]) {
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = i + 1; j < 3; j++)
+            if (j < n && tc[i] > tc[j]) {
                 const uint32_t tf = face[i]; face[i] = face[j]; face[j] = tf;
                 const double tt = tc[i]; tc[i] = tc[j]; tc[j] = tt;
+                for (int k = 0; k < 3; k++) { const int tp = p[i][k]; p[i][k] = p[j][k]; p[j][k] = tp; }
             }
-    const int64_t s0 = 2 * (int64_t)floor(a.x) + (asc ? 1 : 0), s1 = 2 * (int64_t)floor(a.y) + (asc ? 1 : 0),
-                  s2 = 2 * (int64_t)floor(a.z) + (asc ? 1 : 0);
-    if (!m.inside(s0, s1, s2)) return 0;
-    uint32_t cur = m.id(s0, s1, s2);
+    const int s0 = 2 * cell_floor(a.x) + (asc ? 1 : 0), s1 = 2 * cell_floor(a.y) + (asc ? 1 : 0),
+              s2 = 2 * cell_floor(a.z) + (asc ? 1 : 0);
+    if (!m.inside32(s0, s1, s2)) return 0;
+    uint32_t cur = m.id32(s0, s1, s2);
     int k = 0;
-    for (int i = 0; i < n; i++) {
-        int64_t p[3];
-        m.xyz(face[i], p[0], p[1], p[2]);
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        if (i >= n) continue;
         bool has = false;
         uint32_t next = cur;
+#pragma unroll
         for (int d = 0; d < 3; d++) {
-            if (asc ? (p[d] & 1) != 0 : (p[d] & 1) == 0) continue;
-            if (p[d] < m.ext(d) - 1) {
-                const uint32_t c = (uint32_t)((int64_t)face[i] + m.off(d));
+            if (asc ? (p[i][d] & 1) != 0 : (p[i][d] & 1) == 0) continue;
+            if (p[i][d] < (int)m.ext(d) - 1) {
+                const uint32_t c = face[i] + (uint32_t)m.off(d);
                 if (c == cur) has = true; else next = c;
             }
-            if (p[d] > 0) {
-                const uint32_t c = (uint32_t)((int64_t)face[i] - m.off(d));
+            if (p[i][d] > 0) {
+                const uint32_t c = face[i] - (uint32_t)m.off(d);
                 if (c == cur) has = true; else next = c;
             }
         }
         if (!has) continue;
-        out[k++] = cur;
-        out[k++] = face[i];
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+            if (k == 2 * q) {
+                out[2 * q] = cur;
+                out[2 * q + 1] = face[i];
+            }
+        k += 2;
         cur = next;
     }
     return k;
+}
+
+// cells[k] of digitize_cells, by selects.
+__device__ __forceinline__ uint32_t pick6(const uint32_t* cells, int k) {
+    const uint32_t c0 = cells[0], c1 = cells[1], c2 = cells[2], c3 = cells[3], c4 = cells[4], c5 = cells[5];
+    const uint32_t lo = k == 0 ? c0 : (k == 1 ? c1 : c2), hi = k == 3 ? c3 : (k == 4 ? c4 : c5);
+    return k < 3 ? lo : hi;
 }
 
 // The seed cells of saddle s from the short V-path search
@@ -224,9 +265,10 @@ struct TapeLabels {
     uint32_t nhist = 0, last = kNoLine;
     uint32_t head = kNoLine, chunk = kNoLine, fill = 0, nchunks = 0;
     bool over = false, staying = false, asc = false;
-    const CellGeom* geom = nullptr;
+    CellGeom geom{};
     V3<double> from{}, to{};
-    __device__ void append(uint32_t kind, uint32_t c) {
+    // first: the first entry of a list
+    __device__ __forceinline__ void append(uint32_t kind, uint32_t c, bool first = false) {
         if (over) return;
         if (chunk == kNoLine || fill == kTapeChunk - 1) {
             const uint32_t at = nchunks < kMaxTapeChunks ? atomicAdd(pool.top, 1u) : kNoLine;
@@ -241,54 +283,61 @@ struct TapeLabels {
             nchunks++;
         }
         fill++;
-        pool.slots[(uint64_t)chunk * kTapeChunk + fill] = (uint64_t)(kind << kKindShift | kNoPrev) << 32 | c;
+        pool.slots[(uint64_t)chunk * kTapeChunk + fill] =
+            (uint64_t)(kind << kKindShift | kNoPrev | (first ? kFirst : 0u)) << 32 | c;
     }
-    // kind: kList or kStop with the first-of-a-list flag folded in by the caller
-    __device__ void append_list(uint32_t kind, uint32_t c, bool first) {
-        append(kind, c);
-        if (first && !over) pool.slots[(uint64_t)chunk * kTapeChunk + fill] |= (uint64_t)kFirst << 32;
-    }
-    __device__ void finish() {
+    __device__ __forceinline__ void finish() {
         if (!over && chunk != kNoLine) pool.slots[(uint64_t)chunk * kTapeChunk] = (uint64_t)fill << 32 | kNoLine;
     }
-    __device__ void stop_here(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool up) {
+    __device__ __forceinline__ void stop_here(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool up) {
         staying = true;
-        geom = &m;
+        geom = m;
         from = a;
         to = b;
         asc = up;
     }
-    __device__ void leave() { staying = false; }
-    __device__ bool test(uint32_t c) {
+    __device__ __forceinline__ void leave() { staying = false; }
+    __device__ __forceinline__ bool test(uint32_t c) {
         if (c == last) return false;
         last = c;
         append(staying ? kStay : kExit, c);
         if (staying) {
-            uint32_t cells[6];
-            const int n = digitize_cells(*geom, from, to, asc, cells);
-            for (int k = 0; k < n; k++) append_list(kStop, cells[k], k == 0);
+            uint32_t cells[6] = {};
+            const int n = digitize_cells(geom, from, to, asc, cells);
+#pragma unroll 1
+            for (int k = 0; k < n; k++) append(kStop, pick6(cells, k), k == 0);
         }
         bool hit = committed && restr[c] == target;
         const uint32_t n = nhist < kHistory ? nhist : kHistory;
-        for (uint32_t k = 0; k < n; k++) hit = hit || hist[k * hstride] == c;
+        // (reads of eight words in flight at a time; those beyond n count for nothing)
+        for (uint32_t k = 0; k < n; k += 8) {
+            uint32_t h[8];
+#pragma unroll
+            for (uint32_t j = 0; j < 8; j++) h[j] = hist[(k + j) * hstride];
+#pragma unroll
+            for (uint32_t j = 0; j < 8; j++) hit |= (h[j] == c) & (k + j < n);
+        }
         return hit;
     }
-    __device__ void list(const uint32_t* cells, int n) {
+    __device__ __forceinline__ void list(const uint32_t* cells, int n) {
+#pragma unroll 1
         for (int k = 0; k < n; k++) {
-            append_list(kList, cells[k], k == 0);
-            if (cells[k] == last) last = kNoLine;
+            const uint32_t c = pick6(cells, k);
+            append(kList, c, k == 0);
+            if (c == last) last = kNoLine;
         }
         // an exit without a list: the next test is recorded again, so that no
         // later list is taken for this exit's
         if (n > 0) hist[(nhist++ % kHistory) * hstride] = cells[0];
         else last = kNoLine;
     }
-    __device__ bool ok() const { return !over; }
+    __device__ __forceinline__ bool ok() const { return !over; }
 };
 
-__device__ inline void digitize(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool asc, TapeLabels& lab) {
-    uint32_t cells[6];
-    lab.list(cells, digitize_cells(m, a, b, asc, cells));
+__device__ __forceinline__ void digitize(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool asc, TapeLabels& lab) {
+    uint32_t cells[6] = {};
+    const int n = digitize_cells(m, a, b, asc, cells);
+    lab.list(cells, n);
 }
 
 // What a line does along its tape, chunk by chunk.
@@ -545,18 +594,19 @@ struct ReplayLabels {
 // Label the cells of digitize_cells in order; stop at the first one that
 // already carries the target.
 template <class L>
-__device__ void digitize(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool asc, L& lab) {
-    uint32_t cells[6];
+__device__ __forceinline__ void digitize(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool asc, L& lab) {
+    uint32_t cells[6] = {};
     const int n = digitize_cells(m, a, b, asc, cells);
     for (int k = 0; k < n; k++) {
-        if (lab.test(cells[k])) return;
-        lab.write(cells[k]);
+        const uint32_t c = pick6(cells, k);
+        if (lab.test(c)) return;
+        lab.write(c);
         if (!lab.ok()) return;
     }
 }
 
 template <class L>
-__device__ int advect_voxel(const VGrid& g, const CellGeom& m, Tracer<double>& t, const V3<double>& start, double dir,
+__device__ __forceinline__ int advect_voxel(const VGrid& g, const CellGeom& m, Tracer<double>& t, const V3<double>& start, double dir,
                             double gthr, double ethr, bool asc, L& lab) {
     while (true) {
         if (!(t.iters-- > 0)) return kOverMax;
@@ -592,11 +642,11 @@ __device__ int advect_voxel(const VGrid& g, const CellGeom& m, Tracer<double>& t
             lab.stop_here(m, start, t.cur, asc);
         else
             lab.leave();
-        const int64_t cx = asc ? 2 * (int64_t)floor(t.cur.x) + 1 : 2 * (int64_t)floor(t.cur.x + 0.5);
-        const int64_t cy = asc ? 2 * (int64_t)floor(t.cur.y) + 1 : 2 * (int64_t)floor(t.cur.y + 0.5);
-        const int64_t cz = asc ? 2 * (int64_t)floor(t.cur.z) + 1 : 2 * (int64_t)floor(t.cur.z + 0.5);
-        if (!m.inside(cx, cy, cz)) continue;
-        const bool hit = lab.test(m.id(cx, cy, cz));
+        const int cx = asc ? 2 * cell_floor(t.cur.x) + 1 : 2 * cell_floor(t.cur.x + 0.5);
+        const int cy = asc ? 2 * cell_floor(t.cur.y) + 1 : 2 * cell_floor(t.cur.y + 0.5);
+        const int cz = asc ? 2 * cell_floor(t.cur.z) + 1 : 2 * cell_floor(t.cur.z + 0.5);
+        if (!m.inside32(cx, cy, cz)) continue;
+        const bool hit = lab.test(m.id32(cx, cy, cz));
         if (!lab.ok()) return kAbort;
         if (hit) return kHitPreassigned;
     }
@@ -604,7 +654,7 @@ __device__ int advect_voxel(const VGrid& g, const CellGeom& m, Tracer<double>& t
 
 // IntegrateStreamline from the centre of seed cell `seed` (cell coordinates / 2).
 template <class L>
-__device__ int trace_line(const GradSrc<double>& src, const VGrid& g, const CellGeom& m, uint32_t seed, bool asc,
+__device__ __forceinline__ int trace_line(const GradSrc<double>& src, const VGrid& g, const CellGeom& m, uint32_t seed, bool asc,
                           double gthr, double ethr, int max_iters, L& lab, uint32_t* voxels) {
     int64_t sx, sy, sz;
     m.xyz(seed, sx, sy, sz);
