@@ -379,12 +379,6 @@ __device__ __forceinline__ int all6(const VGrid& g, int64_t i, int64_t nb[6]) {
 constexpr uint32_t kEmptySlot = 0xFFFFFFFFu;             // queue slot not written yet
 constexpr uint64_t kIdleTicks = 400000000ull;  // 4 s of the 100 MHz real-time counter
 
-__device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    return x;
-}
-
 __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t x, int lane) {
     uint32_t incl = x;
 #pragma unroll
