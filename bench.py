@@ -193,7 +193,7 @@ def bench_labels(args):
                           "algorithmic_bytes": 8.0 * V, "kernel_ms": stage["integrate"],
                           "pass3_ms": stage["pass3"],
                           "certain_rounds_share_of_total": round(stage["regions"] / stage["total"], 4),
-                          "note": "latency-bound: dependent streamline steps and certain-region levels, "
+                          "note": "latency-bound: dependent streamline steps, "
                                   "not bytes"},
              "stage_ms": stage,
              "counts": {k: int(last[k]) for k in ("minima", "regions", "traced_fp32", "over_budget_fp32",
