@@ -35,7 +35,8 @@
 //     to ten, and then every line is exact;
 //  3. the labels are committed; the next window follows.
 // A line whose tape does not fit the pool ends its window; first in a window,
-// it is traced alone, in order.
+// it is traced alone, in order.  The windows after one that ended early are
+// shorter, and grow again while their tapes leave room.
 //
 // What bounds it: the tracing, the latency of the longest streamline's steps
 // (FP64 chains of a few hundred cycles and, at each voxel entered, a gather
@@ -423,16 +424,21 @@ inline uint32_t blocks_for(uint64_t n) { return (uint32_t)std::max<uint64_t>(1, 
 // Window of lines traced at once (bounds the tapes' scratch; line numbers in
 // the stamps have kLineBits bits).  The
 // environment variable MSCEER_LINE_WINDOW (8 .. 2^20) sets a smaller one,
-// which tests use to exercise many windows on small volumes.
+// which tests use to exercise many windows on small volumes; as
+// MSCEER_LINE_CHUNKS (1 .. 2^22) does for the pool's chunks and
+// MSCEER_LINE_ROUNDS (2 .. 512) for the rounds of a window.
 constexpr uint32_t kWindow = 1u << kLineBits;
+constexpr uint32_t kMaxChunks = 1u << 22;
 
-uint32_t line_window() {
-    if (const char* e = getenv("MSCEER_LINE_WINDOW")) {
+static uint32_t env_size(const char* name, uint32_t least, uint32_t most, uint32_t otherwise) {
+    if (const char* e = getenv(name)) {
         const long v = atol(e);
-        if (v >= 8 && v <= (long)kWindow) return (uint32_t)v;
+        if (v >= (long)least && v <= (long)most) return (uint32_t)v;
     }
-    return kWindow;
+    return otherwise;
 }
+
+uint32_t line_window() { return env_size("MSCEER_LINE_WINDOW", 8, kWindow, kWindow); }
 
 namespace {
 
@@ -483,7 +489,8 @@ int begin_lines(msceer_ctx* ctx, const LineFamily& f, uint32_t S, DevBuf& buf, h
     const uint32_t W = (uint32_t)std::min<uint64_t>(nslots, line_window());
     // tape pool: 128 slots per line of a window (volumes of noise and mixtures
     // record 20 to 40), at least 2^15 chunks
-    const uint32_t chunks = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(2ull * W, 1u << 15), 1u << 22);
+    const uint32_t chunks = env_size("MSCEER_LINE_CHUNKS", 1, kMaxChunks,
+                                     (uint32_t)std::min<uint64_t>(std::max<uint64_t>(2ull * W, 1u << 15), kMaxChunks));
 
     // scratch layout
     size_t tmp_bytes = 0;
@@ -561,10 +568,13 @@ int finish_lines(msceer_ctx* ctx, const LineJob& job, LineStats* out) {
         CHECK_HIP(hipStreamSynchronize(s));
         return MSCEER_OK;
     };
+    const uint32_t max_rounds = env_size("MSCEER_LINE_ROUNDS", 2, kMaxRounds, kMaxRounds);
+    const uint32_t group = std::min(8u, max_rounds);  // rounds between two read-backs
+    uint32_t span = W;  // lines of the next window
     uint64_t w0 = 0;
     while (w0 < nslots) {
         const uint32_t a0 = (uint32_t)w0;
-        const uint32_t w1 = (uint32_t)std::min<uint64_t>(nslots, w0 + W);
+        const uint32_t w1 = (uint32_t)std::min<uint64_t>(nslots, w0 + span);
         const uint32_t n = w1 - a0;
         if (ctx->line_tag <= kMaxRounds) {
             hipLaunchKernelGGL(line_fill_kernel, dim3(2048), dim3(kThreads), 0, s, a.stamp[0],
@@ -583,8 +593,7 @@ int finish_lines(msceer_ctx* ctx, const LineJob& job, LineStats* out) {
         uint32_t round = 0;
         uint32_t cut = 0;
         while (true) {
-            constexpr uint32_t kGroup = 8;
-            for (uint32_t j = 0; j < kGroup; j++, round++)
+            for (uint32_t j = 0; j < group; j++, round++)
                 hipLaunchKernelGGL(line_round_kernel, dim3(wave_blocks), dim3(kThreads), 0, s, a, a0, w1, round,
                                    ctx->line_tag--);
             hipLaunchKernelGGL(line_commit_kernel, dim3(wave_blocks), dim3(kThreads), 0, s, a, a0, w1, round - 1, true);
@@ -597,7 +606,7 @@ int finish_lines(msceer_ctx* ctx, const LineJob& job, LineStats* out) {
                 if (wc < w1) out->overflows++;
                 break;
             }
-            if (round + kGroup > kMaxRounds) {
+            if (round + group > max_rounds) {
                 // the lines before the lowest one still changing are exact
                 cut = h[kLcLowest + (round - 1) % 3];
                 hipLaunchKernelGGL(line_commit_kernel, dim3(wave_blocks), dim3(kThreads), 0, s, a, a0, cut, 0u, false);
@@ -607,6 +616,14 @@ int finish_lines(msceer_ctx* ctx, const LineJob& job, LineStats* out) {
             }
         }
         out->rounds += round;
+        // The lines from the cut on were traced for nothing: the next window
+        // takes no more than this one could resolve, or half of it (the pool
+        // is shared out as the lanes come, so an early line can be the one
+        // without room).  It doubles again where its tapes filled at most two
+        // fifths of the pool and its rounds ended early.
+        if (cut < w1) span = std::max(cut - a0, std::max(n / 2, 1u));
+        else if (5ull * h[kLcTop] <= 2ull * a.pool.chunks && round <= max_rounds / 4)
+            span = (uint32_t)std::min<uint64_t>(W, 2ull * span);
         if (cut == a0) {
             // the first line's tape did not fit the pool: it alone, in order
             hipLaunchKernelGGL(line_direct_kernel, dim3(1), dim3(64), 0, s, a, a0);

@@ -87,6 +87,60 @@ def test_small_windows_give_the_same_bytes(ctx, window):
     assert (g1 == g0).all()
 
 
+def _with_env(values, call):
+    os.environ.update({k: str(v) for k, v in values.items()})
+    try:
+        return call()
+    finally:
+        for k in values:
+            del os.environ[k]
+
+
+def _ridges():
+    # winding ridges along x: streamlines of many voxels, tapes of several chunks
+    z, y, x = np.meshgrid(*(np.arange(n, dtype=np.float64) for n in (28, 30, 260)), indexing="ij")
+    f = np.cos(2 * np.pi * (y + 5 * np.sin(x / 23)) / 14) * np.cos(2 * np.pi * (z + 4 * np.cos(x / 31)) / 13)
+    f += 0.3 * np.cos(2 * np.pi * x / 190 + 1) + 0.003 * synth.smoothed_noise(f.shape, 5, 2.0)
+    return f.astype(np.float32)
+
+
+@pytest.fixture(scope="module")
+def ridges(ctx):
+    """The volume, its oracle .grad and restriction, and how many streamlines one window traces."""
+    f = _ridges()
+    og, _, o_r, _ = oracle_lib.ondemand(f, 1, 1, 0, mode=1)
+    g, _, r, st = labels.ondemand(f, True, True, False, ctx=ctx)
+    assert (r == o_r).all() and (g == og).all()
+    assert st["line_windows"] == 2 and st["line_alone"] == 0  # one a family
+    return f, og, o_r, st["lines_asc"] + st["lines_dsc"]
+
+
+# 1: every tape of two chunks is traced alone; 40: windows of a few dozen lines
+# that end wherever the lanes left an early line without room; 1500: about a
+# fifteenth of what the lines ask for; 3 rounds (7 are needed): windows cut at the first line
+# still changing
+@pytest.mark.parametrize("values", [{"MSCEER_LINE_CHUNKS": 1}, {"MSCEER_LINE_CHUNKS": 40},
+                                    {"MSCEER_LINE_CHUNKS": 1500}, {"MSCEER_LINE_ROUNDS": 3}])
+def test_windows_cut_short_give_the_same_bytes(ctx, ridges, values):
+    f, og, o_r, once = ridges
+    _say(f"lines {values}")
+    g, _, r, st = _with_env(values, lambda: labels.ondemand(f, True, True, False, ctx=ctx))
+    traced = st["lines_asc"] + st["lines_dsc"]
+    _say(f"  traced {traced} for {once}: windows {st['line_windows']} overflows {st['line_overflows']} "
+         f"alone {st['line_alone']} cuts {st['line_cuts']}")
+    assert (r == o_r).all(), int((r != o_r).sum())
+    assert (g == og).all(), int((g != og).sum())
+    if "MSCEER_LINE_CHUNKS" in values:
+        assert st["line_overflows"] > 0
+        assert values["MSCEER_LINE_CHUNKS"] > 1 or st["line_alone"] > 0
+    else:
+        assert st["line_cuts"] > 0
+    # the lines of a window cut short are traced again: halving it down to the
+    # pool's size costs once more what one window does, and a window a little
+    # too long now and then the same again
+    assert traced <= 4 * once, (traced, once)
+
+
 def test_larger_volume_matches_fp64_oracle_and_repeats(ctx):
     f = synth.smoothed_noise((96, 112, 128), 303, 2.0)
     _say(f"lines {f.shape}")
