@@ -478,42 +478,67 @@ CellGeom cell_geom(const Dims& d) {
     return CellGeom{(int64_t)d.Mx, (int64_t)d.My, (int64_t)d.Mz, (int64_t)d.Mx * (int64_t)d.My};
 }
 
-// Seeds and the first window's tapes of a family with S saddles, on stream s
-// (the seeds by a scan, where the saddles are not listed, use the context's
-// counter: then s is its stream).  The tapes of the first window read no label.
-int begin_lines(msceer_ctx* ctx, const LineFamily& f, uint32_t S, DevBuf& buf, hipStream_t s, LineJob* job) {
+// Scratch of a family with S saddles: byte offsets of one buffer.
+struct LineScratch {
+    uint32_t W, chunks;  // lines of a window, chunks of the tape pool
+    size_t keys, sorted, slots, pool, wmask, active, head, ended, lctl, tmp, tmp_bytes, bytes;
+};
+
+int line_scratch(uint32_t S, hipStream_t s, LineScratch* l) {
+    const uint64_t nslots = 7ull * S;
+    l->W = (uint32_t)std::min<uint64_t>(nslots, line_window());
+    // tape pool: 128 slots per line of a window (volumes of noise and mixtures
+    // record 20 to 40), at least 2^15 chunks
+    l->chunks = env_size("MSCEER_LINE_CHUNKS", 1, kMaxChunks,
+                         (uint32_t)std::min<uint64_t>(std::max<uint64_t>(2ull * l->W, 1u << 15), kMaxChunks));
+    l->tmp_bytes = 0;
+    CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(nullptr, l->tmp_bytes, (const uint64_t*)nullptr,
+                                                          (uint64_t*)nullptr, (int)S, 0, 64, s));
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off += (bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    l->keys = take(8 * (size_t)S);
+    l->sorted = take(8 * (size_t)S);
+    l->slots = take(4 * nslots);
+    l->pool = take(8 * (size_t)kTapeChunk * l->chunks);
+    l->wmask = take(8 * (size_t)l->chunks);
+    l->active = take((size_t)l->W * 4);
+    l->head = take((size_t)l->W * 4);
+    l->ended = take((size_t)l->W * 4);
+    l->lctl = take(4 * kLcWords);
+    l->tmp = take(l->tmp_bytes);
+    l->bytes = off;
+    return MSCEER_OK;
+}
+
+// The context's first set of tapes; where there is no memory for it, a second
+// set kept by an earlier call makes room (nothing runs on it between calls).
+int ensure_lines(msceer_ctx* ctx, size_t bytes) {
+    if (ctx->lines.ensure(bytes) == hipSuccess) return MSCEER_OK;
+    (void)hipGetLastError();
+    ctx->lines2.release();
+    CHECK_HIP(ctx->lines.ensure(bytes));
+    return MSCEER_OK;
+}
+
+// Seeds and the first window's tapes of a family with S saddles, in buf (of
+// the scratch's bytes), on stream s (the seeds by a scan, where the saddles are
+// not listed, use the context's counter: then s is its stream).  The tapes of
+// the first window read no label.
+int begin_lines(msceer_ctx* ctx, const LineFamily& f, uint32_t S, const LineScratch& l, const DevBuf& buf, hipStream_t s,
+                LineJob* job) {
     const VGrid g = make_vgrid(f.d.X, f.d.Y, f.d.Z);
     const CellGeom m = cell_geom(f.d);
     uint32_t* count = ctl_dev(ctx) + kCtlCount;
     const uint64_t nslots = 7ull * S;
-    const uint32_t W = (uint32_t)std::min<uint64_t>(nslots, line_window());
-    // tape pool: 128 slots per line of a window (volumes of noise and mixtures
-    // record 20 to 40), at least 2^15 chunks
-    const uint32_t chunks = env_size("MSCEER_LINE_CHUNKS", 1, kMaxChunks,
-                                     (uint32_t)std::min<uint64_t>(std::max<uint64_t>(2ull * W, 1u << 15), kMaxChunks));
-
-    // scratch layout
-    size_t tmp_bytes = 0;
-    CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(nullptr, tmp_bytes, (const uint64_t*)nullptr,
-                                                          (uint64_t*)nullptr, (int)S, 0, 64, s));
-    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    size_t off = 0;
-    const size_t o_keys = off; off += al(8 * (size_t)S);
-    const size_t o_sorted = off; off += al(8 * (size_t)S);
-    const size_t o_slots = off; off += al(4 * nslots);
-    const size_t o_pool = off; off += al(8 * (size_t)kTapeChunk * chunks);
-    const size_t o_wmask = off; off += al(8 * (size_t)chunks);
-    const size_t o_active = off; off += al((size_t)W * 4);
-    const size_t o_head = off; off += al((size_t)W * 4);
-    const size_t o_ended = off; off += al((size_t)W * 4);
-    const size_t o_lctl = off; off += al(4 * kLcWords);
-    const size_t o_tmp = off; off += al(tmp_bytes);
-    CHECK_HIP(buf.ensure(off));
     char* base = buf.as<char>();
-    uint64_t* keys = (uint64_t*)(base + o_keys);
-    uint64_t* sorted = (uint64_t*)(base + o_sorted);
-    uint32_t* slots = (uint32_t*)(base + o_slots);
-    uint32_t* lctl = (uint32_t*)(base + o_lctl);
+    uint64_t* keys = (uint64_t*)(base + l.keys);
+    uint64_t* sorted = (uint64_t*)(base + l.sorted);
+    uint32_t* slots = (uint32_t*)(base + l.slots);
+    uint32_t* lctl = (uint32_t*)(base + l.lctl);
 
     if (f.saddles) {
         hipLaunchKernelGGL(line_saddle_list_kernel, dim3(std::min<uint32_t>(blocks_for(S), 1024)), dim3(kThreads), 0, s,
@@ -524,7 +549,8 @@ int begin_lines(msceer_ctx* ctx, const LineFamily& f, uint32_t S, DevBuf& buf, h
                            f.asc ? 2 : 1, f.asc ? 1 : 0, keys, count, S);
     }
     CHECK_HIP(hipGetLastError());
-    CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(base + o_tmp, tmp_bytes, keys, sorted, (int)S, 0, 64, s));
+    size_t tmp_bytes = l.tmp_bytes;
+    CHECK_HIP(hipcub::DeviceRadixSort::SortKeysDescending(base + l.tmp, tmp_bytes, keys, sorted, (int)S, 0, 64, s));
     hipLaunchKernelGGL(line_seeds_kernel, dim3(blocks_for(S)), dim3(kThreads), 0, s, f.grad, m, sorted, S,
                        f.asc ? 1 : 0, slots);
     CHECK_HIP(hipGetLastError());
@@ -540,11 +566,11 @@ int begin_lines(msceer_ctx* ctx, const LineFamily& f, uint32_t S, DevBuf& buf, h
     a.gthr = (double)f.gthr;
     a.ethr = (double)f.ethr;
     a.max_iters = f.max_iters;
-    a.pool = TapePool{(uint64_t*)(base + o_pool), chunks, lctl + kLcTop};
-    a.wmask = (uint64_t*)(base + o_wmask);
-    a.active = (uint32_t*)(base + o_active);
-    a.head = (uint32_t*)(base + o_head);
-    a.ended = (uint32_t*)(base + o_ended);
+    a.pool = TapePool{(uint64_t*)(base + l.pool), l.chunks, lctl + kLcTop};
+    a.wmask = (uint64_t*)(base + l.wmask);
+    a.active = (uint32_t*)(base + l.active);
+    a.head = (uint32_t*)(base + l.head);
+    a.ended = (uint32_t*)(base + l.ended);
     a.stamp[0] = ctx->line_stamps.as<uint32_t>();
     a.stamp[1] = a.stamp[0] + f.d.cells;
     a.ctl = lctl;
@@ -552,8 +578,8 @@ int begin_lines(msceer_ctx* ctx, const LineFamily& f, uint32_t S, DevBuf& buf, h
     CHECK_HIP(hipGetLastError());
 
     job->nslots = nslots;
-    job->W = W;
-    return enqueue_tapes(a, 0, (uint32_t)std::min<uint64_t>(nslots, W), s);
+    job->W = l.W;
+    return enqueue_tapes(a, 0, (uint32_t)std::min<uint64_t>(nslots, l.W), s);
 }
 
 // The rest of a family's lines, on the context's stream.
@@ -648,11 +674,13 @@ int finish_lines(msceer_ctx* ctx, const LineJob& job, LineStats* out) {
 // A second family's tapes are traced on another stream beside the first's: the
 // tape kernels last as long as their longest streamlines and leave most of the
 // chip idle (256^3 mixture: 2.4 and 3.0 ms one after the other).  The labels
-// are still resolved one family after the other.  Without memory for a second
-// set of tapes the families take turns with one.
+// are still resolved one family after the other.  The first family's set of
+// tapes is allocated first; without memory for a second one the families take
+// turns with it.
 int run_lines(msceer_ctx* ctx, const LineFamily* families, int n, LineStats* out) {
     hipStream_t s = ctx->stream;
     LineJob jobs[2];
+    LineScratch scratch[2] = {};
     uint32_t S[2] = {0, 0};
     bool begun[2] = {false, false};
     for (int i = 0; i < n; i++) {
@@ -664,7 +692,10 @@ int run_lines(msceer_ctx* ctx, const LineFamily* families, int n, LineStats* out
         if ((uint64_t)S[i] * 7 >= 0xFFFFFFFFull) return MSCEER_ETOOBIG;
         // two stamps per cell, refilled when they are new or the tags run out
         if (ctx->line_stamps.bytes < 8 * d.cells) ctx->line_tag = 0;
-        if (S[i]) CHECK_HIP(ctx->line_stamps.ensure(8 * d.cells));
+        if (S[i] == 0) continue;
+        CHECK_HIP(ctx->line_stamps.ensure(8 * d.cells));
+        rc = line_scratch(S[i], s, &scratch[i]);
+        if (rc) return rc;
     }
     // whatever happens, nothing is left running on the second stream
     struct Join {
@@ -675,15 +706,19 @@ int run_lines(msceer_ctx* ctx, const LineFamily* families, int n, LineStats* out
         }
     } join{ctx};
     if (n == 2 && S[0] && S[1] && families[1].saddles) {
+        const int rc = ensure_lines(ctx, scratch[0].bytes);
+        if (rc) return rc;
         if (!ctx->side) CHECK_HIP(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
         if (!ctx->side_ev) CHECK_HIP(hipEventCreateWithFlags(&ctx->side_ev, hipEventDisableTiming));
         CHECK_HIP(hipEventRecord(ctx->side_ev, s));
         CHECK_HIP(hipStreamWaitEvent(ctx->side, ctx->side_ev, 0));
         join.on = true;
-        begun[1] = begin_lines(ctx, families[1], S[1], ctx->lines2, ctx->side, &jobs[1]) == MSCEER_OK;
+        begun[1] = ctx->lines2.ensure(scratch[1].bytes) == hipSuccess &&
+                   begin_lines(ctx, families[1], S[1], scratch[1], ctx->lines2, ctx->side, &jobs[1]) == MSCEER_OK;
         if (!begun[1]) {
             (void)hipGetLastError();
             CHECK_HIP(hipStreamSynchronize(ctx->side));
+            ctx->lines2.release();
             jobs[1] = LineJob{};
         }
     }
@@ -694,7 +729,9 @@ int run_lines(msceer_ctx* ctx, const LineFamily* families, int n, LineStats* out
             CHECK_HIP(hipEventRecord(ctx->side_ev, ctx->side));
             CHECK_HIP(hipStreamWaitEvent(s, ctx->side_ev, 0));
         } else {
-            rc = begin_lines(ctx, families[i], S[i], ctx->lines, s, &jobs[i]);
+            rc = ensure_lines(ctx, scratch[i].bytes);
+            if (rc) return rc;
+            rc = begin_lines(ctx, families[i], S[i], scratch[i], ctx->lines, s, &jobs[i]);
             if (rc) return rc;
         }
         rc = finish_lines(ctx, jobs[i], &out[i]);

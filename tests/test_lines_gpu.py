@@ -12,6 +12,8 @@ arithmetic) the restriction labels differ on at most 0.1 % of the labelled
 cells.  Small speculation windows (MSCEER_LINE_WINDOW) give the same bytes as
 one window.
 """
+import ctypes
+import gc
 import os
 import sys
 
@@ -21,7 +23,7 @@ import pytest
 import gradcheck
 import oracle_lib
 from golden import lines_case_names, load_lines
-from msceer_amd import labels, native, synth
+from msceer_amd import hipmem, labels, native, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -139,6 +141,36 @@ def test_windows_cut_short_give_the_same_bytes(ctx, ridges, values):
     # pool's size costs once more what one window does, and a window a little
     # too long now and then the same again
     assert traced <= 4 * once, (traced, once)
+
+
+def test_families_take_turns_without_memory_for_two_sets(ridges):
+    f, og, o_r, _ = ridges
+    gib = 1 << 30
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    c = native.Context(0)
+    hog = []
+    try:
+        run = lambda: labels.ondemand(f, True, True, False, ctx=c)  # noqa: E731
+        run()  # every other buffer is there
+        hip = hipmem.hip()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        # a set of 2^22 chunks is 2.03 GiB: leave room for one
+        left = free.value - 3 * gib
+        _say(f"lines, {free.value / gib:.1f} GiB free, 3 left")
+        while left > 0:
+            hog.append(hipmem.DeviceBuffer(min(left, 16 * gib)))
+            left -= hog[-1].nbytes
+        for rep in range(3):
+            if rep == 2:  # room for both
+                hog.clear()
+                gc.collect()
+            g, _, r, st = _with_env({"MSCEER_LINE_CHUNKS": 1 << 22}, run)
+            assert (r == o_r).all() and (g == og).all()
+            assert st["line_alone"] == 0 and st["line_overflows"] == 0
+    finally:
+        hog.clear()
+        gc.collect()
+        c.close()
 
 
 def test_larger_volume_matches_fp64_oracle_and_repeats(ctx):
