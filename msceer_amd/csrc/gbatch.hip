@@ -50,6 +50,7 @@ enum GCtl : int {
 
 constexpr uint32_t kMaxItems = 0xFFFFFFFEu;  // cells of a group
 constexpr int kDefaultRounds = 12;           // sweeps in a first capture
+constexpr int kMaxRounds = 64;               // sweeps in any capture
 constexpr int kMaxPlans = 4;
 
 __global__ void times_init_kernel(unsigned long long* t, uint32_t n) {
@@ -458,7 +459,7 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
         it->key = key;
         // sweeps in a first capture (later captures take what the calls
         // needed; 0: none, all run after the replay)
-        if (const char* e = getenv("MSCEER_BATCH_ROUNDS")) it->rounds = std::max(0, std::min(64, atoi(e)));
+        if (const char* e = getenv("MSCEER_BATCH_ROUNDS")) it->rounds = std::max(0, std::min(kMaxRounds, atoi(e)));
         int rc = upload_tables(ctx, s, vols, g, dev, *it);
         if (rc) return rc;
         while ((int)s.plans.size() > kMaxPlans) {
@@ -525,10 +526,14 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
         st.eager_rounds += k - p.rounds;
         CHECK_HIP(launch_ldir_finish_group(group_batch(s, p, timing), (uint32_t)k, s.ctl.as<uint32_t>() + kGActive,
                                            ctx->stream));
-        // the next capture of this plan takes the sweeps this call needed
-        if (p.exec) (void)hipGraphExecDestroy(p.exec);
-        p.exec = nullptr;
-        p.rounds = std::min(k, 64);
+        // the next capture of this plan takes the sweeps this call needed, as
+        // far as a capture's limit goes
+        const int rounds = std::min(k, kMaxRounds);
+        if (rounds != p.rounds) {
+            if (p.exec) (void)hipGraphExecDestroy(p.exec);
+            p.exec = nullptr;
+            p.rounds = rounds;
+        }
     }
     CHECK_HIP(hipEventRecord(s.t1, ctx->stream));
     if (!dev) {

@@ -173,6 +173,30 @@ def test_graph_replays_with_device_buffers(ctx, c4):
         assert (g1 == other_ref).all()
 
 
+def _ridge(nz, seed):
+    """A ridge along z between two valleys: the flood of its edges starts at
+    one end and takes a sweep per tile of 16 layers."""
+    z, y, x = np.meshgrid(np.arange(nz, dtype=np.float64), np.arange(3), np.arange(33), indexing="ij")
+    f = -np.cos(2 * np.pi * (x - 16) / 32) + 0.01 * z + 1e-4 * synth.Stream(seed).uniform(x.size).reshape(x.shape)
+    f[:, 1] -= 0.5
+    return f.astype(np.float32)
+
+
+def test_group_beyond_the_captured_sweeps_keeps_its_graph(ctx):
+    """More sweeps than any graph holds: the rest runs after each replay, and
+    the graph is captured again only once, for the limit."""
+    f = _ridge(16 * 90, 5)
+    ref = oracle_lib.steepest_grad(f)
+    captures = []
+    for rep in range(4):
+        grads, _, st = batch.run_batch_grad([f], ctx=ctx)
+        _say(f"ridge call {rep}: sweeps {st.rounds} eager {st.eager_rounds} captures {st.captures}")
+        assert (grads[0] == ref).all(), int((grads[0] != ref).sum())
+        assert st.eager_rounds > 0
+        captures.append(st.captures)
+    assert captures == [1, 1, 0, 0], captures
+
+
 _FEW_ROUNDS = """
 import numpy as np
 import oracle_lib
