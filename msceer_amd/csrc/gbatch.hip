@@ -79,6 +79,12 @@ struct GroupLayout {
     size_t vals_bytes = 0, grad_bytes = 0;
 };
 
+// What calls measured of a group's shapes; outlives its plans.
+struct GroupTune {
+    LaunchTune launch;
+    int rounds = -1;  // most sweeps a capture was enlarged to; -1: none was
+};
+
 struct GroupPlan {
     std::string key;  // shapes, buffers and launch parameters of the capture
     DevBuf tables;    // GVol table and unit tables
@@ -97,7 +103,7 @@ struct BatchState {
     DevBuf vals, grad, ldir, lists, ctl, times;
     uint64_t generation = 0;  // bumped whenever a shared buffer moves (captured graphs then stale)
     std::list<GroupPlan> plans;  // most recent first
-    std::map<std::string, LaunchTune> tunes;
+    std::map<std::string, GroupTune> tunes;
     msceer_batch_stats last{};
     uint32_t* h_ctl = nullptr;
     int cus = 0;
@@ -442,7 +448,8 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
         tune_suffix = "|m" + std::to_string(ctx->tuning->mode);
     }
     if (const char* e = getenv("MSCEER_BATCH_LAUNCH")) tune_suffix += std::string("|") + e;
-    std::string key = shapes_key(vols, g) + tune_suffix;
+    const std::string tune_key = shapes_key(vols, g) + tune_suffix;
+    std::string key = tune_key;
     char buf[160];
     snprintf(buf, sizeof buf, "|gen%llu|dev%d|t%d", (unsigned long long)s.generation, dev ? 1 : 0, timing ? 1 : 0);
     key += buf;
@@ -457,9 +464,13 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
         s.plans.emplace_front();
         it = s.plans.begin();
         it->key = key;
-        // sweeps in a first capture (later captures take what the calls
-        // needed; 0: none, all run after the replay)
-        if (const char* e = getenv("MSCEER_BATCH_ROUNDS")) it->rounds = std::max(0, std::min(kMaxRounds, atoi(e)));
+        // sweeps in a first capture (later captures, of other plans of these
+        // shapes too, take what the calls needed; 0: none, all run after the
+        // replay)
+        const auto t = s.tunes.find(tune_key);
+        if (t != s.tunes.end() && t->second.rounds >= 0) it->rounds = t->second.rounds;
+        else if (const char* e = getenv("MSCEER_BATCH_ROUNDS"))
+            it->rounds = std::max(0, std::min(kMaxRounds, atoi(e)));
         int rc = upload_tables(ctx, s, vols, g, dev, *it);
         if (rc) return rc;
         while ((int)s.plans.size() > kMaxPlans) {
@@ -481,14 +492,13 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
         }
     }
     if (!p.tuned) {
-        const std::string skey = shapes_key(vols, g) + tune_suffix;
-        auto t = s.tunes.find(skey);
+        const auto t = s.tunes.find(tune_key);
         if (t != s.tunes.end()) {
-            p.tune = t->second;
+            p.tune = t->second.launch;
         } else {
             int rc = tune_group(ctx, s, p, caps, &p.tune);
             if (rc) return rc;
-            s.tunes[skey] = p.tune;
+            s.tunes[tune_key].launch = p.tune;
         }
         p.tuned = true;
     }
@@ -533,6 +543,8 @@ int run_group(msceer_ctx* ctx, BatchState& s, msceer_volume* vols, GroupLayout& 
             if (p.exec) (void)hipGraphExecDestroy(p.exec);
             p.exec = nullptr;
             p.rounds = rounds;
+            GroupTune& t = s.tunes[tune_key];
+            t.rounds = std::max(t.rounds, rounds);
         }
     }
     CHECK_HIP(hipEventRecord(s.t1, ctx->stream));

@@ -197,6 +197,22 @@ def test_group_beyond_the_captured_sweeps_keeps_its_graph(ctx):
     assert captures == [1, 1, 0, 0], captures
 
 
+def test_more_groups_than_kept_plans_remember_their_sweeps(ctx):
+    """Six groups of one volume each, more than the plans a context keeps:
+    every call captures them again, with the sweeps the call before needed."""
+    fs = [_ridge(16 * 20 + i, 6 + i) for i in range(6)]
+    refs = [oracle_lib.steepest_grad(f) for f in fs]
+    eager = []
+    for rep in range(3):
+        grads, _, st = batch.run_batch_grad(fs, max_group_verts=1, ctx=ctx)
+        _say(f"groups call {rep}: {st.groups} groups, eager {st.eager_rounds} captures {st.captures}")
+        for g, ref in zip(grads, refs):
+            assert (g == ref).all()
+        assert st.groups == 6 and st.captures == 6
+        eager.append(st.eager_rounds)
+    assert eager[0] > 0 and eager[1:] == [0, 0], eager
+
+
 _FEW_ROUNDS = """
 import numpy as np
 import oracle_lib
