@@ -721,13 +721,11 @@ pass2_kernel(VGrid g, LabelBuffers b, WorkQueue q) {
 // no unclaimed reserved slot for kLeaveTicks: every item queued later is
 // queued by a wave still running, which drains it before it leaves itself.
 // Waves thus do not wait through the tail of a few long dependent streamlines,
-// and kernels of other streams get their compute units.  q.busy counts the
-// waves that hold anything but traces ahead: once it is zero and no slot is
-// left, nothing can want a trace ahead any more, so those are given up and the
-// waves leave at once.  (256^3 noise: the last re-integration ended at 10.9 ms,
-// the last trace ahead, wanted by none, at 14.5: 13.1 -> 11.5 ms for the pass.
-// The count may be read as zero between a wave's claim and its counting itself;
-// that only gives up traces ahead too early.)
+// and kernels of other streams get their compute units.  Once no wave holds
+// anything but traces ahead and no slot is left (queue_drained), nothing can
+// want a trace ahead any more, so those are given up and the waves leave at
+// once.  (256^3 mixture: the last re-integration ended at 10.9 ms, the last
+// trace ahead, wanted by none, at 14.5: 13.1 -> 11.5 ms for the pass.)
 constexpr uint32_t kRing = 256;                // per-wave ring (a power of two)
 constexpr uint32_t kRingKeep = 192;            // children stay in the ring up to this fill
 constexpr uint32_t kChunk = 64;                // pass-2 items claimed at a time
@@ -744,10 +742,6 @@ __global__ void pass3_prepare_kernel(WorkQueue q) {
         *q.chunk_head = 0u;
         *q.busy = 0u;
     }
-}
-
-__device__ __forceinline__ uint32_t load_agent(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Tracing ahead.  The tail of the pass is a chain of long streamlines run
@@ -873,7 +867,11 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
         if (want && rhead == rtail && chunks) {
             const int leader = __ffsll((unsigned long long)want) - 1;
             uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(q.chunk_head, kChunk);
+            if (lane == leader) {
+                if (!counted) queue_enter(q);
+                base = atomicAdd(q.chunk_head, kChunk);
+            }
+            counted = true;
             base = __shfl(base, leader);
             if (base >= first) {
                 chunks = false;
@@ -899,22 +897,14 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
         if (want && rhead == rtail && !chunks) {
             const int leader = __ffsll((unsigned long long)want) - 1;
             uint32_t base = 0, n = 0, on = 0;
+            bool in = counted;
             if (lane == leader) {
-                uint32_t h = load_agent(q.head);
-                uint32_t t = load_agent(q.tail);
                 on = load_agent(q.ahead_on);
-                t = t < q.capacity ? t : q.capacity;
-                if (h < t) {
-                    const uint32_t nw = (uint32_t)__popcll(want), k = t - h < nw ? t - h : nw;
-                    if (__hip_atomic_compare_exchange_strong(q.head, &h, h + k, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT)) {
-                        base = h;
-                        n = k;
-                    }
-                }
+                n = queue_claim(q, (uint32_t)__popcll(want), in, &base);
             }
             base = __shfl(base, leader);
             n = __shfl(n, leader);
+            counted = __shfl((int)in, leader) != 0;
             ahead_seen = ahead_seen || __shfl(on, leader) != 0u;
             const uint32_t rank = (uint32_t)__popcll(want & below);
             if (need && rank < n) {
@@ -930,7 +920,7 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
             }
         }
         // fin: re-integration of v done, ending at vertex `end`
-        bool fin = false, chain = false;
+        bool fin = false, chain = false, wanted = false;
         int64_t end = 0;
         if (item != kEmptySlot) {
             const bool ahead_item = (item & kSpecItem) != 0u;
@@ -945,6 +935,7 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
                     const int32_t sp = seen == kSpecNone ? kSpecNone : atomicCAS(&spec[v], kSpecBusy, kSpecWanted);
                     if (sp == kSpecBusy) {
                         trace = false;  // the lane tracing v ahead finishes it
+                        wanted = true;
                     } else if (sp >= 0) {
                         trace = false;  // traced ahead
                         fin = chain = true;
@@ -965,6 +956,16 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
                 }
             }
         }
+        const uint64_t wants = __ballot(wanted);
+        if (wants && lane == 0) atomicAdd(q.busy, (uint32_t)__popcll(wants));
+        // traces ahead that turned out to be wanted are this wave's work now
+        auto take_over = [&](bool mine) {
+            const uint64_t m = __ballot(mine);
+            if (!m) return;
+            bool in = counted;
+            if (lane == 0) queue_takeover(q, (uint32_t)__popcll(m), in);
+            counted = true;
+        };
         // no streamline but traces ahead, while no wave holds other work and no
         // item is queued: nothing can reach their vertices any more
         const bool holds = __any((active && !speculative) || fin || claimed) || rhead != rtail || chunks;
@@ -974,16 +975,14 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
         }
         bool done = false;
         if (!holds) {
-            if (lane == 0) {
-                const uint32_t t = load_agent(q.tail);
-                done = load_agent(q.busy) == 0u && load_agent(q.head) >= (t < q.capacity ? t : q.capacity);
-            }
+            if (lane == 0) done = queue_drained(q);
             done = __shfl((int)done, 0) != 0;
             if (done && active) {
-                // (a vertex reached meanwhile, after all, is finished here)
+                // (never wanted: such a trace would be counted)
                 active = atomicExch(&spec[v], kSpecDropped) == kSpecWanted;
                 speculative = false;
             }
+            if (done) take_over(active);
             if (done && !__any(active)) break;
         }
         if (!__any(active || fin)) {
@@ -1030,6 +1029,7 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
         // 19.8 -> 14.8 ms; a half and an eighth measured 15.6)
         const int burst = __any(fin) ? 0 : kBurst;
         const int enough = (__popcll(__ballot(active)) + kBurstShare - 1) / kBurstShare;
+        bool taken = false;
         if (active) {
             int64_t next = 0;
             int ev = kNone;
@@ -1082,12 +1082,14 @@ pass3_kernel(GradSrc<float> srcf, GradSrc<double> srcd, VGrid g, LabelBuffers b,
                 // a vertex traced ahead is finished here only if it was reached meanwhile
                 fin = !speculative || atomicExch(&spec[v], (int32_t)next | (esc ? kSpecFP64 : 0) |
                                                                (ob ? kSpecOver : 0)) == kSpecWanted;
+                taken = speculative && fin;
                 if (fin) {
                     escalated += esc ? 1u : 0u;
                     over += ob ? 1u : 0u;
                 }
             }
         }
+        take_over(taken);
         uint32_t kids[6];
         int nk = 0;
         bool spawn = false;

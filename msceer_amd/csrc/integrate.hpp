@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "work_queue.hpp"
+
 namespace msceer {
 
 struct MList;
@@ -87,19 +89,6 @@ hipError_t launch_pass1_finish(const VGrid& g, const LabelBuffers& b, int stride
                                hipStream_t s);
 // Pass 2: every ASSIGNED vertex with a differently labelled All6 neighbour
 // (or flagged for re-tracing) goes to `out`.
-// Re-integration work queue: `items` (capacity entries, 0xFFFFFFFF until
-// written) and its claim/reserve counters.
-struct WorkQueue {
-    uint32_t* items;
-    uint32_t capacity;
-    uint32_t* head;         // next slot of the items queued during pass 3
-    uint32_t* tail;         // slots reserved
-    uint32_t* overflow;
-    uint32_t* ahead_on;     // set once pass 3 traces vertices ahead
-    uint32_t* chunk_head;   // next chunk of the items pass 2 queued
-    uint32_t* first_count;  // items pass 2 queued
-    uint32_t* busy;         // pass-3 waves that hold anything but traces ahead
-};
 hipError_t launch_pass2(const VGrid& g, const LabelBuffers& b, const WorkQueue& q, hipStream_t s);
 // Certain regions by chains and a flood (certain.hip; seeds labelled
 // beforehand, -1 elsewhere): chain labels and bad vertices (parent: one int32
