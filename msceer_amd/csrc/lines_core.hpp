@@ -1,10 +1,8 @@
 // Device code of the accurate 1-manifolds (lines.hip): cell geometry, the
-// saddles' seed search, one digitizing streamline and the label policies of
-// its speculative, replayed and in-order traces.  Kept in a header so that a
+// saddles' seed search, one digitizing streamline, its trace in order against
+// the labels and its tape, and a tape's evaluation.  Kept in a header so that a
 // host build of the same source can be checked against the CPU oracle; the
-// includer provides what tracer.hpp needs plus the HIP atomics used here
-// (atomicMin, atomicAdd, __hip_atomic_load / _store /
-// _compare_exchange_strong).
+// includer provides what tracer.hpp needs plus atomicAdd.
 #pragma once
 
 #include "tracer.hpp"
@@ -15,7 +13,7 @@ namespace msceer {
 namespace {
 
 constexpr uint32_t kNoLine = 0xFFFFFFFFu;
-constexpr int kAbort = 100;  // trace event: the footprint rule stopped it
+constexpr int kAbort = 100;  // trace event: the label policy stopped it (a tape beyond the pool)
 
 struct CellGeom {
     int64_t Mx, My, Mz, sxy;
@@ -202,8 +200,10 @@ __device__ inline void saddle_seeds(const uint8_t* grad, const CellGeom& m, uint
 // ---- one streamline ----------------------------------------------------------
 
 // Label policies of a trace: test(c) -- does cell c carry the target (a
-// checker or digitizing test); write(c) -- give it the target; ok() -- false
-// once the trace must stop for a footprint rule.
+// checker or digitizing test); write(c) -- give it the target; stop_here() --
+// a test at a step inside a voxel follows, where a stop digitizes no further
+// than that step; leave() -- one at the step out of it; ok() -- false once the
+// trace must stop for the policy's own reasons.
 
 // Alone and in order: the restriction labels themselves.
 struct DirectLabels {
@@ -392,204 +392,6 @@ __device__ inline uint64_t tape_chunk(TapeState& s, uint32_t n, uint64_t test, u
     }
     return w;
 }
-
-// ---- the window algorithm's label policies -----------------------------------
-//
-// A second realisation of the same order on the same traces (speculation with
-// footprints, replay of the components that interact), run by the host
-// emulation, which checks the tracing and digitizing code with it.
-
-// Footprints: every cell a speculative trace tests or labels, appended (with
-// repeats) to chunks of a shared pool, one chain per line (and a second chain
-// of the cells it labelled): chunk = the index of the next chunk (or kNoLine)
-// and kChunk - 1 cells, the last chunk of a footprint ended by kNoLine.
-constexpr uint32_t kChunk = 32;
-
-struct Pool {
-    uint32_t* cells;     // capacity words
-    uint32_t capacity;   // a multiple of kChunk
-    uint32_t* top;       // next free word
-};
-
-// Speculation: committed labels plus the line's own labels, known exactly
-// (own[c]: the last line of the window that labelled c; its second chain
-// where another line overwrote that mark).  Labelled cells claim wstamp (the
-// lowest line of the window labelling them); the first claim of a cell
-// appends it to the window's list of labelled cells.
-struct SpecLabels {
-    const int8_t* restr;
-    int8_t target;
-    uint32_t* wstamp;
-    uint32_t* pstamp;
-    uint32_t* own;
-    uint32_t line;
-    Pool pool;
-    uint32_t* touched;     // cells labelled (or possibly labelled) in the window
-    uint32_t* ntouched;
-    struct Chain {
-        uint32_t head = kNoLine, chunk = kNoLine, fill = 0;
-    } all, wrote, maybe;   // the footprint; the cells labelled; the cells a stop could label
-    uint32_t last[6];      // the cells of the last stop_here, not recorded again
-    int nlast = -1;
-    bool over = false;
-    __device__ void append(Chain& ch, uint32_t c) {
-        if (over) return;
-        if (ch.chunk == kNoLine || ch.fill == kChunk - 1) {
-            const uint32_t at = atomicAdd(pool.top, kChunk);
-            if (at + kChunk > pool.capacity) {
-                over = true;
-                return;
-            }
-            pool.cells[at] = kNoLine;
-            if (ch.chunk == kNoLine) ch.head = at;
-            else pool.cells[ch.chunk] = at;
-            ch.chunk = at;
-            ch.fill = 0;
-        }
-        pool.cells[ch.chunk + 1 + ch.fill] = c;
-        ch.fill++;
-    }
-    __device__ void claim(uint32_t* stamp, uint32_t c) {
-        if (atomicMin(&stamp[c], line) == kNoLine) {
-            const uint32_t at = atomicAdd(ntouched, 1u);
-            if (at < pool.capacity) touched[at] = c;  // (never more cells than pool words)
-        }
-    }
-    // Did this line label c?  own[c] says yes unless another line of the
-    // window labelled c since; wstamp[c] > line says no (a line's own claim
-    // keeps wstamp at or below it); otherwise the line's labels are searched.
-    __device__ bool mine(uint32_t c) const {
-        if (own[c] == line) return true;
-        if (wstamp[c] > line) return false;
-        for (uint32_t ch = wrote.head; ch != kNoLine; ch = pool.cells[ch]) {
-            const uint32_t n = ch == wrote.chunk ? wrote.fill : kChunk - 1;
-            for (uint32_t j = 0; j < n; j++)
-                if (pool.cells[ch + 1 + j] == c) return true;
-        }
-        return false;
-    }
-    __device__ bool test(uint32_t c) {
-        append(all, c);
-        return restr[c] == target || mine(c);
-    }
-    __device__ void write(uint32_t c) {
-        append(all, c);
-        append(wrote, c);
-        if (over) return;  // the window ends before this line
-        own[c] = line;
-        claim(wstamp, c);
-    }
-    // Cells a stop at this point would label (its digitization start ->
-    // here): footprint, and claimed in pstamp, so that a replay stopping here
-    // stays within what the speculation saw.
-    __device__ void stop_here(const CellGeom& m, const V3<double>& a, const V3<double>& b, bool asc) {
-        uint32_t cells[6];
-        const int n = digitize_cells(m, a, b, asc, cells);
-        bool same = n == nlast;
-        for (int k = 0; same && k < n; k++) same = cells[k] == last[k];
-        if (same) return;
-        nlast = n;
-        for (int k = 0; k < n; k++) {
-            last[k] = cells[k];
-            append(all, cells[k]);
-            append(maybe, cells[k]);
-            if (over) return;
-            claim(pstamp, cells[k]);
-        }
-    }
-    __device__ void leave() {}
-    // End marks of the last chunks.
-    __device__ void finish() {
-        if (over) return;
-        if (all.chunk != kNoLine && all.fill < kChunk - 1) pool.cells[all.chunk + 1 + all.fill] = kNoLine;
-        if (wrote.chunk != kNoLine && wrote.fill < kChunk - 1) pool.cells[wrote.chunk + 1 + wrote.fill] = kNoLine;
-        if (maybe.chunk != kNoLine && maybe.fill < kChunk - 1) pool.cells[maybe.chunk + 1 + maybe.fill] = kNoLine;
-    }
-    __device__ bool ok() const { return !over; }
-};
-
-// Union-find over the lines of a window (relative indices).
-__device__ __forceinline__ uint32_t lf_parent(uint32_t* p, uint32_t x) {
-    return __hip_atomic_load(&p[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint32_t lf_find(uint32_t* p, uint32_t x) {
-    uint32_t q = lf_parent(p, x);
-    while (q != x) {
-        const uint32_t gq = lf_parent(p, q);
-        if (gq != q) __hip_atomic_store(&p[x], gq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        x = q;
-        q = gq;
-    }
-    return x;
-}
-// Hook the later root under the earlier one, so a component's root is its
-// first line.
-__device__ void lf_union(uint32_t* p, uint32_t a, uint32_t b) {
-    while (true) {
-        a = lf_find(p, a);
-        b = lf_find(p, b);
-        if (a == b) return;
-        if (a > b) { const uint32_t t = a; a = b; b = t; }
-        uint32_t expected = b;
-        if (__hip_atomic_compare_exchange_strong(&p[b], &expected, a, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT))
-            return;
-    }
-}
-
-
-// Replay of one component, its lines in order: committed labels plus those
-// its earlier lines gave (lstamp).  A cell that lines of the window labelled,
-// or could label by stopping, in speculation belongs to their component; a
-// replayed line may test it only in its own component, and may label only
-// cells it labelled, or could label, itself in speculation.  Anything else
-// means the line went beyond what the speculation saw, and the window is cut
-// before it.
-struct ReplayLabels {
-    const int8_t* restr;
-    int8_t target;
-    const uint32_t* wstamp;
-    const uint32_t* pstamp;
-    uint32_t* lstamp;
-    const uint32_t* own;
-    const uint32_t* pool;
-    uint32_t whead, mhead;  // chains of the cells this line labelled / a stop could label, in speculation
-    uint32_t* parent;
-    uint32_t w0, wc, root, line;
-    uint32_t* why;          // failure counters: [0] tests, [1] labels
-    bool bad;
-    __device__ static bool in_chain(const uint32_t* pool, uint32_t head, uint32_t c) {
-        for (uint32_t ch = head; ch != kNoLine; ch = pool[ch])
-            for (uint32_t j = 1; j < kChunk; j++) {
-                const uint32_t x = pool[ch + j];
-                if (x == kNoLine) break;
-                if (x == c) return true;
-            }
-        return false;
-    }
-    __device__ bool foreign(uint32_t w) const { return w >= w0 && w < wc && lf_find(parent, w - w0) != root; }
-    __device__ bool test(uint32_t c) {
-        if (foreign(wstamp[c]) || foreign(pstamp[c])) {
-            if (!bad) atomicAdd(&why[0], 1u);
-            bad = true;
-            return false;
-        }
-        return restr[c] == target || lstamp[c] != kNoLine;
-    }
-    __device__ void write(uint32_t c) {
-        const bool seen = own[c] == line || (wstamp[c] <= line && in_chain(pool, whead, c)) ||
-                          (pstamp[c] <= line && in_chain(pool, mhead, c));
-        if (!seen) {
-            if (!bad) atomicAdd(&why[1], 1u);
-            bad = true;
-            return;
-        }
-        lstamp[c] = line;
-    }
-    __device__ bool ok() const { return !bad; }
-    __device__ void stop_here(const CellGeom&, const V3<double>&, const V3<double>&, bool) {}
-    __device__ void leave() {}
-};
 
 // Label the cells of digitize_cells in order; stop at the first one that
 // already carries the target.

@@ -257,16 +257,6 @@ __device__ __forceinline__ int tracer_iterate(const GradSrc<T>& src, const VGrid
     return kNone;
 }
 
-// Enter the voxel of a position changed outside a step; returns the vertex nearest to it.
-template <typename T, class C>
-__device__ __forceinline__ int64_t tracer_reenter(const GradSrc<T>& src, const VGrid& g, Tracer<T, C>& t) {
-    int x, y, z;
-    const int64_t next = nearest_xyz(g, t.cur, t.near, x, y, z);
-    tracer_load(src, g, t, x, y, z);
-    tracer_begin(t);
-    return next;
-}
-
 // Start a streamline at vertex (x, y, z).
 template <typename T, class C>
 __device__ __forceinline__ void tracer_start(const GradSrc<T>& src, const VGrid& g, Tracer<T, C>& t, int x, int y,
@@ -438,6 +428,7 @@ __device__ __forceinline__ int tracer_iterate(const GradSrc<float>& src, const V
     return kNone;
 }
 
+// Enter the voxel of the position after kOutOfVoxel; returns the vertex nearest to it.
 template <class C>
 __device__ __forceinline__ int64_t tracer_reenter(const GradSrc<float>& src, const VGrid& g, TracerL<C>& t) {
     int x, y, z;

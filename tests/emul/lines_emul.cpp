@@ -1,11 +1,12 @@
-// Host emulation of the accurate 1-manifold kernels (test infrastructure):
-// the same lines_core.hpp the gfx950 kernels run, driven window by window
-// on the CPU -- every speculative trace, the union-find over footprints, the
-// in-order replay of each component, the commit of the lines before a cut --
-// with the lanes of a launch taken one after another in a chosen order (the
-// order only decides which line's mark a shared cell keeps, which the
-// algorithm must not depend on).  Its restriction labels are compared with
-// the oracle's one-thread saddle loops.
+// A second realisation of the 1-manifolds' order on the host (test
+// infrastructure): the tracing and digitizing code that the gfx950 kernels run
+// (lines_core.hpp), with the label policies of replay_policies.hpp instead of
+// tapes, driven window by window on the CPU -- every speculative trace, the
+// union-find over footprints, the in-order replay of each component, the commit
+// of the lines before a cut -- with the lanes taken one after another in a
+// chosen order (the order only decides which line's mark a shared cell keeps,
+// which the algorithm must not depend on).  Its restriction labels are compared
+// with the oracle's one-thread saddle loops.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -40,6 +41,7 @@ struct VGrid {
 }  // namespace msceer
 
 #include "lines_core.hpp"
+#include "replay_policies.hpp"
 
 using namespace msceer;
 

@@ -1,8 +1,10 @@
-"""The GPU's 1-manifold algorithm (speculation over windows, union-find over
-footprints, in-order replay of components, commit before a cut), built for
-the host from the kernels' own header and checked against the oracle's
-one-thread saddle loops in FP64: equal restriction labels for every lane
-order of a launch and for windows small enough to cut often."""
+"""The streamlines that the GPU's 1-manifold kernels trace and digitize, built
+for the host from the kernels' own header, with their order realised another
+way than on the GPU (speculation over windows, union-find over footprints,
+in-order replay of components, commit before a cut), against the oracle's
+one-thread saddle loops in FP64: equal restriction labels for every lane order
+and for windows small enough to cut often.  (The GPU's own tapes and rounds are
+checked in test_tapes_emul.py.)"""
 import numpy as np
 import pytest
 

@@ -49,11 +49,6 @@ int gpu_trace(const msceer::GradSrc<double>& src, const msceer::VGrid& g, const 
         int64_t next = 0;
         bool moved = false;
         int ev = tracer_iterate(src, g, dest, stop, dir, gthr, ethr, t, next, moved);
-        if (ev == kOutOfVoxel) {
-            next = tracer_reenter(src, g, t);
-            moved = true;
-            ev = kNone;
-        }
         if (moved) path.push_back(next);
         if (ev == kNone) continue;
         if (ev != kHitPreassigned) next = nearest(g, t.cur, t.near);
