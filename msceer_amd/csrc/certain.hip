@@ -64,14 +64,16 @@ __device__ __forceinline__ uint64_t row_word(const Geo& g, int w, int y, int z) 
 // of 64): parent[v] = v where the chain ends, else the vertex where v's chain
 // leaves the tile, or its end inside.
 constexpr int kTX = 66, kTY = 6, kTZ = 6;
+constexpr uint32_t kMaxTiles = 1u << 20;  // of a launch (a grid holds fewer than 2^32 threads), from `first` on
 __global__ void __launch_bounds__(kThreads)
 chain_tile_kernel(const float* __restrict__ f, Geo g, const uint8_t* __restrict__ seedmask, int32_t* __restrict__ parent,
-                  Planes p, uint64_t flip) {
+                  Planes p, uint64_t flip, uint32_t first) {
     __shared__ float tile[kTX * kTY * kTZ];
     __shared__ uint16_t next[1024];   // in-tile successor, or itself
     __shared__ int32_t leave[1024];   // vertex the chain goes on at from there
-    const int w = (int)(blockIdx.x % (uint32_t)g.words);
-    const int q = (int)(blockIdx.x / (uint32_t)g.words);
+    const uint32_t tile_id = first + blockIdx.x;
+    const int w = (int)(tile_id % (uint32_t)g.words);
+    const int q = (int)(tile_id / (uint32_t)g.words);
     const int nby = (g.Y + 3) / 4;
     const int x0 = w * 64, y0 = (q % nby) * 4, z0 = (q / nby) * 4;
     for (int i = threadIdx.x; i < kTX * kTY * kTZ; i += kThreads) {
@@ -326,9 +328,10 @@ hipError_t launch_certain_chains(const VGrid& g, const float* values, const uint
                                  int32_t* parent, int32_t* label, void* scratch, hipStream_t s) {
     const Layout l = layout(g);
     const Planes p = planes(l, scratch);
-    const uint64_t tiles = (uint64_t)l.g.words * ((g.Y + 3) / 4) * ((g.Z + 3) / 4);
-    hipLaunchKernelGGL(chain_tile_kernel, dim3((uint32_t)tiles), dim3(kThreads), 0, s, values, l.g, seedmask, parent, p,
-                       desc ? ~0ull : 0ull);
+    const uint32_t tiles = (uint32_t)l.g.words * (uint32_t)((g.Y + 3) / 4) * (uint32_t)((g.Z + 3) / 4);
+    for (uint32_t k = 0; k < tiles; k += kMaxTiles)
+        hipLaunchKernelGGL(chain_tile_kernel, dim3(std::min(tiles - k, kMaxTiles)), dim3(kThreads), 0, s, values, l.g,
+                           seedmask, parent, p, desc ? ~0ull : 0ull, k);
     const uint32_t blocks = (uint32_t)std::min<int64_t>((g.verts() + kThreads - 1) / kThreads, 32768);
     hipLaunchKernelGGL(chain_label_kernel, dim3(blocks), dim3(kThreads), 0, s, l.g, parent, label);
     hipLaunchKernelGGL(bad_kernel, dim3(row_blocks(l.rows)), dim3(kThreads), 0, s, l.g, label, p);

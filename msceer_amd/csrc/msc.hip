@@ -215,12 +215,14 @@ msc_link_kernel(const uint8_t* __restrict__ grad, MscGeom g, const uint32_t* __r
 // its path leaves the tile, or to its root.  (A closed path, which no gradient
 // has, is left as it is; the jumps report it.)
 constexpr int kTile = 1024;
+constexpr uint32_t kMaxTiles = 1u << 20;  // of a launch (a grid holds fewer than 2^32 threads), from `first` on
 __global__ void __launch_bounds__(kThreads)
-msc_tile_kernel(int32_t* __restrict__ next, uint32_t nx, uint32_t ny, uint32_t nz) {
+msc_tile_kernel(int32_t* __restrict__ next, uint32_t nx, uint32_t ny, uint32_t nz, uint32_t first) {
     __shared__ uint16_t step[kTile];
     __shared__ int32_t out[kTile];
     const uint32_t tx = (nx + 63u) / 64u, ty = (ny + 3u) / 4u;
-    const uint32_t x0 = (blockIdx.x % tx) * 64u, y0 = ((blockIdx.x / tx) % ty) * 4u, z0 = (blockIdx.x / (tx * ty)) * 4u;
+    const uint32_t tile = first + blockIdx.x;
+    const uint32_t x0 = (tile % tx) * 64u, y0 = ((tile / tx) % ty) * 4u, z0 = (tile / (tx * ty)) * 4u;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const int32_t sy = (int32_t)nx, sz = (int32_t)(nx * ny);
 #pragma unroll
@@ -317,9 +319,12 @@ int jump_all(msceer_ctx* ctx, const Forest* forests, int count, uint32_t* flag) 
     for (int f = 0; f < count; f++) {
         const Forest& t = forests[f];
         if (t.n() == 0) continue;
-        const uint64_t tiles = (uint64_t)((t.nx + 63) / 64) * ((t.ny + 3) / 4) * ((t.nz + 3) / 4);
-        hipLaunchKernelGGL(msc_tile_kernel, dim3((uint32_t)tiles), dim3(kThreads), 0, s, t.next, t.nx, t.ny, t.nz);
-        CHECK_HIP(hipGetLastError());
+        const uint32_t tiles = ((t.nx + 63) / 64) * ((t.ny + 3) / 4) * ((t.nz + 3) / 4);
+        for (uint32_t k = 0; k < tiles; k += kMaxTiles) {
+            hipLaunchKernelGGL(msc_tile_kernel, dim3(tiles - k < kMaxTiles ? tiles - k : kMaxTiles), dim3(kThreads), 0, s,
+                               t.next, t.nx, t.ny, t.nz, k);
+            CHECK_HIP(hipGetLastError());
+        }
     }
     for (int it = 0; it < 64; it++) {
         CHECK_HIP(launch_zero(flag, 1, s));

@@ -114,3 +114,30 @@ def test_descending_regions_follow_the_rule(ctx, shape, kind):
                  "msceer_ondemand2")
     hipmem.synchronize()
     assert (dl.download(np.int32, f.size) == _rule(f, _maxima(f), np.arange(f.size), True)).all()
+
+
+def test_more_tiles_than_one_launch_takes(ctx):
+    """2 x 2100 x 8320 vertices, 525 x 2080 tiles in two launches: noise that
+    repeats every 16 layers, so its regions repeat too, but for the first and
+    the last layers.  Four repeats follow the rule, and all of them are alike."""
+    X, Y, P, n = 2, 2100, 16, 520
+    one = _noise((P, Y, X), 74)
+    print("certain, two launches", flush=True)
+
+    def regions(k):
+        f = np.tile(one, (k, 1, 1))
+        _, lab, _ = labels.ondemand_asc(f, ctx=ctx, stop="regions")
+        return f, lab
+
+    f, few = regions(4)
+    Z = 4 * P
+    seed = (((oracle_lib.lstar_pairs(f).reshape(2 * Z - 1, 2 * Y - 1, 2 * X - 1)[::2, ::2, ::2] >> 2) & 7) == 7).ravel()
+    assert (few.ravel() == _rule(f, seed, few.ravel(), False)).all()
+    _, lab = regions(n)
+    step = P * X * Y  # ids of one repeat
+    lab = lab.reshape(n, P, Y, X)
+    for k in range(n):
+        at = min(k, 1) if k < n - 1 else 3  # the first, an inner one, the last
+        assert ((lab[k] == -1) == (few.reshape(4, P, Y, X)[at] == -1)).all(), k
+        known = lab[k] >= 0
+        assert (lab[k][known] - k * step == few.reshape(4, P, Y, X)[at][known] - at * step).all(), k

@@ -72,3 +72,29 @@ def test_tile_edges_against_oracle(ctx, shape):
     assert (c == rc).all()
     assert (b == rb).all(), int((b != rb).sum())
     assert (m == rm).all(), int((m != rm).sum())
+
+
+def test_thin_volume_of_more_tiles_than_a_grid_holds(ctx):
+    """2 x 4100 x 65536 vertices: 1025 x 16384 tiles of 256 threads.  Every
+    vertex is paired towards lower z, so a column's basin is its lowest vertex,
+    the only critical cells there are."""
+    X, Y, Z = 2, 4100, 65536
+    plane = (2 * X - 1) * (2 * Y - 1)
+    dg = hipmem.DeviceBuffer(plane * (2 * Z - 1))
+    db = hipmem.DeviceBuffer(4 * X * Y * Z)
+    dg.fill(1)  # assigned, paired towards higher x
+    db.fill(0x7F)
+    hipmem.synchronize()
+    layer = np.full((2 * Y - 1, 2 * X - 1), 1, np.uint8)
+    for z in range(Z):
+        if z < 2:
+            layer[::2, ::2] = 1 | (7 if z == 0 else 5) << 2
+        dg.upload_at(2 * z * plane, layer)
+    counts = (ctypes.c_int64 * 4)()
+    print("thin volume: uploaded", flush=True)
+    native.check(native.lib().msceer_msc_base(ctx.handle, ctypes.c_void_p(dg.addr), X, Y, Z, ctypes.c_void_p(db.addr),
+                                              None, ctypes.cast(counts, ctypes.c_void_p), native.DEVICE_PTRS), "msc")
+    assert list(counts) == [X * Y, 0, 0, 0]
+    expect = np.tile(np.arange(X * Y, dtype=np.int32), 4096)
+    for z in range(0, Z, 4096):
+        assert np.array_equal(db.download_at(4 * X * Y * z, np.int32, expect.size), expect), z
