@@ -1014,9 +1014,8 @@ extern "C" int msceer_constrained_lstar(msceer_ctx* ctx, const float* values, in
         CHECK_HIP(ctx->grad.ensure(d.cells));
         d_grad = ctx->grad.as<uint8_t>();
     }
-    ListCaps caps{};
-    rc = ensure_lists(ctx, d, &caps);
-    if (rc) return rc;
+    const ListCaps caps = list_caps(d);  // (the lists are filled, and read by nothing here)
+    CHECK_HIP(ctx->lists.ensure(list_bytes(caps)));
     uint32_t* ctl = ctl_dev(ctx);
     const MList list1 = crit_list(ctx, caps, 0), list2 = crit_list(ctx, caps, 1);
     LstarBuffers cb{d_values, d_grad, d_r, &list1, &list2, ctl + kCtlStats, ctl + kCtlOverflow};

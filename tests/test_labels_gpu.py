@@ -8,6 +8,7 @@ the vertices (pass 1 of the reference depends on its threads' visiting
 order, the GPU's levels are synchronous, and the GPU traces in FP32 first).
 The GPU labels themselves are the same from run to run.
 """
+import ctypes
 import sys
 
 import numpy as np
@@ -16,7 +17,7 @@ import pytest
 import gradcheck
 import oracle_lib
 from golden import load_ondemand, ondemand_case_names
-from msceer_amd import labels, native
+from msceer_amd import hipmem, labels, native, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -218,3 +219,30 @@ def test_max_boundary_bit_exact(ctx, name):
         expect = oracle_lib.max_boundary(f, lab, ref["restriction"])
         assert (got == expect).all(), int((got != expect).sum())
         assert int((expect > 1).sum()) > 0
+
+
+def test_constrained_pass_allocates_no_frontiers():
+    """Its lists (10 bytes a vertex) and the ldir planes and bits (3): nothing
+    of the labelling's frontiers (16)."""
+    X = Y = Z = 256
+    V, C = X * Y * Z, (2 * X - 1) * (2 * Y - 1) * (2 * Z - 1)
+    dv, dr, dg = (hipmem.DeviceBuffer(n) for n in (4 * V, C, C))
+    dv.upload(synth.Stream(9).normal(V).astype(np.float32))
+    dr.fill(0)
+    hipmem.synchronize()
+    _say("constrained, memory")
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hipmem.hip().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    c = native.Context(0)
+    before = free()
+    native.check(native.lib().msceer_constrained_lstar(c.handle, ctypes.c_void_p(dv.addr), X, Y, Z,
+                                                       ctypes.c_void_p(dr.addr), ctypes.c_void_p(dg.addr),
+                                                       native.DEVICE_PTRS), "msceer_constrained_lstar")
+    used = before - free()
+    c.close()
+    _say(f"  {used / V:.1f} bytes a vertex")
+    assert used <= 20 * V
