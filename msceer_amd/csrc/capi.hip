@@ -52,9 +52,6 @@ MList front_list(msceer_ctx* ctx, const ListCaps& c, int k) {
     return MList{buf, ctl_dev(ctx) + kCtlRound + (k % 3) * kCountWords, c.front_sub, c.front_spill};
 }
 
-// Critical lists: a quarter of the vertices per sub-list set, spill for as
-// many again as there are vertices; frontiers: the vertex count in sub-lists
-// and as much again in spill.  Entries are cell ids (< 2^32).
 int tuned_shape(msceer_ctx* ctx, const Dims& d, int fallback) {
     std::lock_guard<std::mutex> lk(ctx->tuning->mu);
     if (ctx->tuning->mode == 0) return 0;
@@ -103,6 +100,9 @@ int lstar_shape(msceer_ctx* ctx, const Dims& d, const LstarBuffers& b, int* shap
     return MSCEER_OK;
 }
 
+// Critical lists: a quarter of the vertices per sub-list set, spill for as
+// many again as there are vertices; frontiers: the vertex count in sub-lists
+// and as much again in spill.  Entries are cell ids (< 2^32).
 ListCaps list_caps(const Dims& d) {
     ListCaps c{};
     const uint64_t list_cap = std::min<uint64_t>(kMaxListCap, std::max<uint64_t>(kMinListCap, d.verts / 4));

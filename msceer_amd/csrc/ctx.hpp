@@ -120,7 +120,7 @@ struct msceer_ctx {
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
     msceer::DevBuf values, grad, lists, front0, front1, ctl;
-    msceer::DevBuf ldir;  // ldir walk records and visited bitmaps
+    msceer::DevBuf ldir;  // ldir planes, reached bits and tile marks
     // accurate labelling
     msceer::DevBuf gradf, gradd, scan, label, label2, dest, seedmask, redo, stamp, rep, rep2, restriction, host_io, mask;
     // accurate 1-manifolds: per-cell line stamps (two words, older tags are
@@ -178,7 +178,7 @@ size_t front_bytes(const ListCaps& c);
 // already tuned for this x extent (64x2x2 if none) instead of tuning one.
 constexpr uint32_t kLstarNoTuning = 0x80000000u;
 // The whole .grad of a volume in device memory (msceer_lstar_grad's work after
-// staging): lists, frontiers and ldir scratch from the context; host_out
+// staging): lists and ldir scratch from the context; host_out
 // (may be null) receives a copy before the final wait.
 int lstar_grad_device(msceer_ctx* ctx, const Dims& d, const float* d_values, uint8_t* d_grad, uint8_t* host_out,
                       uint32_t flags);

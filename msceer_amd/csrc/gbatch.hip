@@ -43,7 +43,7 @@ enum GCtl : int {
     kGList2 = kCountWords,
     kGActive = 2 * kCountWords,            // three rotating words of the floods
     kGStats = 2 * kCountWords + 4,         // kSubs * 4 critical counts
-    kGOverflow = kGStats + 4 * kSubs,      // a critical list ran out of room
+    kGOverflow = kGStats + 4 * kSubs,      // a critical list ran out of room (nothing reads the lists)
     kGQueue = kGOverflow + 4,              // kQueues claim counters
     kGWords = kGQueue + kQueues
 };

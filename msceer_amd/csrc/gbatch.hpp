@@ -51,7 +51,7 @@ struct GBatch {
     GUnits bricks;  // lower-star bricks of the launch's brick shape
     GUnits tiles;   // work-groups of the ldir streaming passes
     GUnits floods;  // ldir flood tiles
-    GUnits items;   // the volume's cells
+    GUnits items;   // the volume's cells (numbers of the listed critical cells)
     uint32_t* queue;            // kQueues claim counters (persistent launches; zeroed before each)
     unsigned long long* times;  // 2 per volume: first brick started, last tile finished (wall clock); or null
     uint32_t chunk;             // units per claim

@@ -715,8 +715,8 @@ pass2_kernel(VGrid g, LabelBuffers b, WorkQueue q) {
 // reserved slots (head < tail, by compare-and-swap), so a claimed slot is
 // always about to be written.  A lane whose streamline ends takes new work
 // while the others keep advecting; the wave advects in bursts of up to kBurst
-// steps that end with the first streamline to end, so a wave left with one
-// long streamline does not visit the queue at every step.  A wave that holds
+// steps that end once a quarter of its streamlines have ended, so a wave left
+// with one long streamline does not visit the queue at every step.  A wave that holds
 // no streamline, no ring item and no claimed slot leaves once it has found
 // no unclaimed reserved slot for kLeaveTicks: every item queued later is
 // queued by a wave still running, which drains it before it leaves itself.

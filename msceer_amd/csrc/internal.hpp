@@ -28,8 +28,8 @@ struct LstarBuffers {
     const float* values;        // device, X*Y*Z
     uint8_t* grad;              // device, cells
     const int8_t* restriction;  // device, cells, or null (steepest pass)
-    const MList* list1;         // critical 1-cells (ldir pass 1 start)
-    const MList* list2;         // critical 2-cells (ldir pass 2 start)
+    const MList* list1;         // critical 1-cells: filled by every launch, read after the labelling's
+    const MList* list2;         // critical 2-cells  base pass alone (extremum graphs, 1-manifolds)
     uint32_t* stats;            // device, kSubs*4: critical cells by sub-list and dimension
     uint32_t* overflow;         // device flag: a critical list ran out of room
 };
@@ -47,7 +47,7 @@ void lstar_brick_dims(int shape, int* bx, int* by, int* bz);
 // queues and volume table in g.
 struct GBatch;
 // Lower-star bricks of every volume of the group (list entries: each volume's
-// cells from its first frontier item on; restriction unused): a work-group
+// cells numbered from its first[] of `items` on; restriction unused): a work-group
 // per brick (blocks == 0) or `blocks` persistent work-groups claiming bricks
 // (queue cleared beforehand).
 hipError_t launch_lstar_batch(const GBatch& g, const LstarBuffers& b, uint32_t blocks, hipStream_t s, int shape);

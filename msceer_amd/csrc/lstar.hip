@@ -85,7 +85,7 @@ struct LaneStar {
 
 // Arguments of one launch: a single volume (values .. nbz), or with kBatch
 // the volumes of a group (batch; the lists then hold each volume's cells
-// from its first frontier item on).
+// numbered from its first[] of batch.items on).
 struct LstarArgs {
     const float* values;
     uint8_t* grad;
@@ -277,7 +277,8 @@ __global__ void __launch_bounds__(kThreads) lstar_kernel(LstarArgs a) {
 
         // Copy the stage out, four cells a lane at a time along the rows; a zero
         // byte is a cell no brick vertex owns.  Critical cells (pair code 7) are
-        // counted by dimension and the 1- and 2-cells listed (for the line tracers).
+        // counted by dimension and the 1- and 2-cells listed (the labelling's base
+        // pass reads the lists; after the other launches nothing does).
         // Cell parity: stage x offset 4 j + b is .grad x 2 x0 - 1 + 4 j + b (odd
         // for even b), stage row (j, k) is y 2 y0 - 1 + j, z 2 z0 - 1 + k.
         uint32_t* const lst = reinterpret_cast<uint32_t*>(smem);

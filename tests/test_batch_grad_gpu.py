@@ -8,8 +8,9 @@ and two-vertex-thick volumes) under every brick shape and both launch forms
 16 volumes of the 512-volume workload's family (sides 32..160, smoothed
 noise and Gaussian mixtures) against the oracle; graph replays with other
 GPU work between them, each checked; groups split by a vertex cap; a first
-capture with too few frontier rounds, finished eagerly, and the recapture
-that follows."""
+capture with too few flood sweeps, finished eagerly, and the recapture
+that follows; more sweeps than a graph holds, and more groups than a context
+keeps graphs of."""
 import ctypes
 import os
 import subprocess
@@ -235,8 +236,8 @@ ctx.close()
 
 
 def test_first_capture_without_rounds_sweeps_and_recaptures():
-    """No rounds in the first graph: both passes start from a sweep of every
-    volume after the replay, and the next capture takes the rounds needed."""
+    """No flood sweeps in the first graph: all run after the replay, and the
+    next capture takes the sweeps needed."""
     _fresh_process(_FEW_ROUNDS.format(check="assert eager[0] > 0, eager"), {"MSCEER_BATCH_ROUNDS": "0"})
 
 

@@ -2,7 +2,7 @@
 the CPU against the reference's .grad goldens.
 
 setAscendingManifoldDimensions (gi_topological_gradient_using_algorithms.h:395-478)
-marks cells while it walks; the GPU instead records which items each pass
+marks cells while it walks; the GPU instead floods which items each pass
 reaches (edges in pass 1, quads in pass 2) and derives every cell's ldir from
 that afterwards (msceer_amd/csrc/ldir.hip):
   edge: 2 if reached in pass 1, else 3;

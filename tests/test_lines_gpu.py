@@ -2,15 +2,16 @@
 against the CPU oracle and the reference's runs.
 
 The streamlines run in FP64 on the GPU, as in the oracle's FP64 mode, and the
-GPU keeps the reference's one-thread saddle order exactly (speculation with
-in-order replay), so the digitized cells (4, 5) equal the FP64 oracle's bit
-for bit, and so do the whole restriction and the conforming .grad without
+GPU keeps the reference's one-thread saddle order exactly (tapes of all lines,
+evaluated in rounds until they agree with the order), so the digitized cells
+(4, 5) equal the FP64 oracle's bit for bit, and so do the whole restriction and the conforming .grad without
 needASC2 (with it, the MIN boundary follows labels that may differ by the
 pass-1 visiting order; the .grad is then checked as the oracle's conforming
 gradient of the GPU's restriction).  Against the reference's own runs (mixed FP32/FP64
 arithmetic) the restriction labels differ on at most 0.1 % of the labelled
-cells.  Small speculation windows (MSCEER_LINE_WINDOW) give the same bytes as
-one window.
+cells.  Small windows (MSCEER_LINE_WINDOW), windows cut short by a small pool
+of tapes or few rounds, and lines traced alone give the same bytes as one
+window.
 """
 import ctypes
 import gc
